@@ -4,14 +4,24 @@
 // Reference: BvhtlBuilder::buildTriangleBasedScene (BvhBuilder.cpp:37-253), PERFORMANCE
 // build type (4 candidate planes per axis), SAH segmentation.
 //
-// The build is level-parallel: one workgroup per node of the current level.
-//  * Binning. A candidate plane k on axis a sits at seg*k + bmin (seg = extent/4). The
-//    candidates are non-decreasing in k, so "centroid < plane_k" holds exactly for the
-//    primitives whose bin b = #{k : plane_k <= centroid} is <= k. Per axis the node keeps
-//    5 bins (count, min, max); the left side of candidate k is the union of bins 0..k and the
-//    right side the union of bins k+1..4. Min/max unions are exact, so the reference's
-//    costs hA(L)*nL + hA(R)*nR are reproduced bit for bit, including its NaN -> INT_MAX
-//    sentinel for an empty side and its strict "first minimum below float(INT_MAX)" rule.
+// A node is split by one of three kernels, by its primitive count:
+//  * above 16,384 (kBigNode): many workgroups per node, one set of launches per level;
+//  * above 512 (kSubPrims): one workgroup per node, one launch per level;
+//  * up to 512: one workgroup builds the node's whole subtree in LDS, one launch for all of
+//    them. One launch per level down to the leaves, a workgroup per node, spent most of the
+//    build on nodes of a few primitives: 33 of 40 ms for 1,048,576 triangles, 7.2 ms for one
+//    level of 400 k nodes. subtree_kernel takes 0.6 ms for all of them, the build 2.9 ms.
+//
+// What they share:
+//  * Cost. A candidate plane k on axis a sits at seg*k + bmin (seg = extent/4); the left side
+//    holds the primitives with centroid < plane. Min/max unions are exact and order-free, so
+//    the reference's costs hA(L)*nL + hA(R)*nR are reproduced bit for bit, including its
+//    NaN -> INT_MAX sentinel for an empty side and its strict "first minimum below
+//    float(INT_MAX)" rule. The 12 candidates (3 axes x 4 planes) are 12 lanes of a 16-lane
+//    row: each lane walks the primitives and keeps its own candidate's two boxes. Nodes above
+//    kSubPrims bin instead: candidates are non-decreasing in k, so "centroid < plane_k" holds
+//    exactly for the primitives whose bin b = #{k : plane_k <= centroid} is <= k, and the
+//    two sides of candidate k are the unions of bins 0..k and k+1..4.
 //  * Partition. The reference partitions with an in-place swap loop (BvhBuilder.cpp:186-203)
 //    whose output order the children inherit. With nL the left count, H = [0,nL) and
 //    T = [nL,n) (positions relative to the node), h_r the r-th right-class position in H
@@ -19,11 +29,14 @@
 //    q = t_{k-1} (n if H holds no right-class element), the loop's result is:
 //      left-class x in H stays; right-class h_r moves to t_{r-1}-1; left-class t_r moves
 //      to h_r; right-class x_p in T moves to p-1, except x_nL which moves to q-1.
-//    Ranks come from block-wide ballot/mbcnt prefix sums; the partition is applied even
-//    when the split is then rejected (nL = 0 or n), as in the reference.
-//  * Children are allocated in pairs (left, left+1), so node.left / node.left+1 address
-//    them as the reference's traversal expects. Node numbering is breadth-first per level;
-//    the primitive order prim_idx does not depend on it.
+//    Ranks come from ballots; the partition is applied even when the split is then rejected
+//    (nL = 0 or n), as in the reference.
+//  * Node numbers. Every split owns the boundary position b = first + nL between its two
+//    children, and no two splits share one, so the children are nodes 2b-1 and 2b of a sparse
+//    array: no allocation counter (an atomic on one address costs about 15 ns on this chip,
+//    which at 700 k nodes would be 10 ms). A scan over the used boundaries then packs the nodes
+//    in boundary order, children in pairs (left, left+1) as the reference's traversal expects.
+//    The primitive order prim_idx does not depend on the numbering.
 #include <algorithm>
 #include <vector>
 
@@ -35,6 +48,7 @@ namespace nova_hip {
 
 constexpr int kBuildBlock = 256;
 constexpr float kIntMaxF = 2147483648.f;  // float(INT_MAX)
+constexpr int kCands = 12;                // 3 axes x 4 candidate planes
 
 __device__ __forceinline__ int ford(float f) {  // order-preserving float -> int
   int i = __float_as_int(f);
@@ -42,502 +56,1030 @@ __device__ __forceinline__ int ford(float f) {  // order-preserving float -> int
 }
 __device__ __forceinline__ float unford(int i) { return __int_as_float(i >= 0 ? i : i ^ 0x7FFFFFFF); }
 
-struct BlockScan {
-  int wave_tot[kBuildBlock / 64];
-  int total;
+// One primitive as the build reads it: its box as ordered ints and its centroid, three
+// 16-byte loads instead of nine scattered words.
+struct alignas(16) BuildPrim {
+  int lo[3];
+  float cx;
+  int hi[3];
+  float cy;
+  float cz;
+  int pad[3];
 };
+static_assert(sizeof(BuildPrim) == 48, "BuildPrim layout");
 
-// Exclusive block prefix of `bit`; returns the rank and sets `chunk_total`.
-__device__ __forceinline__ int block_rank(int bit, BlockScan &sc, int &chunk_total) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint64_t m = __ballot(bit);
-  int in_wave = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-  if (lane == 0) sc.wave_tot[wave] = __popcll(m);
-  __syncthreads();
-  int before = 0, tot = 0;
-  for (int w = 0; w < kBuildBlock / 64; w++) {
-    int t = sc.wave_tot[w];
-    before += (w < wave) ? t : 0;
-    tot += t;
-  }
-  __syncthreads();
-  chunk_total = tot;
-  return before + in_wave;
-}
-
-struct LevelShared {
-  int cnt[3][5];
-  int bmn[3][5][3];
-  int bmx[3][5][3];
-  int cmn[2][3], cmx[2][3];  // child bounds
-  int nl;
-  int split, axis;
-  float pos;
-  BlockScan sc;
-};
-
-// Candidate planes of a node: seg*k + bmin per axis (axis_subdiv_sah, BvhBuilder.cpp:117-150).
-struct NodeCands {
-  float ext[3], cand[3][4];
-};
-__device__ __forceinline__ NodeCands node_cands(const BNode &nd) {
-  NodeCands c;
-  for (int a = 0; a < 3; a++) {
-    c.ext[a] = nd.mx[a] - nd.mn[a];
-    const float seg = c.ext[a] / 4.f;
-    for (int k = 0; k < 4; k++) c.cand[a][k] = seg * (float)k + nd.mn[a];
-  }
-  return c;
-}
-
-// Adds primitive p to the 3 x 5 bins (count, min, max as ordered ints; layout [axis*5+bin]).
-__device__ __forceinline__ void bin_primitive(const NodeCands &c, const float *__restrict__ aabb, const float *__restrict__ centroid, int p, int *cnt,
-                                              int *bmn, int *bmx) {
-  const float cc[3] = {centroid[(size_t)p * 3], centroid[(size_t)p * 3 + 1], centroid[(size_t)p * 3 + 2]};
-  int lo[3], hi[3];
-  for (int q = 0; q < 3; q++) {
-    lo[q] = ford(aabb[(size_t)p * 6 + q]);
-    hi[q] = ford(aabb[(size_t)p * 6 + 3 + q]);
-  }
-  for (int a = 0; a < 3; a++) {
-    if (c.ext[a] == 0) continue;
-    int b = 0;
-    for (int k = 0; k < 4; k++) b += (cc[a] < c.cand[a][k]) ? 0 : 1;
-    atomicAdd(&cnt[a * 5 + b], 1);
+// Two child boxes as ordered ints: empty boxes are the reference's (1e32, -1e32).
+struct SideBoxes {
+  int lmn[3], lmx[3], rmn[3], rmx[3];
+  __device__ __forceinline__ void clear() {
     for (int q = 0; q < 3; q++) {
-      atomicMin(&bmn[(a * 5 + b) * 3 + q], lo[q]);
-      atomicMax(&bmx[(a * 5 + b) * 3 + q], hi[q]);
+      lmn[q] = rmn[q] = ford(1e32f);
+      lmx[q] = rmx[q] = ford(-1e32f);
     }
   }
-}
-
-struct SplitChoice {
-  int split, axis;
-  float pos;
+  // selects, not a branch per side: the two sides' stores would become one store through a
+  // selected address and the boxes would live in scratch memory
+  __device__ __forceinline__ void add(bool left, const int *lo, const int *hi) {
+    const int mn = ford(1e32f), mx = ford(-1e32f);
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      lmn[q] = min(lmn[q], left ? lo[q] : mn);
+      lmx[q] = max(lmx[q], left ? hi[q] : mx);
+      rmn[q] = min(rmn[q], left ? mn : lo[q]);
+      rmx[q] = max(rmx[q], left ? mx : hi[q]);
+    }
+  }
 };
 
-// eval_sah over the 4 candidates of each axis from the bins, the first strict minimum
-// below float(INT_MAX) (empty side -> NaN -> INT_MAX), then the leaf test against the
-// node's own cost (BvhBuilder.cpp:117-184, 206-253).
-__device__ __forceinline__ SplitChoice decide_split(const BNode &nd, const NodeCands &c, const int *cnt, const int *bmn, const int *bmx, int n) {
-  float best_cost = kIntMaxF, best_pos = 0.f;
-  int best_axis = 0;
-  for (int a = 0; a < 3; a++) {
-    if (c.ext[a] == 0) continue;
-    for (int k = 0; k < 4; k++) {
-      float lmn[3] = {1e32f, 1e32f, 1e32f}, lmx[3] = {-1e32f, -1e32f, -1e32f};
-      float rmn[3] = {1e32f, 1e32f, 1e32f}, rmx[3] = {-1e32f, -1e32f, -1e32f};
-      int nl = 0, nr = 0;
-      for (int b = 0; b < 5; b++) {
-        const bool left = b <= k;
-        if (left)
-          nl += cnt[a * 5 + b];
-        else
-          nr += cnt[a * 5 + b];
-        for (int q = 0; q < 3; q++) {
-          const float bn = unford(bmn[(a * 5 + b) * 3 + q]), bx = unford(bmx[(a * 5 + b) * 3 + q]);
-          if (left) {
-            lmn[q] = gmin(lmn[q], bn);
-            lmx[q] = gmax(lmx[q], bx);
-          } else {
-            rmn[q] = gmin(rmn[q], bn);
-            rmx[q] = gmax(rmx[q], bx);
-          }
-        }
-      }
-      float cost = half_area(lmn[0], lmn[1], lmn[2], lmx[0], lmx[1], lmx[2]) * (float)nl +
-                   half_area(rmn[0], rmn[1], rmn[2], rmx[0], rmx[1], rmx[2]) * (float)nr;
-      cost = cost > 0.f ? cost : kIntMaxF;
-      if (cost < best_cost) {
-        best_cost = cost;
-        best_axis = a;
-        best_pos = c.cand[a][k];
-      }
-    }
-  }
-  const float node_cost = half_area(nd.mn[0], nd.mn[1], nd.mn[2], nd.mx[0], nd.mx[1], nd.mx[2]) * (float)n;
-  return SplitChoice{best_cost >= node_cost ? 0 : 1, best_axis, best_pos};
+// Candidate plane k of an axis of a box: seg*k + bmin (axis_subdiv_sah, BvhBuilder.cpp:117-150).
+__device__ __forceinline__ float cand_plane(float mn, float mx, int k) { return ((mx - mn) / 4.f) * (float)k + mn; }
+
+// eval_sah of one candidate (BvhBuilder.cpp:152-184): empty side -> NaN -> INT_MAX.
+__device__ __forceinline__ float side_cost(const SideBoxes &s, int nl, int nr) {
+  const float cost = half_area(unford(s.lmn[0]), unford(s.lmn[1]), unford(s.lmn[2]), unford(s.lmx[0]), unford(s.lmx[1]), unford(s.lmx[2])) * (float)nl +
+                     half_area(unford(s.rmn[0]), unford(s.rmn[1]), unford(s.rmn[2]), unford(s.rmx[0]), unford(s.rmx[1]), unford(s.rmx[2])) * (float)nr;
+  return cost > 0.f ? cost : kIntMaxF;
 }
 
-// Final position (relative to the node) of the element at rel under the swap loop's closed form.
-__device__ __forceinline__ int partition_dest(int rel, int bit, int rankL, int nL, int n, int q, const int32_t *__restrict__ hr_pos_s,
-                                              const int32_t *__restrict__ tl_pos_s) {
+// The split choice of a wave whose lanes 0..11 hold the candidates' costs (axis-major, as the
+// reference visits them): the first strict minimum below float(INT_MAX), then the leaf test
+// against the node's own cost (BvhBuilder.cpp:117-184, 206-253). best: the winning lane, -1
+// when no candidate lies below the sentinel (the reference then splits at x < 0).
+struct SplitChoice {
+  bool split;
+  int best, axis;
+  float pos;
+};
+__device__ __forceinline__ SplitChoice choose_split(float cost, float plane, bool valid, const float *mn, const float *mx, int n) {
+  const int lane = threadIdx.x & 63;
+  const float c = (valid && lane < kCands && cost < kIntMaxF) ? cost : kIntMaxF;
+  float m = c;
+  for (int d = 8; d > 0; d >>= 1) m = fminf(m, __shfl_xor(m, d, 64));  // lanes 0-15
+  const float best_cost = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(m)));
+  const uint64_t at = __ballot(c == best_cost && c < kIntMaxF) & ((1ull << kCands) - 1);
+  SplitChoice s;
+  s.best = at ? __builtin_ffsll((long long)at) - 1 : -1;
+  s.axis = at ? s.best >> 2 : 0;
+  s.pos = at ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(plane), s.best)) : 0.f;
+  const float node_cost = half_area(mn[0], mn[1], mn[2], mx[0], mx[1], mx[2]) * (float)n;
+  s.split = !(best_cost >= node_cost);
+  return s;
+}
+
+// Final position (relative to the node) of the element at rel under the swap loop's closed
+// form; hr and tl point at the node's part of the h_r and t_r maps.
+template <class Pos>
+__device__ __forceinline__ int partition_dest(int rel, bool bit, int rankL, int nL, int n, int q, const Pos *hr, const Pos *tl) {
   if (rel < nL) {
     if (bit) return rel;
     const int r = rel - rankL;
-    return (r == 0 ? n : tl_pos_s[r - 1]) - 1;
+    return (r == 0 ? n : (int)tl[r - 1]) - 1;
   }
-  if (bit) return hr_pos_s[nL - 1 - rankL];
+  if (bit) return (int)hr[nL - 1 - rankL];
   return (rel == nL && nL < q) ? q - 1 : rel - 1;
 }
 
-__global__ __launch_bounds__(kBuildBlock) void bvh_level_kernel(const int32_t *__restrict__ active, BNode *__restrict__ nodes,
-                                                                int32_t *__restrict__ prim_idx, int32_t *__restrict__ tmp_idx,
-                                                                const float *__restrict__ aabb, const float *__restrict__ centroid,
-                                                                uint8_t *__restrict__ cls, int32_t *__restrict__ rk, int32_t *__restrict__ hr_pos,
-                                                                int32_t *__restrict__ tl_pos, int32_t *__restrict__ node_counter,
-                                                                int32_t *__restrict__ next_active, int32_t *__restrict__ next_count,
-                                                                int32_t *__restrict__ parent, int32_t *__restrict__ depth) {
-  __shared__ LevelShared sh;
-  const int tid = threadIdx.x;
-  const int32_t id = active[blockIdx.x];
-  const BNode nd = nodes[id];
-  const int s = nd.left, n = nd.count;
-  const NodeCands nc = node_cands(nd);
-  for (int i = tid; i < 15; i += kBuildBlock) {
-    int a = i / 5, b = i % 5;
-    sh.cnt[a][b] = 0;
-    for (int q = 0; q < 3; q++) {
-      sh.bmn[a][b][q] = ford(1e32f);
-      sh.bmx[a][b][q] = ford(-1e32f);
-    }
-  }
-  __syncthreads();
+constexpr int kBigNode = 16384;  // above: many workgroups per node
+constexpr int kSubPrims = 512;   // up to: the whole subtree in one workgroup
+constexpr int kShards = 64;      // parts of a node list, each with a counter on its own cache line
+constexpr int kShardStride = 32;
 
-  // ---- binning (axis_subdiv_sah + eval_sah, BvhBuilder.cpp:117-184)
-  for (int i = s + tid; i < s + n; i += kBuildBlock) bin_primitive(nc, aabb, centroid, prim_idx[i], &sh.cnt[0][0], &sh.bmn[0][0][0], &sh.bmx[0][0][0]);
-  __syncthreads();
+// A level's work lists and the sparse node arrays. Nodes of a list start at distinct
+// positions, so a list cut into kShards ranges of start positions needs exactly one entry
+// per position, and its counters are hit by few workgroups each.
+struct BuildState {
+  const BuildPrim *prims;
+  int32_t *prim_idx, *tmp_idx;
+  BNode *nodes;       // 2n: node ids 0, then 2b-1 and 2b for the split at boundary b; an inner node's left is its boundary
+  int32_t *pair_parent, *pair_depth;  // by boundary
+  uint8_t *used;      // by boundary: a split owns it
+  int32_t *mid[2];    // by shard: nodes of this level and of the next
+  int32_t *sub;       // by shard: subtrees to build at the end
+  int32_t *big[2];
+  int32_t *mid_count[2], *sub_count, *depth_max;  // kShards counters each, kShardStride ints apart
+  int32_t *big_count;  // [2]
+  int32_t shard_shift;
+  int32_t n;
+};
+__device__ __forceinline__ int shard_of(const BuildState &b, int32_t pos) { return pos >> b.shard_shift; }
 
-  if (tid == 0) {
-    const SplitChoice sc = decide_split(nd, nc, &sh.cnt[0][0], &sh.bmn[0][0][0], &sh.bmx[0][0][0], n);
-    sh.split = sc.split;
-    sh.axis = sc.axis;
-    sh.pos = sc.pos;
-    sh.nl = 0;
-    for (int q = 0; q < 3; q++)
-      for (int c2 = 0; c2 < 2; c2++) {
-        sh.cmn[c2][q] = ford(1e32f);
-        sh.cmx[c2][q] = ford(-1e32f);
-      }
-  }
-  __syncthreads();
-  if (!sh.split) return;  // leaf: the reference returns before create_nodes
-  const int axis = sh.axis;
-  const float pos = sh.pos;
+__device__ __forceinline__ void list_push(const BuildState &b, int32_t *list, int32_t *count, int32_t pos, int32_t id) {
+  const int sh = shard_of(b, pos);
+  list[((size_t)sh << b.shard_shift) + atomicAdd(&count[sh * kShardStride], 1)] = id;
+}
+// A child of the current level: to the list of the kernel that will split it.
+__device__ __forceinline__ void push_child(const BuildState &b, int parity, int32_t id, int32_t pos, int32_t count) {
+  if (count > kBigNode)
+    b.big[parity ^ 1][atomicAdd(&b.big_count[parity ^ 1], 1)] = id;
+  else if (count > kSubPrims)
+    list_push(b, b.mid[parity ^ 1], b.mid_count[parity ^ 1], pos, id);
+  else
+    list_push(b, b.sub, b.sub_count, pos, id);
+}
+__device__ __forceinline__ void note_depth(const BuildState &b, int32_t pos, int32_t depth) {
+  int32_t *d = &b.depth_max[shard_of(b, pos) * kShardStride];
+  if (depth > *(volatile int32_t *)d) atomicMax(d, depth);
+}
+__device__ __forceinline__ int32_t node_depth(const BuildState &b, int32_t id) { return id == 0 ? 0 : b.pair_depth[(id + 1) >> 1]; }
 
-  // ---- classify and count (create_nodes predicate, BvhBuilder.cpp:194-199)
-  int my_l = 0;
-  for (int i = s + tid; i < s + n; i += kBuildBlock) {
-    const int p = prim_idx[i];
-    const int b = centroid[(size_t)p * 3 + axis] < pos ? 1 : 0;
-    cls[i] = (uint8_t)b;
-    my_l += b;
-  }
-  atomicAdd(&sh.nl, my_l);
-  __syncthreads();
-  const int nL = sh.nl;
-
-  // ---- ranks and the h_r / t_r maps
-  int running = 0;
-  for (int base = s; base < s + n; base += kBuildBlock) {
-    const int i = base + tid;
-    const int bit = (i < s + n) ? cls[i] : 0;
-    int tot;
-    const int r_in = block_rank(bit, sh.sc, tot);
-    if (i < s + n) {
-      const int rankL = running + r_in;
-      rk[i] = rankL;
-      const int rel = i - s;
-      if (rel < nL && !bit) hr_pos[s + (rel - rankL)] = rel;
-      if (rel >= nL && bit) tl_pos[s + (nL - 1 - rankL)] = rel;
-    }
-    running += tot;
-  }
-  __syncthreads();
-  const int LH = (nL < n) ? rk[s + nL] : nL;  // left-class elements inside H
-  const int k = nL - LH;                         // right-class elements inside H
-  const int q = (k == 0) ? n : tl_pos[s + k - 1];
-
-  // ---- scatter to the swap loop's final order
-  for (int i = s + tid; i < s + n; i += kBuildBlock) {
-    const int rel = i - s;
-    const int bit = cls[i];
-    const int rankL = rk[i];
-    tmp_idx[s + partition_dest(rel, bit, rankL, nL, n, q, hr_pos + s, tl_pos + s)] = prim_idx[i];
-  }
-  __syncthreads();
-
-  // ---- copy back and reduce the children's bounds (update_aabb, BvhBuilder.cpp:77-101)
-  int lmn[2][3], lmx[2][3];
-  for (int c2 = 0; c2 < 2; c2++)
-    for (int qq = 0; qq < 3; qq++) {
-      lmn[c2][qq] = ford(1e32f);
-      lmx[c2][qq] = ford(-1e32f);
-    }
-  for (int i = s + tid; i < s + n; i += kBuildBlock) {
-    const int p = tmp_idx[i];
-    prim_idx[i] = p;
-    const int side = (i - s) < nL ? 0 : 1;
-    for (int qq = 0; qq < 3; qq++) {
-      lmn[side][qq] = min(lmn[side][qq], ford(aabb[(size_t)p * 6 + qq]));
-      lmx[side][qq] = max(lmx[side][qq], ford(aabb[(size_t)p * 6 + 3 + qq]));
-    }
-  }
-  for (int c2 = 0; c2 < 2; c2++)
-    for (int qq = 0; qq < 3; qq++) {
-      atomicMin(&sh.cmn[c2][qq], lmn[c2][qq]);
-      atomicMax(&sh.cmx[c2][qq], lmx[c2][qq]);
-    }
-  __syncthreads();
-  if (tid != 0 || nL == 0 || nL == n) return;
-  const int32_t li = atomicAdd(node_counter, 2);
+// The two children of a split at relative position nL of node id = [s, s + n), boxes as
+// ordered ints (left min, left max, right min, right max).
+__device__ __forceinline__ void write_children(const BuildState &b, int32_t id, const BNode &nd, int32_t s, int32_t n, int32_t nL, const int *box,
+                                               int32_t depth) {
+  const int32_t at = s + nL;
   BNode L, R;
-  for (int qq = 0; qq < 3; qq++) {
-    L.mn[qq] = unford(sh.cmn[0][qq]);
-    L.mx[qq] = unford(sh.cmx[0][qq]);
-    R.mn[qq] = unford(sh.cmn[1][qq]);
-    R.mx[qq] = unford(sh.cmx[1][qq]);
+  for (int q = 0; q < 3; q++) {
+    L.mn[q] = unford(box[q]);
+    L.mx[q] = unford(box[3 + q]);
+    R.mn[q] = unford(box[6 + q]);
+    R.mx[q] = unford(box[9 + q]);
   }
   L.left = s;
   L.count = nL;
-  R.left = s + nL;
+  R.left = at;
   R.count = n - nL;
-  nodes[li] = L;
-  nodes[li + 1] = R;
-  parent[li] = parent[li + 1] = id;
-  depth[li] = depth[li + 1] = depth[id] + 1;
+  b.nodes[2 * (size_t)at - 1] = L;
+  b.nodes[2 * (size_t)at] = R;
+  b.pair_parent[at] = id;
+  b.pair_depth[at] = depth + 1;
+  b.used[at] = 1;
   BNode P = nd;
-  P.left = li;
+  P.left = at;
   P.count = 0;
-  nodes[id] = P;
-  const int32_t slot = atomicAdd(next_count, 2);
-  next_active[slot] = li;
-  next_active[slot + 1] = li + 1;
+  b.nodes[id] = P;
+}
+
+// -------------------------------------------------------- bins of the larger nodes
+// 3 axes x 5 bins x (min3, max3), 32 copies so that the 64 lanes of a wave update at most two
+// to an address: one copy made the wave's 64 updates of the same few words queue up (a node of
+// 16,384 primitives took 0.4 ms). Word w of copy c is at w * 32 + c.
+constexpr int kBinWords = 90, kBinCopies = 32;
+struct Bins {
+  int word[kBinWords * kBinCopies];
+  int sum[kBinWords];
+  int nl[kCands];  // left counts
+};
+
+template <int kBlock>
+__device__ __forceinline__ void bins_clear(Bins &b) {
+  const int mn = ford(1e32f), mx = ford(-1e32f);
+  for (int i = threadIdx.x; i < kBinWords * kBinCopies; i += kBlock) b.word[i] = (i / kBinCopies) % 6 < 3 ? mn : mx;
+  if (threadIdx.x < kCands) b.nl[threadIdx.x] = 0;
+}
+
+// Bins positions [start, end) of prim_idx; every thread of the workgroup takes part. `axes`:
+// bit a clear where the node has no extent (the reference skips that axis).
+template <int kBlock>
+__device__ __forceinline__ void bins_add(Bins &b, const BuildState &st, int32_t start, int32_t end, const float *mn, const float *mx) {
+  float plane[3][4];
+  for (int a = 0; a < 3; a++)
+    for (int k = 0; k < 4; k++) plane[a][k] = cand_plane(mn[a], mx[a], k);
+  const int lane = threadIdx.x & 63, copy = lane & (kBinCopies - 1);
+  int nl[kCands];
+  for (int c = 0; c < kCands; c++) nl[c] = 0;
+  for (int32_t i0 = start; i0 < end; i0 += kBlock) {  // uniform trip count: the ballots below count lanes
+    const int32_t i = i0 + (int32_t)threadIdx.x;
+    const bool in = i < end;
+    const int4 *r = reinterpret_cast<const int4 *>(st.prims + (in ? st.prim_idx[i] : 0));
+    const int4 r0 = r[0], r1 = r[1];
+    const float cc[3] = {__int_as_float(r0.w), __int_as_float(r1.w), reinterpret_cast<const float *>(r)[8]};
+    const int box[6] = {r0.x, r0.y, r0.z, r1.x, r1.y, r1.z};
+    for (int a = 0; a < 3; a++) {
+      int bin = 0;
+      for (int k = 0; k < 4; k++) {
+        const bool left = cc[a] < plane[a][k];
+        nl[a * 4 + k] += (int)__popcll(__ballot(in && left));
+        bin += left ? 0 : 1;
+      }
+      if (in) {
+        int *w = &b.word[(a * 5 + bin) * 6 * kBinCopies + copy];
+        for (int q = 0; q < 3; q++) {
+          atomicMin(w + q * kBinCopies, box[q]);
+          atomicMax(w + (3 + q) * kBinCopies, box[3 + q]);
+        }
+      }
+    }
+  }
+  for (int c = 0; c < kCands; c++)
+    if (lane == 0) atomicAdd(&b.nl[c], nl[c]);
+}
+
+// Copies -> sums (call between barriers).
+__device__ __forceinline__ void bins_reduce(Bins &b) {
+  if (threadIdx.x < kBinWords) {
+    const int w = threadIdx.x;
+    int v = b.word[w * kBinCopies + (w & (kBinCopies - 1))];
+    for (int c = 1; c < kBinCopies; c++) {  // each lane starts at another copy: no bank conflicts
+      const int x = b.word[w * kBinCopies + ((w + c) & (kBinCopies - 1))];
+      v = w % 6 < 3 ? min(v, x) : max(v, x);
+    }
+    b.sum[w] = v;
+  }
+}
+
+// One wave: the split choice from the bins; with a winner, its side boxes go to box[12].
+__device__ __forceinline__ SplitChoice bins_choose(const int *sum, const int *nl, const float *mn, const float *mx, int n, int *box) {
+  const int lane = threadIdx.x & 63, c = min(lane, kCands - 1), axis = c >> 2, k = c & 3;
+  SideBoxes s;
+  s.clear();
+  for (int bin = 0; bin < 5; bin++) {
+    const int *w = sum + (axis * 5 + bin) * 6;
+    s.add(bin <= k, w, w + 3);
+  }
+  const float amn = axis == 0 ? mn[0] : axis == 1 ? mn[1] : mn[2], amx = axis == 0 ? mx[0] : axis == 1 ? mx[1] : mx[2];
+  const SplitChoice ch = choose_split(side_cost(s, nl[c], n - nl[c]), cand_plane(amn, amx, k), amx - amn != 0.f, mn, mx, n);
+  if (ch.split && lane == ch.best)
+    for (int q = 0; q < 3; q++) {
+      box[q] = s.lmn[q];
+      box[3 + q] = s.lmx[q];
+      box[6 + q] = s.rmn[q];
+      box[9 + q] = s.rmx[q];
+    }
+  return ch;
+}
+
+__device__ __forceinline__ float prim_centroid(const BuildPrim *prims, int32_t p, int axis) {
+  const float *f = reinterpret_cast<const float *>(prims + p);
+  return f[axis == 0 ? 3 : axis == 1 ? 7 : 8];
+}
+
+// Merges every lane's side boxes over the wave and adds them to box[12] (ordered ints: left
+// min, left max, right min, right max). The split at x < 0 of a node whose costs all exceed
+// float(INT_MAX) has no candidate's boxes to reuse; the large scenes' top levels are such nodes.
+__device__ __forceinline__ void merge_sides(SideBoxes &s, int *box) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1)
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      s.lmn[q] = min(s.lmn[q], __shfl_xor(s.lmn[q], d, 64));
+      s.lmx[q] = max(s.lmx[q], __shfl_xor(s.lmx[q], d, 64));
+      s.rmn[q] = min(s.rmn[q], __shfl_xor(s.rmn[q], d, 64));
+      s.rmx[q] = max(s.rmx[q], __shfl_xor(s.rmx[q], d, 64));
+    }
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      atomicMin(&box[q], s.lmn[q]);
+      atomicMax(&box[3 + q], s.lmx[q]);
+      atomicMin(&box[6 + q], s.rmn[q]);
+      atomicMax(&box[9 + q], s.rmx[q]);
+    }
+}
+
+// ------------------------------------------- nodes of one workgroup (kSubPrims < n <= kBigNode)
+constexpr int kMidBlock = 512;
+struct MidShared {
+  Bins bins;
+  uint64_t mask[kBigNode / 64];  // class bits by position
+  int before[kBigNode / 64];     // left-class elements before each word
+  int wave_sum[kMidBlock / 64];
+  int box[12];
+  SplitChoice choice;
+};
+
+__global__ __launch_bounds__(kMidBlock) void mid_level_kernel(BuildState b, int parity, int32_t *hr_pos, int32_t *tl_pos) {
+  __shared__ MidShared sh;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int shard = blockIdx.x & (kShards - 1);
+  const int32_t have = b.mid_count[parity][shard * kShardStride];
+  for (int32_t item = blockIdx.x / kShards; item < have; item += gridDim.x / kShards) {
+    const int32_t id = b.mid[parity][((size_t)shard << b.shard_shift) + item];
+    const BNode nd = b.nodes[id];
+    const int32_t s = nd.left, n = nd.count;
+    bins_clear<kMidBlock>(sh.bins);
+    __syncthreads();
+    bins_add<kMidBlock>(sh.bins, b, s, s + n, nd.mn, nd.mx);
+    __syncthreads();
+    bins_reduce(sh.bins);
+    __syncthreads();
+    if (wave == 0) {
+      const SplitChoice ch = bins_choose(sh.bins.sum, sh.bins.nl, nd.mn, nd.mx, n, sh.box);
+      if (lane == 0) sh.choice = ch;
+    }
+    __syncthreads();
+    const SplitChoice ch = sh.choice;
+    const bool fallback = ch.best < 0;  // split at x < 0: no candidate's boxes
+    if (ch.split) {
+      if (fallback && tid < 12) sh.box[tid] = tid % 6 < 3 ? ford(1e32f) : ford(-1e32f);
+      if (fallback) __syncthreads();
+      // class bits, a word of 64 positions per wave and turn
+      const int words = (n + 63) >> 6;
+      SideBoxes sd;
+      sd.clear();
+      for (int j = wave; j < words; j += kMidBlock / 64) {
+        const int rel = j * 64 + lane;
+        const int32_t p = rel < n ? b.prim_idx[s + rel] : 0;
+        const bool bit = rel < n && prim_centroid(b.prims, p, ch.axis) < ch.pos;
+        const uint64_t m = __ballot(bit);
+        if (lane == 0) sh.mask[j] = m;
+        if (fallback && rel < n) sd.add(bit, b.prims[p].lo, b.prims[p].hi);
+      }
+      if (fallback) merge_sides(sd, sh.box);
+      __syncthreads();
+      // prefix over the words (at most 256 of them, one per thread of the first four waves)
+      const int pc = tid < words ? (int)__popcll(sh.mask[tid]) : 0;
+      int incl = pc;
+      for (int d = 1; d < 64; d <<= 1) {
+        const int x = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += x;
+      }
+      if (lane == 63) sh.wave_sum[wave] = incl;
+      __syncthreads();
+      int base = 0, nL = 0;
+      for (int w = 0; w < kMidBlock / 64; w++) {
+        base += w < wave ? sh.wave_sum[w] : 0;
+        nL += sh.wave_sum[w];
+      }
+      if (tid < words) sh.before[tid] = base + incl - pc;
+      __syncthreads();
+      auto rank = [&](int rel) { return sh.before[rel >> 6] + (int)__popcll(sh.mask[rel >> 6] & ((1ull << (rel & 63)) - 1)); };
+      for (int rel = tid; rel < n; rel += kMidBlock) {
+        const bool bit = (sh.mask[rel >> 6] >> (rel & 63)) & 1u;
+        const int r = rank(rel);
+        if (rel < nL && !bit) hr_pos[s + (rel - r)] = rel;
+        if (rel >= nL && bit) tl_pos[s + (nL - 1 - r)] = rel;
+      }
+      __syncthreads();
+      const int LH = nL < n ? rank(nL) : nL;  // left-class elements inside H
+      const int k = nL - LH;                  // right-class elements inside H
+      const int q = k == 0 ? n : tl_pos[s + k - 1];
+      for (int rel = tid; rel < n; rel += kMidBlock) {
+        const bool bit = (sh.mask[rel >> 6] >> (rel & 63)) & 1u;
+        b.tmp_idx[s + partition_dest(rel, bit, rank(rel), nL, n, q, hr_pos + s, tl_pos + s)] = b.prim_idx[s + rel];
+      }
+      __syncthreads();
+      for (int rel = tid; rel < n; rel += kMidBlock) b.prim_idx[s + rel] = b.tmp_idx[s + rel];
+      if (tid == 0 && nL != 0 && nL != n) {
+        const int32_t d = node_depth(b, id);
+        write_children(b, id, nd, s, n, nL, sh.box, d);
+        note_depth(b, s, d + 1);
+        push_child(b, parity, 2 * (s + nL) - 1, s, nL);
+        push_child(b, parity, 2 * (s + nL), s + nL, n - nL);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// ------------------------------------------------------- whole subtrees in LDS (n <= kSubPrims)
+// The primitives of the subtree are in LDS in position order and move there at each
+// partition. 16-lane rows evaluate the 12 candidates (lane = candidate). Nodes above 64
+// primitives are split by the workgroup (its 16 rows share out the primitives), nodes above 16
+// by one wave each (4 rows), and smaller ones, nine nodes in ten, by one row each, so a wave
+// works on four of them at a time. What bounds it is latency, a chain of LDS reads and lane
+// exchanges per node; nothing in the loops loads from memory, since a load would first wait for
+// the node records that the loops store.
+constexpr int kSubBlock = 256, kSubWaves = kSubBlock / 64, kWavePrims = 64, kRowPrims = 16;
+// A node waiting to be split: where it lies in the subtree, which child of its split it is
+// (bit 30: the right one), its depth below the subtree's root, and its box as ordered ints.
+struct SubNode {
+  int32_t at;  // a | m << 10 | depth << 20 | right << 30
+  int32_t box[6];
+};
+static_assert(kSubPrims <= 512, "SubNode fields");
+// Compiler vectors: a choice between members of HIP's vector structs becomes a load through a
+// selected address, which puts them into scratch memory, whose loads wait for every store in
+// flight (2.4 ms instead of 0.7 ms for 1,048,576 triangles).
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+struct SubShared {
+  v4i d0[kSubPrims];  // box min, centroid x
+  v4i d1[kSubPrims];  // box max, centroid y
+  v2i d2[kSubPrims];  // centroid z, primitive
+  short hr[kSubPrims], tl[kSubPrims];
+  uint64_t mask[kSubPrims / 64];
+  int part[kSubWaves][kCands][13];
+  int box[12];
+  // lists of disjoint nodes: above kWavePrims, above kRowPrims, at least 2 primitives
+  SubNode coop[kSubPrims / kWavePrims + 1];
+  SubNode wave_list[kSubPrims / kRowPrims + 1];
+  SubNode row_list[kSubPrims / 2 + 1];
+  SubNode stack[kSubBlock / 16][kRowPrims / 2 + 1];  // a row's pending nodes; a wave's use its first row's
+  int ncoop, nwave, nrow, next_wave, next_row, dmax;
+};
+
+// One of three values by axis.
+__device__ __forceinline__ float by_axis(int axis, int x, int y, int z) { return __int_as_float(axis == 0 ? x : axis == 1 ? y : z); }
+
+__device__ __forceinline__ void wave_sync_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// One lane's candidate (`plane` on `axis`) against positions a + row, a + row + rows, ...
+__device__ __forceinline__ void lane_sides(const SubShared &sh, int a, int m, int row, int rows, int axis, float plane, SideBoxes &s, int &nl) {
+  s.clear();
+  nl = 0;
+  for (int i = a + row; i < a + m; i += rows) {
+    const v4i p0 = sh.d0[i], p1 = sh.d1[i];
+    const bool left = by_axis(axis, p0.w, p1.w, sh.d2[i].x) < plane;
+    const int lo[3] = {p0.x, p0.y, p0.z}, hi[3] = {p1.x, p1.y, p1.z};
+    s.add(left, lo, hi);
+    nl += left ? 1 : 0;
+  }
+}
+// Over the wave's four rows: every row then holds the wave's result.
+__device__ __forceinline__ void merge_rows(SideBoxes &s, int &nl) {
+#pragma unroll
+  for (int d = 16; d <= 32; d <<= 1) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      s.lmn[q] = min(s.lmn[q], __shfl_xor(s.lmn[q], d, 64));
+      s.lmx[q] = max(s.lmx[q], __shfl_xor(s.lmx[q], d, 64));
+      s.rmn[q] = min(s.rmn[q], __shfl_xor(s.rmn[q], d, 64));
+      s.rmx[q] = max(s.rmx[q], __shfl_xor(s.rmx[q], d, 64));
+    }
+    nl += __shfl_xor(nl, d, 64);
+  }
+}
+
+// The fallback split at x < 0: its side boxes over [a, a + m).
+__device__ __forceinline__ void fallback_sides(const SubShared &sh, int a, int m, SideBoxes &s) {
+  s.clear();
+  for (int i = a; i < a + m; i++) {
+    const v4i p0 = sh.d0[i], p1 = sh.d1[i];
+    const int lo[3] = {p0.x, p0.y, p0.z}, hi[3] = {p1.x, p1.y, p1.z};
+    s.add(__int_as_float(p0.w) < 0.f, lo, hi);
+  }
+}
+
+// One lane: the children of node e (its split at relative position nL accepted) into the
+// sparse arrays, and each child with at least two primitives onto the list of its size.
+__device__ __forceinline__ void push_sub(SubShared &sh, const SubNode &c, int m) {
+  if (m > kWavePrims)
+    sh.coop[atomicAdd(&sh.ncoop, 1)] = c;
+  else if (m > kRowPrims)
+    sh.wave_list[atomicAdd(&sh.nwave, 1)] = c;
+  else if (m > 1)
+    sh.row_list[atomicAdd(&sh.nrow, 1)] = c;
+}
+struct SubPlace {
+  int a, m, depth;
+  bool right;
+  int32_t id;
+};
+__device__ __forceinline__ SubPlace sub_place(int32_t at, int32_t s0, int32_t root) {
+  SubPlace p;
+  p.a = at & 1023;
+  p.m = (at >> 10) & 1023;
+  p.depth = (at >> 20) & 1023;
+  p.right = (at >> 30) & 1;
+  // a child's id follows from its split's boundary; the root's was given
+  p.id = p.depth == 0 ? root : p.right ? 2 * (s0 + p.a) : 2 * (s0 + p.a + p.m) - 1;
+  return p;
+}
+__device__ __forceinline__ void split_sub(const BuildState &b, const SubPlace &p, const int32_t *box, int32_t s0, int32_t depth0, int nL,
+                                          const SideBoxes &sd, SubNode &L, SubNode &R) {
+  BNode rec;
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    rec.mn[q] = unford(box[q]);
+    rec.mx[q] = unford(box[3 + q]);
+    L.box[q] = sd.lmn[q];
+    L.box[3 + q] = sd.lmx[q];
+    R.box[q] = sd.rmn[q];
+    R.box[3 + q] = sd.rmx[q];
+  }
+  const int boxes[12] = {sd.lmn[0], sd.lmn[1], sd.lmn[2], sd.lmx[0], sd.lmx[1], sd.lmx[2], sd.rmn[0], sd.rmn[1], sd.rmn[2], sd.rmx[0], sd.rmx[1], sd.rmx[2]};
+  write_children(b, p.id, rec, s0 + p.a, p.m, nL, boxes, depth0 + p.depth);
+  L.at = p.a | nL << 10 | (p.depth + 1) << 20;
+  R.at = (p.a + nL) | (p.m - nL) << 10 | (p.depth + 1) << 20 | 1 << 30;
+}
+
+// A position's record on its way through a partition.
+struct Moving {
+  v4i r0, r1;
+  v2i r2;
+  bool bit;
+  int rank;
+};
+
+// 4 workgroups per CU (128 registers, 37 KB of LDS); 3 and 5 measured the same, and so did 256
+// primitives per subtree (2.85 to 2.92 ms per build of 1,048,576 triangles).
+__global__ __launch_bounds__(kSubBlock, 4) void subtree_kernel(BuildState b) {
+  __shared__ SubShared sh;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row = tid >> 4;
+  const int cand = min(lane & 15, kCands - 1), axis = cand >> 2, kplane = cand & 3;
+  const int shard = blockIdx.x & (kShards - 1);
+  const int32_t have = b.sub_count[shard * kShardStride];
+  // this lane's axis of a box, and its candidate plane
+  auto on_axis = [&](float x, float y, float z) { return axis == 0 ? x : axis == 1 ? y : z; };
+  for (int32_t item = blockIdx.x / kShards; item < have; item += gridDim.x / kShards) {
+    const int32_t root = b.sub[((size_t)shard << b.shard_shift) + item];
+    const BNode rn = b.nodes[root];
+    const int32_t s0 = rn.left, n0 = rn.count, depth0 = node_depth(b, root);
+    for (int i = tid; i < n0; i += kSubBlock) {
+      const int32_t p = b.prim_idx[s0 + i];
+      const v4i *r = reinterpret_cast<const v4i *>(b.prims + p);
+      sh.d0[i] = r[0];
+      sh.d1[i] = r[1];
+      sh.d2[i] = v2i{reinterpret_cast<const int *>(r)[8], p};
+    }
+    if (tid == 0) {
+      sh.ncoop = sh.nwave = sh.nrow = sh.next_wave = sh.next_row = 0;
+      sh.dmax = 0;
+      SubNode c;
+      c.at = n0 << 10;
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        c.box[q] = ford(rn.mn[q]);
+        c.box[3 + q] = ford(rn.mx[q]);
+      }
+      push_sub(sh, c, n0);
+    }
+    __syncthreads();
+
+    // ---- nodes above kWavePrims: the whole workgroup
+    while (sh.ncoop > 0) {
+      const SubNode nd = sh.coop[sh.ncoop - 1];
+      const SubPlace pl = sub_place(nd.at, s0, root);
+      const int a = pl.a, m = pl.m;
+      const float mn[3] = {unford(nd.box[0]), unford(nd.box[1]), unford(nd.box[2])}, mx[3] = {unford(nd.box[3]), unford(nd.box[4]), unford(nd.box[5])};
+      const float amn = on_axis(mn[0], mn[1], mn[2]), amx = on_axis(mx[0], mx[1], mx[2]);
+      const float plane = cand_plane(amn, amx, kplane);
+      SideBoxes sd;
+      int nl;
+      lane_sides(sh, a, m, row, kSubBlock / 16, axis, plane, sd, nl);
+      merge_rows(sd, nl);
+      if (lane < kCands) {
+        int *o = sh.part[wave][lane];
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+          o[q] = sd.lmn[q];
+          o[3 + q] = sd.lmx[q];
+          o[6 + q] = sd.rmn[q];
+          o[9 + q] = sd.rmx[q];
+        }
+        o[12] = nl;
+      }
+      __syncthreads();  // also: every thread has read ncoop and the node
+      for (int w = 0; w < kSubWaves; w++) {  // every wave merges the waves' parts and decides alike
+        if (w == wave) continue;
+        const int *o = sh.part[w][cand];
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+          sd.lmn[q] = min(sd.lmn[q], o[q]);
+          sd.lmx[q] = max(sd.lmx[q], o[3 + q]);
+          sd.rmn[q] = min(sd.rmn[q], o[6 + q]);
+          sd.rmx[q] = max(sd.rmx[q], o[9 + q]);
+        }
+        nl += o[12];
+      }
+      const SplitChoice ch = choose_split(side_cost(sd, nl, m - nl), plane, amx - amn != 0.f, mn, mx, m);
+      if (tid == 0) sh.ncoop--;
+      if (!ch.split) {  // a leaf: its record is written already
+        __syncthreads();
+        continue;
+      }
+      if (ch.best < 0 && tid == 0) fallback_sides(sh, a, m, sd);  // before the barriers: positions move after them
+      // positions tid and tid + 256 of the node
+      auto read = [&](int rel, int word, Moving &x) {
+        const bool in = rel < m;
+        const int i = a + (in ? rel : 0);
+        x.r0 = sh.d0[i];
+        x.r1 = sh.d1[i];
+        x.r2 = sh.d2[i];
+        x.bit = in && by_axis(ch.axis, x.r0.w, x.r1.w, x.r2.x) < ch.pos;
+        const uint64_t mk = __ballot(x.bit);
+        if (lane == 0) sh.mask[word] = mk;
+      };
+      Moving x0, x1;
+      read(tid, wave, x0);
+      if (kSubPrims > kSubBlock) read(tid + kSubBlock, kSubWaves + wave, x1);
+      __syncthreads();
+      int nL = 0;
+      for (int w = 0; w < kSubPrims / 64; w++) nL += (int)__popcll(sh.mask[w]);
+      auto rank = [&](int x) {  // left-class elements before position x
+        int r = 0;
+        for (int w = 0; w < kSubPrims / 64; w++) {
+          const int in = x - w * 64;
+          r += in <= 0 ? 0 : (int)__popcll(in >= 64 ? sh.mask[w] : sh.mask[w] & ((1ull << in) - 1));
+        }
+        return r;
+      };
+      auto map = [&](int rel, Moving &x) {
+        x.rank = rank(rel);
+        if (rel < nL && rel < m && !x.bit) sh.hr[a + (rel - x.rank)] = (short)rel;
+        if (rel >= nL && rel < m && x.bit) sh.tl[a + (nL - 1 - x.rank)] = (short)rel;
+      };
+      map(tid, x0);
+      if (kSubPrims > kSubBlock) map(tid + kSubBlock, x1);
+      const int k = nL - (nL < m ? rank(nL) : nL);
+      __syncthreads();
+      const int q = k == 0 ? m : (int)sh.tl[a + k - 1];
+      auto move = [&](int rel, const Moving &x) {
+        if (rel >= m) return;
+        const int to = a + partition_dest(rel, x.bit, x.rank, nL, m, q, sh.hr + a, sh.tl + a);
+        sh.d0[to] = x.r0;
+        sh.d1[to] = x.r1;
+        sh.d2[to] = x.r2;
+      };
+      move(tid, x0);
+      if (kSubPrims > kSubBlock) move(tid + kSubBlock, x1);
+      if (nL != 0 && nL != m && tid == max(ch.best, 0)) {
+        SubNode L, R;
+        split_sub(b, pl, nd.box, s0, depth0, nL, sd, L, R);
+        push_sub(sh, L, nL);
+        push_sub(sh, R, m - nL);
+        atomicMax(&sh.dmax, pl.depth + 1);
+      }
+      __syncthreads();
+    }
+
+    // ---- nodes above kRowPrims: one wave each, one split per turn; the children go to the
+    // lists (a wave takes nodes as long as there are any, its own children among them)
+    SubNode *stack = sh.stack[wave * 4];
+    int dmax = 0;
+    const int nwave = sh.nwave;
+    for (;;) {
+      int t = 0;
+      if (lane == 0) t = atomicAdd(&sh.next_wave, 1);
+      t = __builtin_amdgcn_readfirstlane(t);
+      if (t >= nwave) break;
+      if (lane == 0) stack[0] = sh.wave_list[t];
+      int sp = 1;
+      while (sp > 0) {
+        wave_sync_lds();
+        const SubNode nd = stack[--sp];
+        const SubPlace pl = sub_place(__builtin_amdgcn_readfirstlane(nd.at), s0, root);
+        const int a = pl.a, m = pl.m;
+        const float mn[3] = {unford(nd.box[0]), unford(nd.box[1]), unford(nd.box[2])}, mx[3] = {unford(nd.box[3]), unford(nd.box[4]), unford(nd.box[5])};
+        const float amn = on_axis(mn[0], mn[1], mn[2]), amx = on_axis(mx[0], mx[1], mx[2]);
+        const float plane = cand_plane(amn, amx, kplane);
+        SideBoxes sd;
+        int nl;
+        lane_sides(sh, a, m, lane >> 4, 4, axis, plane, sd, nl);
+        merge_rows(sd, nl);
+        const SplitChoice ch = choose_split(side_cost(sd, nl, m - nl), plane, amx - amn != 0.f, mn, mx, m);
+        if (!ch.split) continue;
+        const bool in = lane < m;
+        const int i = a + (in ? lane : 0);
+        const v4i r0 = sh.d0[i], r1 = sh.d1[i];
+        const v2i r2 = sh.d2[i];
+        const bool bit = in && by_axis(ch.axis, r0.w, r1.w, r2.x) < ch.pos;
+        const uint64_t mk = __ballot(bit);
+        const int nL = (int)__popcll(mk);
+        const int rk = __builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0));
+        if (in && lane < nL && !bit) sh.hr[a + (lane - rk)] = (short)lane;
+        if (in && lane >= nL && bit) sh.tl[a + (nL - 1 - rk)] = (short)lane;
+        const int k = nL - (nL < m ? (int)__popcll(mk & ((1ull << nL) - 1)) : nL);
+        wave_sync_lds();
+        const int q = k == 0 ? m : (int)sh.tl[a + k - 1];
+        const int to = a + (in ? partition_dest(lane, bit, rk, nL, m, q, sh.hr + a, sh.tl + a) : 0);
+        if (ch.best < 0) fallback_sides(sh, a, m, sd);
+        wave_sync_lds();
+        if (in) {
+          sh.d0[to] = r0;
+          sh.d1[to] = r1;
+          sh.d2[to] = r2;
+        }
+        if (nL == 0 || nL == m) continue;
+        if (lane == max(ch.best, 0)) {
+          SubNode L, R;
+          split_sub(b, pl, nd.box, s0, depth0, nL, sd, L, R);
+          int at = sp;
+          if (nL > kRowPrims)
+            stack[at++] = L;
+          else
+            push_sub(sh, L, nL);
+          if (m - nL > kRowPrims)
+            stack[at] = R;
+          else
+            push_sub(sh, R, m - nL);
+        }
+        sp += (nL > kRowPrims ? 1 : 0) + (m - nL > kRowPrims ? 1 : 0);
+        dmax = max(dmax, pl.depth + 1);
+      }
+    }
+    __syncthreads();
+
+    // ---- the rest: one row each
+    stack = sh.stack[row];
+    const int nrow = sh.nrow, r16 = lane & 48;
+    int sp = 0;
+    bool done = false;
+    while (__ballot(!done) != 0) {
+      if (sp == 0 && !done) {  // this row's next node
+        int t = 0;
+        if ((lane & 15) == 0) t = atomicAdd(&sh.next_row, 1);
+        t = __shfl(t, r16, 64);
+        done = t >= nrow;
+        if (!done) {
+          if ((lane & 15) == 0) stack[0] = sh.row_list[t];
+          sp = 1;
+        }
+      }
+      wave_sync_lds();
+      const bool live = sp > 0;
+      SubNode nd{};
+      if (live) nd = stack[--sp];
+      const SubPlace pl = sub_place(nd.at, s0, root);
+      const int a = pl.a, m = live ? pl.m : 0;
+      const float mn[3] = {unford(nd.box[0]), unford(nd.box[1]), unford(nd.box[2])}, mx[3] = {unford(nd.box[3]), unford(nd.box[4]), unford(nd.box[5])};
+      const float amn = on_axis(mn[0], mn[1], mn[2]), amx = on_axis(mx[0], mx[1], mx[2]);
+      const float plane = cand_plane(amn, amx, kplane);
+      SideBoxes sd;
+      int nl;
+      lane_sides(sh, a, m, 0, 1, axis, plane, sd, nl);
+      // choose_split, per row
+      const float cost = side_cost(sd, nl, m - nl);
+      const float c = ((lane & 15) < kCands && amx - amn != 0.f && cost < kIntMaxF) ? cost : kIntMaxF;
+      float best_cost = c;
+#pragma unroll
+      for (int d = 8; d > 0; d >>= 1) best_cost = fminf(best_cost, __shfl_xor(best_cost, d, 64));
+      const uint32_t at = (uint32_t)(__ballot(c == best_cost && c < kIntMaxF) >> r16) & ((1u << kCands) - 1);
+      const int best = at ? __builtin_ffs((int)at) - 1 : -1;
+      const int saxis = at ? best >> 2 : 0;
+      const float pos = at ? __shfl(plane, r16 + best, 64) : 0.f;
+      const float node_cost = half_area(mn[0], mn[1], mn[2], mx[0], mx[1], mx[2]) * (float)m;
+      const bool split = live && !(best_cost >= node_cost);
+      // partition
+      const int rel = lane & 15;
+      const bool in = split && rel < m;
+      const int i = a + (in ? rel : 0);
+      const v4i r0 = sh.d0[i], r1 = sh.d1[i];
+      const v2i r2 = sh.d2[i];
+      const bool bit = in && by_axis(saxis, r0.w, r1.w, r2.x) < pos;
+      const uint32_t mk = (uint32_t)(__ballot(bit) >> r16) & 0xFFFFu;
+      const int nL = __popc(mk), rk = __popc(mk & ((1u << rel) - 1));
+      if (in && rel < nL && !bit) sh.hr[a + (rel - rk)] = (short)rel;
+      if (in && rel >= nL && bit) sh.tl[a + (nL - 1 - rk)] = (short)rel;
+      const int k = nL - (nL < m ? __popc(mk & ((1u << nL) - 1)) : nL);
+      wave_sync_lds();
+      int to = 0;
+      if (in) {
+        const int q = k == 0 ? m : (int)sh.tl[a + k - 1];
+        to = a + partition_dest(rel, bit, rk, nL, m, q, sh.hr + a, sh.tl + a);
+      }
+      if (split && best < 0) fallback_sides(sh, a, m, sd);
+      wave_sync_lds();
+      if (in) {
+        sh.d0[to] = r0;
+        sh.d1[to] = r1;
+        sh.d2[to] = r2;
+      }
+      if (split && nL != 0 && nL != m) {
+        if (rel == max(best, 0)) {
+          SubNode L, R;
+          split_sub(b, pl, nd.box, s0, depth0, nL, sd, L, R);
+          if (nL > 1) stack[sp] = L;
+          if (m - nL > 1) stack[sp + (nL > 1 ? 1 : 0)] = R;
+        }
+        sp += (nL > 1 ? 1 : 0) + (m - nL > 1 ? 1 : 0);
+        dmax = max(dmax, pl.depth + 1);
+      }
+    }
+    atomicMax(&sh.dmax, dmax);
+    __syncthreads();
+    for (int i = tid; i < n0; i += kSubBlock) b.prim_idx[s0 + i] = sh.d2[i].y;
+    if (tid == 0) note_depth(b, s0, depth0 + sh.dmax);
+    __syncthreads();
+  }
 }
 
 // ------------------------------------------------- nodes too large for one workgroup
 // A node with more than kBigNode primitives is processed by many workgroups, kBigChunk
-// primitives each, in eight steps that compute exactly what bvh_level_kernel computes:
-// bin (per-chunk LDS bins merged with atomics: min/max/count unions are order-free),
-// decide, classify + count per chunk, scan of the chunk counts in chunk order, ranks
-// (chunk base + in-chunk rank = the node-wide rank), scatter by the same closed form,
-// copy back with child bounds, allocate the children.
-constexpr int kBigNode = 16384;
+// primitives each, in steps that compute exactly what mid_level_kernel computes: bin
+// (per-chunk bins merged with atomics: min/max/count unions are order-free), decide,
+// classify + count per chunk, scan of the chunk counts in chunk order, ranks (chunk base +
+// in-chunk rank = the node-wide rank), scatter by the same closed form, copy back. The chunk
+// table is made on the device (big_setup_kernel), so the host launches the steps of a level
+// without knowing how many nodes it has.
 constexpr int kBigChunk = 4096;
 
 struct BigNode {
   int32_t id, s, n;
   int32_t chunk_first, chunk_count;
-  int32_t split, axis, nL;
+  int32_t split, axis, nL, fallback;
   float pos;
-  int32_t cnt[15], bmn[45], bmx[45];  // bins
-  int32_t cmn[2][3], cmx[2][3];       // child bounds
+  int32_t sum[kBinWords], nl[kCands];  // bins
+  int32_t box[12];                     // child boxes
 };
 
 struct BigChunk {
   int32_t big, start, end;  // prim_idx positions [start, end)
 };
+struct BigState {
+  BigNode *nodes;
+  BigChunk *chunks;
+  int32_t *chunk_count;  // chunks of this level
+  int32_t *chunk_nl, *chunk_base;
+  uint8_t *cls;
+  int32_t *rk, *hr_pos, *tl_pos;
+};
 
-// Splits the level's nodes: big ones into `big` (id, s, n), the rest into `small`.
-__global__ void split_active_kernel(const int32_t *__restrict__ active, int32_t count, const BNode *__restrict__ nodes, BigNode *big,
-                                    int32_t *big_count, int32_t *small, int32_t *small_count) {
-  for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
-    const int32_t id = active[i];
-    const BNode nd = nodes[id];
-    if (nd.count > kBigNode) {
-      const int32_t k = atomicAdd(big_count, 1);
-      big[k].id = id;
-      big[k].s = nd.left;
-      big[k].n = nd.count;
-    } else {
-      small[atomicAdd(small_count, 1)] = id;
-    }
+// One workgroup: the level's big nodes with empty bins, their chunks, and empty lists for the
+// next level.
+__global__ __launch_bounds__(kBuildBlock) void big_setup_kernel(BuildState b, BigState g, int parity, int max_chunks) {
+  const int32_t have = b.big_count[parity];
+  __shared__ int32_t total, wave_tot[kBuildBlock / 64];
+  if (threadIdx.x < kShards) b.mid_count[parity ^ 1][threadIdx.x * kShardStride] = 0;
+  if (threadIdx.x == 0) {
+    b.big_count[parity ^ 1] = 0;
+    total = 0;
   }
-}
-
-__global__ void big_init_kernel(BigNode *big, int32_t count) {
-  for (int32_t b = blockIdx.x; b < count; b += gridDim.x) {
-    BigNode &B = big[b];
-    for (int i = threadIdx.x; i < 15; i += blockDim.x) B.cnt[i] = 0;
-    for (int i = threadIdx.x; i < 45; i += blockDim.x) {
-      B.bmn[i] = ford(1e32f);
-      B.bmx[i] = ford(-1e32f);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int32_t k0 = 0; k0 < have; k0 += kBuildBlock) {  // uniform: barriers inside
+    const int32_t k = k0 + (int32_t)threadIdx.x;
+    const int32_t id = k < have ? b.big[parity][k] : 0;
+    const BNode nd = b.nodes[id];
+    const int32_t mine = k < have ? (nd.count + kBigChunk - 1) / kBigChunk : 0;
+    int32_t incl = mine;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int32_t x = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += x;
     }
-    if (threadIdx.x < 6) {
-      B.cmn[threadIdx.x / 3][threadIdx.x % 3] = ford(1e32f);
-      B.cmx[threadIdx.x / 3][threadIdx.x % 3] = ford(-1e32f);
+    if (lane == 63) wave_tot[wave] = incl;
+    __syncthreads();
+    int32_t first = total + incl - mine;
+    for (int w = 0; w < wave; w++) first += wave_tot[w];
+    __syncthreads();
+    if (threadIdx.x == kBuildBlock - 1) total = first + mine;
+    if (k < have) {
+      BigNode &B = g.nodes[k];
+      B.id = id;
+      B.s = nd.left;
+      B.n = nd.count;
+      B.chunk_first = first;
+      B.chunk_count = mine;
     }
-  }
-}
-
-__global__ __launch_bounds__(kBuildBlock) void big_bin_kernel(BigNode *big, const BigChunk *__restrict__ chunks, const BNode *__restrict__ nodes,
-                                                              const int32_t *__restrict__ prim_idx, const float *__restrict__ aabb,
-                                                              const float *__restrict__ centroid) {
-  __shared__ int cnt[15], bmn[45], bmx[45];
-  const BigChunk ch = chunks[blockIdx.x];
-  BigNode &B = big[ch.big];
-  const NodeCands nc = node_cands(nodes[B.id]);
-  for (int i = threadIdx.x; i < 45; i += blockDim.x) {
-    if (i < 15) cnt[i] = 0;
-    bmn[i] = ford(1e32f);
-    bmx[i] = ford(-1e32f);
   }
   __syncthreads();
-  for (int i = ch.start + threadIdx.x; i < ch.end; i += kBuildBlock) bin_primitive(nc, aabb, centroid, prim_idx[i], cnt, bmn, bmx);
-  __syncthreads();
-  for (int i = threadIdx.x; i < 45; i += blockDim.x) {
-    if (i < 15 && cnt[i]) atomicAdd(&B.cnt[i], cnt[i]);
-    atomicMin(&B.bmn[i], bmn[i]);
-    atomicMax(&B.bmx[i], bmx[i]);
+  if (threadIdx.x == 0) *g.chunk_count = min(total, max_chunks);  // the nodes are disjoint: never more than the table holds
+  for (int32_t k = 0; k < have; k++) {
+    BigNode &B = g.nodes[k];
+    for (int32_t c = threadIdx.x; c < B.chunk_count && B.chunk_first + c < max_chunks; c += kBuildBlock) {
+      const int32_t at = B.s + c * kBigChunk;
+      g.chunks[B.chunk_first + c] = BigChunk{k, at, min(at + kBigChunk, B.s + B.n)};
+    }
+    for (int i = threadIdx.x; i < kBinWords; i += kBuildBlock) B.sum[i] = i % 6 < 3 ? ford(1e32f) : ford(-1e32f);
+    if (threadIdx.x < kCands) B.nl[threadIdx.x] = 0;
+    if (threadIdx.x < 12) B.box[threadIdx.x] = threadIdx.x % 6 < 3 ? ford(1e32f) : ford(-1e32f);
   }
 }
 
-__global__ void big_decide_kernel(BigNode *big, int32_t count, const BNode *__restrict__ nodes) {
-  const int32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= count) return;
-  BigNode &B = big[b];
-  const BNode nd = nodes[B.id];
-  const SplitChoice sc = decide_split(nd, node_cands(nd), B.cnt, B.bmn, B.bmx, B.n);
-  B.split = sc.split;
-  B.axis = sc.axis;
-  B.pos = sc.pos;
+// Levels without big nodes: only the next level's lists are emptied.
+__global__ void level_begin_kernel(BuildState b, int parity) {
+  if (threadIdx.x < kShards) b.mid_count[parity ^ 1][threadIdx.x * kShardStride] = 0;
+  if (threadIdx.x == 0) b.big_count[parity ^ 1] = 0;
 }
 
-__global__ __launch_bounds__(kBuildBlock) void big_classify_kernel(const BigNode *__restrict__ big, const BigChunk *__restrict__ chunks,
-                                                                   const int32_t *__restrict__ prim_idx, const float *__restrict__ centroid,
-                                                                   uint8_t *__restrict__ cls, int32_t *__restrict__ chunk_nl) {
-  __shared__ int nl;
-  const BigChunk ch = chunks[blockIdx.x];
-  const BigNode &B = big[ch.big];
+__global__ __launch_bounds__(kMidBlock) void big_bin_kernel(BuildState b, BigState g) {
+  __shared__ Bins bins;
+  if ((int32_t)blockIdx.x >= *g.chunk_count) return;
+  const BigChunk ch = g.chunks[blockIdx.x];
+  BigNode &B = g.nodes[ch.big];
+  const BNode nd = b.nodes[B.id];
+  bins_clear<kMidBlock>(bins);
+  __syncthreads();
+  bins_add<kMidBlock>(bins, b, ch.start, ch.end, nd.mn, nd.mx);
+  __syncthreads();
+  bins_reduce(bins);
+  __syncthreads();
+  for (int i = threadIdx.x; i < kBinWords; i += kMidBlock) {
+    if (i % 6 < 3)
+      atomicMin(&B.sum[i], bins.sum[i]);
+    else
+      atomicMax(&B.sum[i], bins.sum[i]);
+  }
+  if (threadIdx.x < kCands) atomicAdd(&B.nl[threadIdx.x], bins.nl[threadIdx.x]);
+}
+
+__global__ __launch_bounds__(64) void big_decide_kernel(BuildState b, BigState g, int parity) {
+  for (int32_t k = blockIdx.x; k < b.big_count[parity]; k += gridDim.x) {
+    BigNode &B = g.nodes[k];
+    const BNode nd = b.nodes[B.id];
+    const SplitChoice ch = bins_choose(B.sum, B.nl, nd.mn, nd.mx, B.n, B.box);
+    if (threadIdx.x == 0) {
+      B.split = ch.split ? 1 : 0;
+      B.axis = ch.axis;
+      B.pos = ch.pos;
+      B.fallback = ch.best < 0 ? 1 : 0;
+    }
+  }
+}
+
+__global__ __launch_bounds__(kBuildBlock) void big_classify_kernel(BuildState b, BigState g) {
+  __shared__ int nl, box[12];
+  if ((int32_t)blockIdx.x >= *g.chunk_count) return;
+  const BigChunk ch = g.chunks[blockIdx.x];
+  BigNode &B = g.nodes[ch.big];
   if (!B.split) return;
   if (threadIdx.x == 0) nl = 0;
+  if (threadIdx.x < 12) box[threadIdx.x] = threadIdx.x % 6 < 3 ? ford(1e32f) : ford(-1e32f);
   __syncthreads();
+  const bool fallback = B.fallback != 0;
+  SideBoxes sd;
+  sd.clear();
   int my = 0;
-  for (int i = ch.start + threadIdx.x; i < ch.end; i += kBuildBlock) {
-    const int bit = centroid[(size_t)prim_idx[i] * 3 + B.axis] < B.pos ? 1 : 0;
-    cls[i] = (uint8_t)bit;
+  for (int32_t i = ch.start + (int32_t)threadIdx.x; i < ch.end; i += kBuildBlock) {
+    const int32_t p = b.prim_idx[i];
+    const int bit = prim_centroid(b.prims, p, B.axis) < B.pos ? 1 : 0;
+    g.cls[i] = (uint8_t)bit;
     my += bit;
+    if (fallback) sd.add(bit != 0, b.prims[p].lo, b.prims[p].hi);
+  }
+  if (fallback) {  // split at x < 0: the child boxes come from the classes, not from a candidate
+    merge_sides(sd, box);
+    __syncthreads();
+    if (threadIdx.x < 12) {
+      if (threadIdx.x % 6 < 3)
+        atomicMin(&B.box[threadIdx.x], box[threadIdx.x]);
+      else
+        atomicMax(&B.box[threadIdx.x], box[threadIdx.x]);
+    }
   }
   atomicAdd(&nl, my);
   __syncthreads();
-  if (threadIdx.x == 0) chunk_nl[blockIdx.x] = nl;
+  if (threadIdx.x == 0) g.chunk_nl[blockIdx.x] = nl;
 }
 
-// Exclusive prefix of the chunk counts in chunk order, and the node's left count.
-__global__ void big_scan_kernel(BigNode *big, int32_t count, const int32_t *__restrict__ chunk_nl, int32_t *__restrict__ chunk_base) {
-  const int32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= count || !big[b].split) return;
-  int running = 0;
-  for (int32_t c = big[b].chunk_first; c < big[b].chunk_first + big[b].chunk_count; c++) {
-    chunk_base[c] = running;
-    running += chunk_nl[c];
+// Exclusive prefix of the chunk counts in chunk order, and the node's left count: one wave
+// per node.
+__global__ __launch_bounds__(64) void big_scan_kernel(BuildState b, BigState g, int parity) {
+  const int lane = threadIdx.x;
+  for (int32_t k = blockIdx.x; k < b.big_count[parity]; k += gridDim.x) {
+    BigNode &B = g.nodes[k];
+    if (!B.split) continue;
+    int running = 0;
+    for (int32_t c0 = 0; c0 < B.chunk_count; c0 += 64) {
+      const int32_t c = c0 + lane;
+      const int v = c < B.chunk_count ? g.chunk_nl[B.chunk_first + c] : 0;
+      int incl = v;
+      for (int d = 1; d < 64; d <<= 1) {
+        const int x = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += x;
+      }
+      if (c < B.chunk_count) g.chunk_base[B.chunk_first + c] = running + incl - v;
+      running += __shfl(incl, 63, 64);
+    }
+    if (lane == 0) B.nL = running;
   }
-  big[b].nL = running;
 }
 
-__global__ __launch_bounds__(kBuildBlock) void big_rank_kernel(const BigNode *__restrict__ big, const BigChunk *__restrict__ chunks,
-                                                               const uint8_t *__restrict__ cls, const int32_t *__restrict__ chunk_base,
-                                                               int32_t *__restrict__ rk, int32_t *__restrict__ hr_pos, int32_t *__restrict__ tl_pos) {
-  __shared__ BlockScan sc;
-  const BigChunk ch = chunks[blockIdx.x];
-  const BigNode &B = big[ch.big];
+__global__ __launch_bounds__(kBuildBlock) void big_rank_kernel(BigState g) {
+  __shared__ int wave_tot[kBuildBlock / 64];
+  if ((int32_t)blockIdx.x >= *g.chunk_count) return;
+  const BigChunk ch = g.chunks[blockIdx.x];
+  const BigNode &B = g.nodes[ch.big];
   if (!B.split) return;
-  const int s = B.s, nL = B.nL;
-  int running = chunk_base[blockIdx.x];
-  for (int base = ch.start; base < ch.end; base += kBuildBlock) {
-    const int i = base + threadIdx.x;
-    const int bit = (i < ch.end) ? cls[i] : 0;
-    int tot;
-    const int r_in = block_rank(bit, sc, tot);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int32_t s = B.s, nL = B.nL;
+  int running = g.chunk_base[blockIdx.x];
+  for (int32_t base = ch.start; base < ch.end; base += kBuildBlock) {
+    const int32_t i = base + (int32_t)threadIdx.x;
+    const bool bit = i < ch.end && g.cls[i] != 0;
+    const uint64_t m = __ballot(bit);
+    if (lane == 0) wave_tot[wave] = (int)__popcll(m);
+    __syncthreads();
+    int rankL = running + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+    for (int w = 0; w < kBuildBlock / 64; w++) {
+      rankL += w < wave ? wave_tot[w] : 0;
+      running += wave_tot[w];
+    }
+    __syncthreads();
     if (i < ch.end) {
-      const int rankL = running + r_in;
-      rk[i] = rankL;
+      g.rk[i] = rankL;
       const int rel = i - s;
-      if (rel < nL && !bit) hr_pos[s + (rel - rankL)] = rel;
-      if (rel >= nL && bit) tl_pos[s + (nL - 1 - rankL)] = rel;
+      if (rel < nL && !bit) g.hr_pos[s + (rel - rankL)] = rel;
+      if (rel >= nL && bit) g.tl_pos[s + (nL - 1 - rankL)] = rel;
     }
-    running += tot;
   }
 }
 
-__global__ __launch_bounds__(kBuildBlock) void big_scatter_kernel(const BigNode *__restrict__ big, const BigChunk *__restrict__ chunks,
-                                                                  const uint8_t *__restrict__ cls, const int32_t *__restrict__ rk,
-                                                                  const int32_t *__restrict__ hr_pos, const int32_t *__restrict__ tl_pos,
-                                                                  const int32_t *__restrict__ prim_idx, int32_t *__restrict__ tmp_idx) {
-  const BigChunk ch = chunks[blockIdx.x];
-  const BigNode &B = big[ch.big];
+__global__ __launch_bounds__(kBuildBlock) void big_scatter_kernel(BuildState b, BigState g) {
+  if ((int32_t)blockIdx.x >= *g.chunk_count) return;
+  const BigChunk ch = g.chunks[blockIdx.x];
+  const BigNode &B = g.nodes[ch.big];
   if (!B.split) return;
-  const int s = B.s, n = B.n, nL = B.nL;
-  const int LH = (nL < n) ? rk[s + nL] : nL;  // left-class elements inside H
+  const int32_t s = B.s, n = B.n, nL = B.nL;
+  const int LH = (nL < n) ? g.rk[s + nL] : nL;  // left-class elements inside H
   const int k = nL - LH;                         // right-class elements inside H
-  const int q = (k == 0) ? n : tl_pos[s + k - 1];
-  for (int i = ch.start + threadIdx.x; i < ch.end; i += kBuildBlock)
-    tmp_idx[s + partition_dest(i - s, cls[i], rk[i], nL, n, q, hr_pos + s, tl_pos + s)] = prim_idx[i];
+  const int q = (k == 0) ? n : g.tl_pos[s + k - 1];
+  for (int32_t i = ch.start + (int32_t)threadIdx.x; i < ch.end; i += kBuildBlock)
+    b.tmp_idx[s + partition_dest(i - s, g.cls[i] != 0, g.rk[i], nL, n, q, g.hr_pos + s, g.tl_pos + s)] = b.prim_idx[i];
 }
 
-__global__ __launch_bounds__(kBuildBlock) void big_copyback_kernel(BigNode *big, const BigChunk *__restrict__ chunks,
-                                                                   const int32_t *__restrict__ tmp_idx, int32_t *__restrict__ prim_idx,
-                                                                   const float *__restrict__ aabb) {
-  __shared__ int cmn[2][3], cmx[2][3];
-  const BigChunk ch = chunks[blockIdx.x];
-  BigNode &B = big[ch.big];
+// The new order, and (one thread per node) the children.
+__global__ __launch_bounds__(kBuildBlock) void big_finish_kernel(BuildState b, BigState g, int parity) {
+  if ((int32_t)blockIdx.x >= *g.chunk_count) return;
+  const BigChunk ch = g.chunks[blockIdx.x];
+  const BigNode &B = g.nodes[ch.big];
   if (!B.split) return;
-  if (threadIdx.x < 6) {
-    cmn[threadIdx.x / 3][threadIdx.x % 3] = ford(1e32f);
-    cmx[threadIdx.x / 3][threadIdx.x % 3] = ford(-1e32f);
-  }
-  __syncthreads();
-  int lmn[2][3], lmx[2][3];
-  for (int c2 = 0; c2 < 2; c2++)
-    for (int qq = 0; qq < 3; qq++) {
-      lmn[c2][qq] = ford(1e32f);
-      lmx[c2][qq] = ford(-1e32f);
-    }
-  for (int i = ch.start + threadIdx.x; i < ch.end; i += kBuildBlock) {
-    const int p = tmp_idx[i];
-    prim_idx[i] = p;
-    const int side = (i - B.s) < B.nL ? 0 : 1;
-    for (int qq = 0; qq < 3; qq++) {
-      lmn[side][qq] = min(lmn[side][qq], ford(aabb[(size_t)p * 6 + qq]));
-      lmx[side][qq] = max(lmx[side][qq], ford(aabb[(size_t)p * 6 + 3 + qq]));
-    }
-  }
-  for (int c2 = 0; c2 < 2; c2++)
-    for (int qq = 0; qq < 3; qq++) {
-      atomicMin(&cmn[c2][qq], lmn[c2][qq]);
-      atomicMax(&cmx[c2][qq], lmx[c2][qq]);
-    }
-  __syncthreads();
-  if (threadIdx.x < 6) {
-    atomicMin(&B.cmn[threadIdx.x / 3][threadIdx.x % 3], cmn[threadIdx.x / 3][threadIdx.x % 3]);
-    atomicMax(&B.cmx[threadIdx.x / 3][threadIdx.x % 3], cmx[threadIdx.x / 3][threadIdx.x % 3]);
-  }
+  for (int32_t i = ch.start + (int32_t)threadIdx.x; i < ch.end; i += kBuildBlock) b.prim_idx[i] = b.tmp_idx[i];
+  if (threadIdx.x != 0 || ch.start != B.s || B.nL == 0 || B.nL == B.n) return;
+  const int32_t d = node_depth(b, B.id);
+  write_children(b, B.id, b.nodes[B.id], B.s, B.n, B.nL, B.box, d);
+  note_depth(b, B.s, d + 1);
+  push_child(b, parity, 2 * (B.s + B.nL) - 1, B.s, B.nL);
+  push_child(b, parity, 2 * (B.s + B.nL), B.s + B.nL, B.n - B.nL);
 }
 
-__global__ void big_alloc_kernel(const BigNode *__restrict__ big, int32_t count, BNode *__restrict__ nodes, int32_t *__restrict__ node_counter,
-                                 int32_t *__restrict__ next_active, int32_t *__restrict__ next_count, int32_t *__restrict__ parent,
-                                 int32_t *__restrict__ depth) {
-  const int32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= count) return;
-  const BigNode &B = big[b];
-  if (!B.split || B.nL == 0 || B.nL == B.n) return;
-  const int32_t li = atomicAdd(node_counter, 2);
-  BNode L, R;
-  for (int qq = 0; qq < 3; qq++) {
-    L.mn[qq] = unford(B.cmn[0][qq]);
-    L.mx[qq] = unford(B.cmx[0][qq]);
-    R.mn[qq] = unford(B.cmn[1][qq]);
-    R.mx[qq] = unford(B.cmx[1][qq]);
-  }
-  L.left = B.s;
-  L.count = B.nL;
-  R.left = B.s + B.nL;
-  R.count = B.n - B.nL;
-  nodes[li] = L;
-  nodes[li + 1] = R;
-  parent[li] = parent[li + 1] = B.id;
-  depth[li] = depth[li + 1] = depth[B.id] + 1;
-  BNode P = nodes[B.id];
-  P.left = li;
-  P.count = 0;
-  nodes[B.id] = P;
-  const int32_t slot = atomicAdd(next_count, 2);
-  next_active[slot] = li;
-  next_active[slot + 1] = li + 1;
-}
-
-// Root bounds: min/max over every primitive AABB (update_aabb of node 0).
-__global__ void root_bounds_kernel(const float *__restrict__ aabb, uint32_t n, int *__restrict__ out) {
+// ------------------------------------------------------------- before and after the levels
+// Build records, the primitive order's start and the root's bounds (update_aabb of node 0).
+__global__ __launch_bounds__(kBuildBlock) void build_prims_kernel(const float *__restrict__ aabb, const float *__restrict__ centroid, uint32_t n,
+                                                                  BuildPrim *__restrict__ prims, int32_t *__restrict__ prim_idx,
+                                                                  uint8_t *__restrict__ used, int *__restrict__ bounds) {
   __shared__ int smn[3], smx[3];
   if (threadIdx.x < 3) {
     smn[threadIdx.x] = ford(1e32f);
@@ -545,118 +1087,236 @@ __global__ void root_bounds_kernel(const float *__restrict__ aabb, uint32_t n, i
   }
   __syncthreads();
   int mn[3] = {ford(1e32f), ford(1e32f), ford(1e32f)}, mx[3] = {ford(-1e32f), ford(-1e32f), ford(-1e32f)};
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    BuildPrim p;
     for (int q = 0; q < 3; q++) {
-      mn[q] = min(mn[q], ford(aabb[(size_t)i * 6 + q]));
-      mx[q] = max(mx[q], ford(aabb[(size_t)i * 6 + 3 + q]));
+      p.lo[q] = ford(aabb[(size_t)i * 6 + q]);
+      p.hi[q] = ford(aabb[(size_t)i * 6 + 3 + q]);
+      mn[q] = min(mn[q], p.lo[q]);
+      mx[q] = max(mx[q], p.hi[q]);
+      p.pad[q] = 0;
     }
-  for (int q = 0; q < 3; q++) {
-    atomicMin(&smn[q], mn[q]);
-    atomicMax(&smx[q], mx[q]);
+    p.cx = centroid[(size_t)i * 3];
+    p.cy = centroid[(size_t)i * 3 + 1];
+    p.cz = centroid[(size_t)i * 3 + 2];
+    prims[i] = p;
+    prim_idx[i] = (int32_t)i;
+    used[i] = 0;
   }
+  for (int d = 1; d < 64; d <<= 1)
+    for (int q = 0; q < 3; q++) {
+      mn[q] = min(mn[q], __shfl_xor(mn[q], d, 64));
+      mx[q] = max(mx[q], __shfl_xor(mx[q], d, 64));
+    }
+  if ((threadIdx.x & 63) == 0)
+    for (int q = 0; q < 3; q++) {
+      atomicMin(&smn[q], mn[q]);
+      atomicMax(&smx[q], mx[q]);
+    }
   __syncthreads();
   if (threadIdx.x < 3) {
-    atomicMin(&out[threadIdx.x], smn[threadIdx.x]);
-    atomicMax(&out[3 + threadIdx.x], smx[threadIdx.x]);
+    atomicMin(&bounds[threadIdx.x], smn[threadIdx.x]);
+    atomicMax(&bounds[3 + threadIdx.x], smx[threadIdx.x]);
   }
 }
 
-// Binary leaf holding each prim_idx position (the tie rule of the traversal needs it).
-// Per binary leaf: the leaf of each of its positions, and its size in the first traversal
-// record's b.w.
-__global__ void leaf_of_position_kernel(const BNode *__restrict__ nodes, uint32_t count, int32_t *__restrict__ leaf_of_pos,
-                                        TriMT *__restrict__ tri_leaf) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
-    const BNode nd = nodes[i];
-    for (int32_t k = 0; k < nd.count; k++) leaf_of_pos[nd.left + k] = (int32_t)i;
-    if (nd.count > 0) tri_leaf[nd.left].b.w = __builtin_bit_cast(float, nd.count);
-  }
-}
-
-__global__ void init_root_kernel(BNode *nodes, const int *bounds, uint32_t n, int32_t *prim_idx, int32_t *counters, int32_t *parent, int32_t *depth) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) prim_idx[i] = (int32_t)i;
-  if (i == 0) {
-    BNode r;
-    for (int q = 0; q < 3; q++) {
-      r.mn[q] = unford(bounds[q]);
-      r.mx[q] = unford(bounds[3 + q]);
-    }
-    r.left = 0;
-    r.count = (int32_t)n;
-    nodes[0] = r;
-    parent[0] = -1;
-    depth[0] = 0;
-    counters[0] = 1;  // node counter
-    counters[1] = 0;  // next level size
-  }
-}
-
-__global__ void reset_level_counters_kernel(int32_t *counters) {
-  counters[1] = 0;
-  counters[4] = 0;
-  counters[5] = 0;
-}
-
-__global__ void init_bounds_kernel(int *b) {
+// Counters at zero, empty bounds.
+__global__ void build_init_kernel(int32_t *counters, int32_t words, int *bounds) {
+  for (int32_t i = threadIdx.x; i < words; i += blockDim.x) counters[i] = 0;
   if (threadIdx.x < 3) {
-    b[threadIdx.x] = ford(1e32f);
-    b[3 + threadIdx.x] = ford(-1e32f);
+    bounds[threadIdx.x] = ford(1e32f);
+    bounds[3 + threadIdx.x] = ford(-1e32f);
+  }
+}
+
+__global__ void root_kernel(BuildState b, const int *bounds) {
+  BNode r;
+  for (int q = 0; q < 3; q++) {
+    r.mn[q] = unford(bounds[q]);
+    r.mx[q] = unford(bounds[3 + q]);
+  }
+  r.left = 0;
+  r.count = b.n;
+  b.nodes[0] = r;
+  push_child(b, 1, 0, 0, b.n);  // level 0 has parity 0
+}
+
+// Packing: rank[b] = used boundaries below b. Three launches: counts per workgroup of
+// kPackChunk boundaries, their prefix (one workgroup), the ranks.
+constexpr int kPackChunk = 2048;
+__global__ __launch_bounds__(kBuildBlock) void pack_count_kernel(const uint8_t *__restrict__ used, uint32_t n, int32_t *__restrict__ chunk_sum) {
+  __shared__ int sum;
+  if (threadIdx.x == 0) sum = 0;
+  __syncthreads();
+  int my = 0;
+  for (uint32_t i = blockIdx.x * kPackChunk + threadIdx.x; i < min(n, (blockIdx.x + 1u) * (uint32_t)kPackChunk); i += kBuildBlock) my += used[i];
+  for (int d = 1; d < 64; d <<= 1) my += __shfl_xor(my, d, 64);
+  if ((threadIdx.x & 63) == 0) atomicAdd(&sum, my);
+  __syncthreads();
+  if (threadIdx.x == 0) chunk_sum[blockIdx.x] = sum;
+}
+
+__global__ __launch_bounds__(kBuildBlock) void pack_scan_kernel(int32_t *chunk_sum, int32_t chunks, int32_t *total, const int32_t *depth_max,
+                                                                int32_t *depth_out) {
+  __shared__ int wave_tot[kBuildBlock / 64], deepest;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x == 0) deepest = 0;
+  int running = 0;
+  for (int32_t c0 = 0; c0 < chunks; c0 += kBuildBlock) {
+    const int32_t c = c0 + (int32_t)threadIdx.x;
+    const int v = c < chunks ? chunk_sum[c] : 0;
+    int incl = v;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int x = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += x;
+    }
+    if (lane == 63) wave_tot[wave] = incl;
+    __syncthreads();
+    int base = running;
+    for (int w = 0; w < kBuildBlock / 64; w++) {
+      base += w < wave ? wave_tot[w] : 0;
+      running += wave_tot[w];
+    }
+    if (c < chunks) chunk_sum[c] = base + incl - v;
+    __syncthreads();
+  }
+  if (threadIdx.x < kShards) atomicMax(&deepest, depth_max[threadIdx.x * kShardStride]);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    *total = running;
+    *depth_out = deepest;
+  }
+}
+
+__global__ __launch_bounds__(kBuildBlock) void pack_rank_kernel(const uint8_t *__restrict__ used, uint32_t n, const int32_t *__restrict__ chunk_base,
+                                                                int32_t *__restrict__ rank) {
+  __shared__ int wave_tot[kBuildBlock / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t end = min(n, (blockIdx.x + 1u) * (uint32_t)kPackChunk);
+  int running = chunk_base[blockIdx.x];
+  for (uint32_t base = blockIdx.x * kPackChunk; base < end; base += kBuildBlock) {
+    const uint32_t i = base + threadIdx.x;
+    const uint64_t m = __ballot(i < end && used[i] != 0);
+    if (lane == 0) wave_tot[wave] = (int)__popcll(m);
+    __syncthreads();
+    int r = running + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+    for (int w = 0; w < kBuildBlock / 64; w++) {
+      r += w < wave ? wave_tot[w] : 0;
+      running += wave_tot[w];
+    }
+    __syncthreads();
+    if (i < end) rank[i] = r;
+  }
+}
+
+__device__ __forceinline__ int32_t packed_id(const int32_t *rank, int32_t id) { return id == 0 ? 0 : 1 + 2 * rank[(id + 1) >> 1] + ((id & 1) ? 0 : 1); }
+
+// The pair of every used boundary (and the root) into the packed arrays; a leaf also names
+// itself to its positions (the traversal's tie rule) and its first traversal record gets its
+// size (b.w).
+__global__ __launch_bounds__(kBuildBlock) void pack_nodes_kernel(BuildState b, const int32_t *__restrict__ rank, BNode *__restrict__ out,
+                                                                 int32_t *__restrict__ parent, int32_t *__restrict__ depth,
+                                                                 int32_t *__restrict__ leaf_of_pos, TriMT *__restrict__ tri_leaf) {
+  for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < 2 * (int64_t)b.n - 1; k += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t id = (int32_t)k, at = (id + 1) >> 1;  // id 0: the root; 2b-1, 2b: boundary b's pair
+    if (id != 0 && !b.used[at]) continue;
+    const int32_t to = packed_id(rank, id);
+    BNode nd = b.nodes[id];
+    if (nd.count > 0) {
+      for (int32_t j = 0; j < nd.count; j++) leaf_of_pos[nd.left + j] = to;
+      tri_leaf[nd.left].b.w = __builtin_bit_cast(float, nd.count);
+    } else {
+      nd.left = 1 + 2 * rank[nd.left];
+    }
+    out[to] = nd;
+    parent[to] = id == 0 ? -1 : packed_id(rank, b.pair_parent[at]);
+    depth[to] = id == 0 ? 0 : b.pair_depth[at];
   }
 }
 
 // ---------------------------------------------------------------- collapse
 
-// One thread per frontier entry: binary inner node -> 4-wide node by repeatedly opening
-// the child with the largest half area.
-__global__ void collapse_kernel(const int32_t *__restrict__ frontier_bin, const int32_t *__restrict__ frontier_slot, int32_t count,
-                                const BNode *__restrict__ bn, Node4 *__restrict__ out, int32_t *__restrict__ wide_counter,
-                                int32_t *__restrict__ next_bin, int32_t *__restrict__ next_slot, int32_t *__restrict__ next_count) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= count) return;
-  const int32_t b = frontier_bin[t];
-  const int32_t slot = frontier_slot[t];
-  int32_t ch[4];
-  const int m = collapse_children(bn, b, ch);
-  Node4 nd;
-  set_node_boxes(nd, bn, ch, m);
-  for (int k = 0; k < 4; k++) {
-    if (k >= m) {
-      nd.child[k] = -1;  // empty slot, never entered
-      continue;
+// One level of the collapse, a thread per wide node of the level: binary inner node -> 4-wide
+// node by repeatedly opening the child with the largest half area. Wide ids are breadth-first:
+// level L holds ids start[L] .. start[L] + count[L] - 1 (rings of kCollapseRing levels), and a
+// workgroup takes the ids of its nodes' inner children in one piece, so siblings are adjacent
+// and the level costs one atomic per workgroup. The node is written twice, on its byte grid for
+// the per-ray walk and with the planes decoded (grid_plane, the value the walks compute) for
+// the wave-coherent one.
+constexpr int kCollapseRing = 64;
+__global__ __launch_bounds__(kBuildBlock) void collapse_kernel(int level, int32_t *start, int32_t *count, int32_t *__restrict__ front,
+                                                               const BNode *__restrict__ bn, Node4 *__restrict__ out, Node4F *__restrict__ outf) {
+  __shared__ int wave_tot[kBuildBlock / 64], block_base;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int32_t lo = start[level % kCollapseRing], have = count[level % kCollapseRing], hi = lo + have;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    start[(level + 1) % kCollapseRing] = hi;
+    count[(level + 2) % kCollapseRing] = 0;
+  }
+  for (int32_t t0 = lo + (int32_t)blockIdx.x * kBuildBlock; t0 < hi; t0 += (int32_t)gridDim.x * kBuildBlock) {  // uniform per workgroup
+    const int32_t t = t0 + (int32_t)threadIdx.x;
+    Node4 nd;
+    int32_t ch[4];
+    bool inner[4] = {false, false, false, false};
+    int mine = 0;
+    if (t < hi) {
+      const int m = collapse_children(bn, front[t], ch);
+      set_node_boxes(nd, bn, ch, m);
+      for (int k = 0; k < 4; k++) {
+        nd.child[k] = -1;  // empty slot, never entered
+        if (k >= m) continue;
+        const BNode &c = bn[ch[k]];
+        inner[k] = c.count == 0;
+        mine += inner[k] ? 1 : 0;
+        if (!inner[k]) nd.child[k] = leaf_ref(c.left);
+      }
     }
-    const BNode &c = bn[ch[k]];
-    if (c.count > 0) {
-      nd.child[k] = leaf_ref(c.left);
-    } else {
-      const int32_t w = atomicAdd(wide_counter, 1);
-      nd.child[k] = w;
-      const int32_t j = atomicAdd(next_count, 1);
-      next_bin[j] = ch[k];
-      next_slot[j] = w;
+    int incl = mine;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int x = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += x;
+    }
+    if (lane == 63) wave_tot[wave] = incl;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int tot = 0;
+      for (int w = 0; w < kBuildBlock / 64; w++) tot += wave_tot[w];
+      block_base = tot ? atomicAdd(&count[(level + 1) % kCollapseRing], tot) : 0;
+    }
+    __syncthreads();
+    int32_t w = hi + block_base + incl - mine;
+    for (int v = 0; v < wave; v++) w += wave_tot[v];
+    __syncthreads();
+    if (t < hi) {
+      for (int k = 0; k < 4; k++)
+        if (inner[k]) {
+          front[w] = ch[k];
+          nd.child[k] = w++;
+        }
+      out[t] = nd;
+      const float org[3] = {nd.orgx, nd.orgy, nd.orgz}, step[3] = {nd.stepx, nd.stepy, nd.stepz};
+      const uint32_t qmn[3] = {nd.qminx, nd.qminy, nd.qminz}, qmx[3] = {nd.qmaxx, nd.qmaxy, nd.qmaxz};
+      Node4F f;
+      for (int a = 0; a < 3; a++)
+        for (int k = 0; k < 4; k++) {
+          f.plane[a][0][k] = grid_plane((qmn[a] >> (8 * k)) & 255u, step[a], org[a]);
+          f.plane[a][1][k] = grid_plane((qmx[a] >> (8 * k)) & 255u, step[a], org[a]);
+        }
+      for (int k = 0; k < 4; k++) {
+        f.child[k] = nd.child[k];
+        f.pad[k] = 0;
+      }
+      outf[t] = f;
     }
   }
-  out[slot] = nd;
 }
 
-// Node4 -> Node4F: every plane decoded with grid_plane, the value the walks compute.
-__global__ void decode_nodes_kernel(const Node4 *__restrict__ in, Node4F *__restrict__ out, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const Node4 nd = in[i];
-  const float org[3] = {nd.orgx, nd.orgy, nd.orgz}, step[3] = {nd.stepx, nd.stepy, nd.stepz};
-  const uint32_t qmn[3] = {nd.qminx, nd.qminy, nd.qminz}, qmx[3] = {nd.qmaxx, nd.qmaxy, nd.qmaxz};
-  Node4F f;
-  for (int a = 0; a < 3; a++)
-    for (int k = 0; k < 4; k++) {
-      f.plane[a][0][k] = grid_plane((qmn[a] >> (8 * k)) & 255u, step[a], org[a]);
-      f.plane[a][1][k] = grid_plane((qmx[a] >> (8 * k)) & 255u, step[a], org[a]);
-    }
-  for (int k = 0; k < 4; k++) {
-    f.child[k] = nd.child[k];
-    f.pad[k] = 0;
+__global__ void collapse_begin_kernel(int32_t *start, int32_t *count, int32_t *front) {
+  for (int i = threadIdx.x; i < kCollapseRing; i += blockDim.x) {
+    start[i] = 0;
+    count[i] = i == 0 ? 1 : 0;
   }
-  out[i] = f;
+  if (threadIdx.x == 0) front[0] = 0;
 }
 
 __global__ void gather_leaf_tris(const int32_t *__restrict__ prim_idx, const TriMT *__restrict__ tri, TriMT *__restrict__ out, uint32_t n) {
@@ -665,6 +1325,177 @@ __global__ void gather_leaf_tris(const int32_t *__restrict__ prim_idx, const Tri
 }
 
 uint32_t traversal_stack_bound(const nova_hip_ctx *ctx) { return 3u * ctx->bvh_info.wide_depth + 4u; }
+
+// One build's temporaries, carved from one allocation in 256-byte pieces (with base null: the
+// bytes they need).
+struct BuildTemps {
+  char *base;
+  size_t used = 0;
+  template <class T>
+  T *take(size_t count) {
+    const size_t at = used;
+    used += (count * sizeof(T) + 255) / 256 * 256;
+    return base ? reinterpret_cast<T *>(base + at) : nullptr;
+  }
+};
+
+struct BuildPlan {
+  BuildState b;
+  BigState g;
+  int32_t *rank, *chunk_sum, *front, *counters, *ring_start, *ring_count, *results;
+  int *bounds;
+  int32_t counter_words;
+  int32_t max_chunks, pack_chunks;
+};
+
+static size_t carve_build(BuildPlan &P, char *base, uint32_t n) {
+  BuildTemps t{base};
+  int shift = 0;
+  while (((n - 1) >> shift) >= (uint32_t)kShards) shift++;
+  const size_t list = (size_t)kShards << shift;
+  const int32_t max_big = (int32_t)(n / kBigNode + 1);
+  P.max_chunks = (int32_t)(n / kBigChunk + max_big + 1);
+  P.pack_chunks = (int32_t)((n + kPackChunk - 1) / kPackChunk);
+  P.b.prims = t.take<BuildPrim>(n);
+  P.b.prim_idx = nullptr;
+  P.b.tmp_idx = t.take<int32_t>(n);
+  P.b.nodes = t.take<BNode>(2 * (size_t)n);
+  P.b.pair_parent = t.take<int32_t>(n);
+  P.b.pair_depth = t.take<int32_t>(n);
+  P.b.used = t.take<uint8_t>(n);
+  P.b.mid[0] = t.take<int32_t>(list);
+  P.b.mid[1] = t.take<int32_t>(list);
+  P.b.sub = t.take<int32_t>(list);
+  P.b.big[0] = t.take<int32_t>((size_t)max_big);
+  P.b.big[1] = t.take<int32_t>((size_t)max_big);
+  // counters: two level lists, the subtree list and the depths (kShards lines each), then the rest
+  P.counter_words = 4 * kShards * kShardStride + 64 + 2 * kCollapseRing;
+  P.counters = t.take<int32_t>((size_t)P.counter_words);
+  P.b.mid_count[0] = P.counters;
+  P.b.mid_count[1] = P.counters ? P.counters + kShards * kShardStride : nullptr;
+  P.b.sub_count = P.counters ? P.counters + 2 * kShards * kShardStride : nullptr;
+  P.b.depth_max = P.counters ? P.counters + 3 * kShards * kShardStride : nullptr;
+  int32_t *rest = P.counters ? P.counters + 4 * kShards * kShardStride : nullptr;
+  P.b.big_count = rest;                       // [2]
+  P.g.chunk_count = rest ? rest + 2 : nullptr;
+  P.results = rest ? rest + 4 : nullptr;      // splits, depth of the deepest node
+  P.ring_start = rest ? rest + 64 : nullptr;
+  P.ring_count = rest ? rest + 64 + kCollapseRing : nullptr;
+  P.b.shard_shift = shift;
+  P.b.n = (int32_t)n;
+  P.g.nodes = t.take<BigNode>((size_t)max_big);
+  P.g.chunks = t.take<BigChunk>((size_t)P.max_chunks);
+  P.g.chunk_nl = t.take<int32_t>((size_t)P.max_chunks);
+  P.g.chunk_base = t.take<int32_t>((size_t)P.max_chunks);
+  P.g.cls = t.take<uint8_t>(n);
+  P.g.rk = t.take<int32_t>(n);
+  P.g.hr_pos = t.take<int32_t>(n);
+  P.g.tl_pos = t.take<int32_t>(n);
+  P.rank = t.take<int32_t>(n);
+  P.chunk_sum = t.take<int32_t>((size_t)P.pack_chunks);
+  P.front = t.take<int32_t>(n);
+  P.bounds = t.take<int>(6);
+  return t.used;
+}
+
+// The levels, the packed nodes and the collapse, into buffers of ctx that the caller has
+// allocated (the wide nodes are allocated here, once the node count is known).
+static int run_build(nova_hip_ctx *ctx, BuildPlan &P, uint32_t n, hipStream_t s) {
+  BuildState &b = P.b;
+  BigState &g = P.g;
+  const uint32_t kGroup = 4;  // levels per look at the counters
+  hipLaunchKernelGGL(build_init_kernel, dim3(1), dim3(1024), 0, s, P.counters, P.counter_words, P.bounds);
+  hipLaunchKernelGGL(build_prims_kernel, dim3(std::min<uint32_t>(1024, (n + kBuildBlock - 1) / kBuildBlock)), dim3(kBuildBlock), 0, s, ctx->prim_aabb,
+                     ctx->prim_centroid, n, const_cast<BuildPrim *>(b.prims), b.prim_idx, b.used, P.bounds);
+  hipLaunchKernelGGL(root_kernel, dim3(1), dim3(1), 0, s, b, P.bounds);
+  NOVA_HIP_CHECK(ctx, hipGetLastError());
+  // one workgroup per middle node and turn; at least one per shard
+  const uint32_t mid_blocks = (uint32_t)std::min<size_t>(1024, ((size_t)n / kSubPrims + kShards) / kShards * kShards);
+  bool big = n > (uint32_t)kBigNode, mid = n > (uint32_t)kSubPrims;
+  uint32_t level = 0;
+  std::vector<int32_t> words((size_t)(2 * kShards * kShardStride));
+  while (big || mid) {
+    if (level > n) return set_error(ctx, NOVA_HIP_DEVICE_ERROR, "BVH build did not converge");
+    for (uint32_t k = 0; k < kGroup; k++, level++) {
+      const int parity = (int)(level & 1u);
+      if (big) {
+        const dim3 grid((unsigned)P.max_chunks);
+        const unsigned nb = std::min<unsigned>((unsigned)(n / kBigNode + 1), 1024u);
+        hipLaunchKernelGGL(big_setup_kernel, dim3(1), dim3(kBuildBlock), 0, s, b, g, parity, P.max_chunks);
+        hipLaunchKernelGGL(big_bin_kernel, grid, dim3(kMidBlock), 0, s, b, g);
+        hipLaunchKernelGGL(big_decide_kernel, dim3(nb), dim3(64), 0, s, b, g, parity);
+        hipLaunchKernelGGL(big_classify_kernel, grid, dim3(kBuildBlock), 0, s, b, g);
+        hipLaunchKernelGGL(big_scan_kernel, dim3(nb), dim3(64), 0, s, b, g, parity);
+        hipLaunchKernelGGL(big_rank_kernel, grid, dim3(kBuildBlock), 0, s, g);
+        hipLaunchKernelGGL(big_scatter_kernel, grid, dim3(kBuildBlock), 0, s, b, g);
+        hipLaunchKernelGGL(big_finish_kernel, grid, dim3(kBuildBlock), 0, s, b, g, parity);
+      } else {
+        hipLaunchKernelGGL(level_begin_kernel, dim3(1), dim3(64), 0, s, b, parity);
+      }
+      hipLaunchKernelGGL(mid_level_kernel, dim3(mid_blocks), dim3(kMidBlock), 0, s, b, parity, g.hr_pos, g.tl_pos);
+      NOVA_HIP_CHECK(ctx, hipGetLastError());
+    }
+    // what the next level holds
+    int32_t nbig[2] = {0, 0};
+    NOVA_HIP_CHECK(ctx, hipMemcpyAsync(nbig, b.big_count, sizeof(nbig), hipMemcpyDeviceToHost, s));
+    NOVA_HIP_CHECK(ctx, hipMemcpyAsync(words.data(), b.mid_count[0], words.size() * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    NOVA_HIP_CHECK(ctx, hipStreamSynchronize(s));
+    big = nbig[level & 1u] > 0;
+    mid = big;
+    for (int k = 0; k < kShards; k++) mid = mid || words[(size_t)((level & 1u) * kShards + k) * kShardStride] > 0;
+  }
+  const uint32_t sub_blocks = (uint32_t)std::min<size_t>(4096, ((size_t)n / 64 + kShards) / kShards * kShards);
+  hipLaunchKernelGGL(subtree_kernel, dim3(sub_blocks), dim3(kSubBlock), 0, s, b);
+  hipLaunchKernelGGL(gather_leaf_tris, dim3((n + 255) / 256), dim3(256), 0, s, b.prim_idx, ctx->tri_world, ctx->tri_leaf, n);
+  hipLaunchKernelGGL(pack_count_kernel, dim3((unsigned)P.pack_chunks), dim3(kBuildBlock), 0, s, b.used, n, P.chunk_sum);
+  hipLaunchKernelGGL(pack_scan_kernel, dim3(1), dim3(kBuildBlock), 0, s, P.chunk_sum, P.pack_chunks, P.results, b.depth_max, P.results + 1);
+  hipLaunchKernelGGL(pack_rank_kernel, dim3((unsigned)P.pack_chunks), dim3(kBuildBlock), 0, s, b.used, n, P.chunk_sum, P.rank);
+  hipLaunchKernelGGL(pack_nodes_kernel, dim3(std::min<uint32_t>(8192, (2 * n + 255) / 256)), dim3(kBuildBlock), 0, s, b, P.rank, ctx->bnodes, ctx->bparent,
+                     ctx->bdepth, ctx->leaf_of_pos, ctx->tri_leaf);
+  NOVA_HIP_CHECK(ctx, hipGetLastError());
+  int32_t res[2] = {0, 0};  // splits, deepest level
+  NOVA_HIP_CHECK(ctx, hipMemcpyAsync(res, P.results, sizeof(res), hipMemcpyDeviceToHost, s));
+  NOVA_HIP_CHECK(ctx, hipStreamSynchronize(s));
+  const uint32_t splits = (uint32_t)res[0], depth = (uint32_t)res[1] + 1;
+  if (splits >= n) return set_error(ctx, NOVA_HIP_DEVICE_ERROR, "BVH build: inconsistent node count");
+  ctx->bnode_count = 2 * splits + 1;
+
+  // ---- collapse to 4-wide: every wide node stands for an inner node of the binary tree
+  const size_t wide_max = std::max<size_t>(1, splits);
+  NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->nodes4, wide_max * sizeof(Node4)));
+  NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->nodes4f, wide_max * sizeof(Node4F)));
+  hipLaunchKernelGGL(collapse_begin_kernel, dim3(1), dim3(64), 0, s, P.ring_start, P.ring_count, P.front);
+  uint32_t wdepth = 0, wide = 0, wl = 0;
+  int32_t ring[2 * kCollapseRing] = {};
+  for (bool more = true; more;) {
+    if (wl > depth + kCollapseRing) return set_error(ctx, NOVA_HIP_DEVICE_ERROR, "BVH collapse did not converge");
+    // a wide level opens two binary levels or more where the tree is full: most trees end within
+    // the first group
+    const uint32_t group = wl == 0 ? std::min<uint32_t>(depth / 2 + 1, kCollapseRing / 2) : 4;
+    const uint32_t first = wl;
+    for (uint32_t k = 0; k < group; k++, wl++) {
+      const size_t most = wl < 16 ? std::min<size_t>(wide_max, (size_t)1 << (2 * wl)) : wide_max;
+      hipLaunchKernelGGL(collapse_kernel, dim3((unsigned)std::min<size_t>(2048, (most + kBuildBlock - 1) / kBuildBlock)), dim3(kBuildBlock), 0, s, (int)wl,
+                         P.ring_start, P.ring_count, P.front, ctx->bnodes, ctx->nodes4, ctx->nodes4f);
+    }
+    NOVA_HIP_CHECK(ctx, hipGetLastError());
+    NOVA_HIP_CHECK(ctx, hipMemcpyAsync(ring, P.ring_start, sizeof(ring), hipMemcpyDeviceToHost, s));
+    NOVA_HIP_CHECK(ctx, hipStreamSynchronize(s));
+    for (uint32_t l = first; l < wl; l++)
+      if (ring[kCollapseRing + l % kCollapseRing] > 0) {
+        wdepth = l + 1;
+        wide = (uint32_t)(ring[l % kCollapseRing] + ring[kCollapseRing + l % kCollapseRing]);
+      }
+    more = ring[kCollapseRing + wl % kCollapseRing] > 0;
+  }
+  ctx->bvh_info.primitive_count = n;
+  ctx->bvh_info.binary_nodes = ctx->bnode_count;
+  ctx->bvh_info.binary_depth = depth;
+  ctx->bvh_info.wide_nodes = wide;
+  ctx->bvh_info.wide_depth = wdepth;
+  ctx->bvh_info.leaves = splits + 1;  // every split has two children
+  return NOVA_HIP_SUCCESS;
+}
 
 }  // namespace nova_hip
 
@@ -678,6 +1509,7 @@ extern "C" int nova_hip_bvh_build(nova_hip_ctx *ctx, int build_candidates, nova_
   hipStream_t s = (hipStream_t)stream;
   NOVA_HIP_CHECK(ctx, hipSetDevice(ctx->device));
   const uint32_t n = ctx->prim_count;
+  if (n > 1u << 30) return set_error(ctx, NOVA_HIP_INVALID_ARGUMENT, "too many primitives");
   const size_t maxnodes = 2 * (size_t)n - 1;
   (void)hipDeviceSynchronize();  // render work queued without a wait may still read the old tree
   for (void **p : {(void **)&ctx->prim_idx, (void **)&ctx->bnodes, (void **)&ctx->nodes4, (void **)&ctx->nodes4f, (void **)&ctx->tri_leaf,
@@ -692,155 +1524,31 @@ extern "C" int nova_hip_bvh_build(nova_hip_ctx *ctx, int build_candidates, nova_
   NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->bparent, maxnodes * sizeof(int32_t)));
   NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->bdepth, maxnodes * sizeof(int32_t)));
   NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->leaf_of_pos, (size_t)n * sizeof(int32_t)));
+  NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->tri_leaf, (size_t)n * sizeof(TriMT)));
   NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->tie, sizeof(TieTables)));
   const TieTables tie{ctx->bnodes, ctx->bparent, ctx->bdepth, ctx->leaf_of_pos, ctx->xf_inv};
   NOVA_HIP_CHECK(ctx, hipMemcpy(ctx->tie, &tie, sizeof(TieTables), hipMemcpyHostToDevice));
-
-  // temporaries
-  int32_t *tmp_idx, *rk, *hr, *tl, *act0, *act1, *counters;
-  uint8_t *cls;
-  int *bounds;
-  NOVA_HIP_CHECK(ctx, hipMalloc(&tmp_idx, n * sizeof(int32_t)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&rk, n * sizeof(int32_t)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&hr, n * sizeof(int32_t)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&tl, n * sizeof(int32_t)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&act0, (n + 2) * sizeof(int32_t)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&act1, (n + 2) * sizeof(int32_t)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&counters, 8 * sizeof(int32_t)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&cls, n));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&bounds, 6 * sizeof(int)));
+  BuildPlan P{};
+  char *temps = nullptr;
+  NOVA_HIP_CHECK(ctx, hipMalloc(&temps, carve_build(P, nullptr, n)));
+  carve_build(P, temps, n);
+  P.b.prim_idx = ctx->prim_idx;
 
   hipEvent_t ev0, ev1;
   NOVA_HIP_CHECK(ctx, hipEventCreate(&ev0));
   NOVA_HIP_CHECK(ctx, hipEventCreate(&ev1));
   NOVA_HIP_CHECK(ctx, hipEventRecord(ev0, s));
-
-  hipLaunchKernelGGL(init_bounds_kernel, dim3(1), dim3(64), 0, s, bounds);
-  hipLaunchKernelGGL(root_bounds_kernel, dim3(std::min<uint32_t>(1024, (n + 255) / 256)), dim3(256), 0, s, ctx->prim_aabb, n, bounds);
-  hipLaunchKernelGGL(init_root_kernel, dim3((n + 255) / 256), dim3(256), 0, s, ctx->bnodes, bounds, n, ctx->prim_idx, counters, ctx->bparent,
-                     ctx->bdepth);
-  const int32_t zero = 0;
-  NOVA_HIP_CHECK(ctx, hipMemcpyAsync(act0, &zero, sizeof(int32_t), hipMemcpyHostToDevice, s));
-  int32_t active = 1;
-  uint32_t depth = 0;
-  int32_t *cur = act0, *nxt = act1;
-  // per-level work lists of the big-node path
-  const int32_t max_big = (int32_t)(n / kBigNode + 1), max_chunks = (int32_t)(n / kBigChunk + max_big + 1);
-  BigNode *big = nullptr;
-  BigChunk *chunks = nullptr;
-  int32_t *small = nullptr, *chunk_nl = nullptr, *chunk_base = nullptr;
-  NOVA_HIP_CHECK(ctx, hipMalloc(&big, max_big * sizeof(BigNode)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&chunks, max_chunks * sizeof(BigChunk)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&small, (n + 2) * sizeof(int32_t)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&chunk_nl, max_chunks * sizeof(int32_t)));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&chunk_base, max_chunks * sizeof(int32_t)));
-  std::vector<BigNode> hbig;
-  std::vector<BigChunk> hchunks;
-  while (active > 0) {
-    if (depth > n) return set_error(ctx, NOVA_HIP_DEVICE_ERROR, "BVH build did not converge");
-    // counters: [1] next level size, [4] big nodes, [5] small nodes
-    hipLaunchKernelGGL(reset_level_counters_kernel, dim3(1), dim3(1), 0, s, counters);
-    hipLaunchKernelGGL(split_active_kernel, dim3(std::min<int32_t>((active + 255) / 256, 4096)), dim3(256), 0, s, cur, active, ctx->bnodes, big,
-                       counters + 4, small, counters + 5);
-    NOVA_HIP_CHECK(ctx, hipGetLastError());
-    int32_t split_counts[2] = {0, 0};
-    NOVA_HIP_CHECK(ctx, hipMemcpyAsync(split_counts, counters + 4, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    NOVA_HIP_CHECK(ctx, hipStreamSynchronize(s));
-    const int32_t nbig = split_counts[0], nsmall = split_counts[1];
-    if (nbig > max_big || nsmall > active) return set_error(ctx, NOVA_HIP_DEVICE_ERROR, "BVH build: inconsistent level split");
-    if (nsmall > 0)
-      hipLaunchKernelGGL(bvh_level_kernel, dim3(nsmall), dim3(kBuildBlock), 0, s, small, ctx->bnodes, ctx->prim_idx, tmp_idx, ctx->prim_aabb,
-                         ctx->prim_centroid, cls, rk, hr, tl, counters, nxt, counters + 1, ctx->bparent, ctx->bdepth);
-    if (nbig > 0) {
-      hbig.resize(nbig);
-      NOVA_HIP_CHECK(ctx, hipMemcpy(hbig.data(), big, nbig * sizeof(BigNode), hipMemcpyDeviceToHost));
-      hchunks.clear();
-      for (int32_t b = 0; b < nbig; b++) {
-        hbig[b].chunk_first = (int32_t)hchunks.size();
-        for (int32_t c0 = hbig[b].s; c0 < hbig[b].s + hbig[b].n; c0 += kBigChunk)
-          hchunks.push_back(BigChunk{b, c0, std::min(c0 + kBigChunk, hbig[b].s + hbig[b].n)});
-        hbig[b].chunk_count = (int32_t)hchunks.size() - hbig[b].chunk_first;
-      }
-      const int32_t nch = (int32_t)hchunks.size();
-      if (nch > max_chunks) return set_error(ctx, NOVA_HIP_DEVICE_ERROR, "BVH build: chunk table overflow");
-      NOVA_HIP_CHECK(ctx, hipMemcpyAsync(big, hbig.data(), nbig * sizeof(BigNode), hipMemcpyHostToDevice, s));
-      NOVA_HIP_CHECK(ctx, hipMemcpyAsync(chunks, hchunks.data(), nch * sizeof(BigChunk), hipMemcpyHostToDevice, s));
-      const unsigned bb = (unsigned)((nbig + 63) / 64);
-      hipLaunchKernelGGL(big_init_kernel, dim3(nbig), dim3(64), 0, s, big, nbig);
-      hipLaunchKernelGGL(big_bin_kernel, dim3(nch), dim3(kBuildBlock), 0, s, big, chunks, ctx->bnodes, ctx->prim_idx, ctx->prim_aabb,
-                         ctx->prim_centroid);
-      hipLaunchKernelGGL(big_decide_kernel, dim3(bb), dim3(64), 0, s, big, nbig, ctx->bnodes);
-      hipLaunchKernelGGL(big_classify_kernel, dim3(nch), dim3(kBuildBlock), 0, s, big, chunks, ctx->prim_idx, ctx->prim_centroid, cls, chunk_nl);
-      hipLaunchKernelGGL(big_scan_kernel, dim3(bb), dim3(64), 0, s, big, nbig, chunk_nl, chunk_base);
-      hipLaunchKernelGGL(big_rank_kernel, dim3(nch), dim3(kBuildBlock), 0, s, big, chunks, cls, chunk_base, rk, hr, tl);
-      hipLaunchKernelGGL(big_scatter_kernel, dim3(nch), dim3(kBuildBlock), 0, s, big, chunks, cls, rk, hr, tl, ctx->prim_idx, tmp_idx);
-      hipLaunchKernelGGL(big_copyback_kernel, dim3(nch), dim3(kBuildBlock), 0, s, big, chunks, tmp_idx, ctx->prim_idx, ctx->prim_aabb);
-      hipLaunchKernelGGL(big_alloc_kernel, dim3(bb), dim3(64), 0, s, big, nbig, ctx->bnodes, counters, nxt, counters + 1, ctx->bparent,
-                         ctx->bdepth);
-    }
-    NOVA_HIP_CHECK(ctx, hipGetLastError());
-    NOVA_HIP_CHECK(ctx, hipMemcpyAsync(&active, counters + 1, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    NOVA_HIP_CHECK(ctx, hipStreamSynchronize(s));
-    std::swap(cur, nxt);
-    depth++;
-  }
-  for (void *p : {(void *)big, (void *)chunks, (void *)small, (void *)chunk_nl, (void *)chunk_base}) hipFree(p);
-  int32_t used = 0;
-  NOVA_HIP_CHECK(ctx, hipMemcpy(&used, counters, sizeof(int32_t), hipMemcpyDeviceToHost));
-  ctx->bnode_count = (uint32_t)used;
-
-  // ---- collapse to 4-wide
-  NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->nodes4, std::max<size_t>(1, used) * sizeof(Node4)));
-  int32_t *fb0 = act0, *fb1 = act1, *fs0 = rk, *fs1 = hr;  // reuse temporaries
-  int32_t h_counters[2] = {1, 0};                        // wide counter, next count
-  NOVA_HIP_CHECK(ctx, hipMemcpyAsync(counters + 2, h_counters, 2 * sizeof(int32_t), hipMemcpyHostToDevice, s));
-  NOVA_HIP_CHECK(ctx, hipMemcpyAsync(fb0, &zero, sizeof(int32_t), hipMemcpyHostToDevice, s));
-  NOVA_HIP_CHECK(ctx, hipMemcpyAsync(fs0, &zero, sizeof(int32_t), hipMemcpyHostToDevice, s));
-  int32_t frontier = 1;
-  uint32_t wdepth = 0;
-  while (frontier > 0) {
-    if (wdepth > depth + 1) return set_error(ctx, NOVA_HIP_DEVICE_ERROR, "BVH collapse did not converge");
-    NOVA_HIP_CHECK(ctx, hipMemsetAsync(counters + 3, 0, sizeof(int32_t), s));
-    hipLaunchKernelGGL(collapse_kernel, dim3((frontier + 127) / 128), dim3(128), 0, s, fb0, fs0, frontier, ctx->bnodes, ctx->nodes4, counters + 2,
-                       fb1, fs1, counters + 3);
-    NOVA_HIP_CHECK(ctx, hipGetLastError());
-    NOVA_HIP_CHECK(ctx, hipMemcpyAsync(&frontier, counters + 3, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    NOVA_HIP_CHECK(ctx, hipStreamSynchronize(s));
-    std::swap(fb0, fb1);
-    std::swap(fs0, fs1);
-    wdepth++;
-  }
-  int32_t wide = 0;
-  NOVA_HIP_CHECK(ctx, hipMemcpy(&wide, counters + 2, sizeof(int32_t), hipMemcpyDeviceToHost));
-  NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->nodes4f, std::max<size_t>(1, (size_t)wide) * sizeof(Node4F)));
-  hipLaunchKernelGGL(decode_nodes_kernel, dim3((wide + 255) / 256), dim3(256), 0, s, ctx->nodes4, ctx->nodes4f, (uint32_t)wide);
-  NOVA_HIP_CHECK(ctx, hipMalloc(&ctx->tri_leaf, (size_t)n * sizeof(TriMT)));
-  hipLaunchKernelGGL(gather_leaf_tris, dim3((n + 255) / 256), dim3(256), 0, s, ctx->prim_idx, ctx->tri_world, ctx->tri_leaf, n);
-  hipLaunchKernelGGL(leaf_of_position_kernel, dim3(std::min<uint32_t>(4096, (used + 255) / 256)), dim3(256), 0, s, ctx->bnodes, (uint32_t)used,
-                     ctx->leaf_of_pos, ctx->tri_leaf);
-  NOVA_HIP_CHECK(ctx, hipGetLastError());
-  NOVA_HIP_CHECK(ctx, hipEventRecord(ev1, s));
-  NOVA_HIP_CHECK(ctx, hipEventSynchronize(ev1));
+  const int st = run_build(ctx, P, n, s);
   float ms = 0.f;
-  hipEventElapsedTime(&ms, ev0, ev1);
+  if (st == NOVA_HIP_SUCCESS) {
+    NOVA_HIP_CHECK(ctx, hipEventRecord(ev1, s));
+    NOVA_HIP_CHECK(ctx, hipEventSynchronize(ev1));
+    hipEventElapsedTime(&ms, ev0, ev1);
+  }
   hipEventDestroy(ev0);
   hipEventDestroy(ev1);
-
-  // leaves = binary nodes with count > 0 among the used ones
-  std::vector<BNode> host(used);
-  NOVA_HIP_CHECK(ctx, hipMemcpy(host.data(), ctx->bnodes, used * sizeof(BNode), hipMemcpyDeviceToHost));
-  uint32_t leaves = 0;
-  for (const BNode &b : host) leaves += b.count > 0 ? 1 : 0;
-
-  for (void *p : {(void *)tmp_idx, (void *)rk, (void *)hr, (void *)tl, (void *)act0, (void *)act1, (void *)counters, (void *)cls, (void *)bounds})
-    hipFree(p);
-
-  ctx->bvh_info.primitive_count = n;
-  ctx->bvh_info.binary_nodes = (uint32_t)used;
-  ctx->bvh_info.binary_depth = depth;
-  ctx->bvh_info.wide_nodes = (uint32_t)wide;
-  ctx->bvh_info.wide_depth = wdepth;
-  ctx->bvh_info.leaves = leaves;
+  hipFree(temps);  // waits for the device
+  if (st) return st;
   ctx->bvh_info.build_ms = ms;
   if (info) *info = ctx->bvh_info;
   ctx->tail_hint = 0;
