@@ -203,6 +203,29 @@ __host__ __device__ inline
   return new_later ? reached : !reached;
 }
 
+#ifndef NOVA_LDS_STACK
+#define NOVA_LDS_STACK 16
+#endif
+constexpr int kTraceBlock = 256;
+constexpr int kLdsStack = NOVA_LDS_STACK;  // traversal stack levels held in LDS per lane
+
+// Traversal stack of one lane of a kTraceBlock-thread block: the first kLdsStack levels in
+// LDS (lane-interleaved), the rest in a global overflow area strided by the grid size.
+struct LdsStack {
+  uint32_t *lds;
+  uint32_t *gstack;
+  uint32_t gstride, gtid, lane;
+  __device__ __forceinline__ void push(int sp, uint32_t v) {
+    if (sp < kLdsStack)
+      lds[sp * kTraceBlock + lane] = v;
+    else
+      gstack[(size_t)(sp - kLdsStack) * gstride + gtid] = v;
+  }
+  __device__ __forceinline__ uint32_t at(int sp) const {
+    return sp < kLdsStack ? lds[sp * kTraceBlock + lane] : gstack[(size_t)(sp - kLdsStack) * gstride + gtid];
+  }
+};
+
 // Per-ray traversal state, so that a lane can be handed a new ray as soon as its ray ends.
 struct TraceState {
   f3 o, d, inv;
@@ -239,6 +262,38 @@ NOVA_HD void trace_init(TraceState &st, f3 o, f3 d) {
 struct TieFromCtx {
   NOVA_HD const TieTables *operator()(const TraceCtx &tc) const { return tc.tie; }
 };
+
+// The inner children among cref[0..3] (near to far; negative: not an inner node) onto the
+// stack far to near, all but the nearest, which is returned (negative: none).
+template <class Stack>
+NOVA_HD int32_t push_inner(Stack &stack, int &sp, const int32_t *cref) {
+  int32_t next = -1;
+#pragma unroll
+  for (int a = 3; a >= 0; a--) {
+    if (cref[a] < 0) continue;
+    if (next >= 0) stack.push(sp++, (uint32_t)next);
+    next = cref[a];
+  }
+  return next;
+}
+#ifdef __HIP_DEVICE_COMPILE__
+// On the LDS stack, while no lane of the wave is within three levels of its end: every
+// candidate is written and the level counts only those kept, so nothing branches (twelve
+// nested branches per node before; with the branch-free entry tests, per-ray walks of the 1080p
+// job 23.55 -> 23.2 ms, 262,147 rays of one closest-hit call 157 -> 147 us).
+__device__ __forceinline__ int32_t push_inner(LdsStack &stack, int &sp, const int32_t *cref) {
+  if (__ballot(sp > kLdsStack - 3) != 0) return push_inner<LdsStack>(stack, sp, cref);
+  const bool i0 = cref[0] >= 0, i1 = cref[1] >= 0, i2 = cref[2] >= 0, i3 = cref[3] >= 0;
+  uint32_t *at = stack.lds + stack.lane;
+  at[sp * kTraceBlock] = (uint32_t)cref[3];
+  sp += (i3 & (i0 | i1 | i2)) ? 1 : 0;
+  at[sp * kTraceBlock] = (uint32_t)cref[2];
+  sp += (i2 & (i0 | i1)) ? 1 : 0;
+  at[sp * kTraceBlock] = (uint32_t)cref[1];
+  sp += (i1 & i0) ? 1 : 0;
+  return i0 ? cref[0] : i1 ? cref[1] : i2 ? cref[2] : cref[3];
+}
+#endif
 
 // One node of the walk: test the node's four children with a slightly widened slab (no box
 // holding a hit the reference's division-form test accepts is culled), order them near to
@@ -315,7 +370,8 @@ NOVA_HD bool trace_step(const TraceCtx &tc, Stack &stack, TraceState &st, float 
         const float tfz = (grid_plane((fqz >> (8 * k)) & 255u, sz, orgz) - st.o.z) * st.inv.z;
         const float t0 = fmaxf(fmaxf(tnx, tny), tnz);
         const float t1 = fminf(fminf(tfx, tfy), tfz) * kUp;
-        const bool hit = chv[k] != -1 && t0 <= t1 && t1 >= 0.f && t0 <= st.tbest * kUp;
+        // no short circuit: a branch per child would keep the four children's arithmetic apart
+        const bool hit = (chv[k] != -1) & (t0 <= t1) & (t1 >= 0.f) & (t0 <= st.tbest * kUp);
         key[k] = hit ? t0 : kInf;
         cref[k] = hit ? chv[k] : -1;
       }
@@ -336,13 +392,7 @@ NOVA_HD bool trace_step(const TraceCtx &tc, Stack &stack, TraceState &st, float 
     exch(0, 2);
     exch(1, 3);
     exch(1, 2);
-    int32_t next = -1;
-#pragma unroll
-    for (int a = 3; a >= 0; a--) {  // far to near: push inner nodes, keep the nearest
-      if (cref[a] < 0) continue;
-      if (next >= 0) stack.push(st.sp++, (uint32_t)next);
-      next = cref[a];
-    }
+    const int32_t next = push_inner(stack, st.sp, cref);  // far to near; the nearest is visited next
 #pragma unroll
     for (int a = 0; a < 4; a++) {  // leaves now, near to far
       if (cref[a] > -2) continue;
@@ -408,7 +458,13 @@ NOVA_HD int trace_closest(const TraceCtx &tc, Stack &stack, f3 o, f3 d, float tn
 // rounding of a small determinant), a walk that first finds the neighbouring triangle culls
 // that box and one that reaches the box first keeps the closer hit. The reference's own
 // walk is order-dependent there too; the per-ray walk follows each ray's near-to-far order. The stack is the wave's: (node, lane mask) entries, entry e held
-// in lane e of three registers, so a push is a compare-and-select and a pop a lane read.
+// in lane e of three registers, so a push is a lane write and a pop a lane read.
+//
+// What bounds it is issue: the vector and the scalar unit were each 86% busy (225 and 210
+// instructions per node). Most nodes have at most one inner child to go on with, which
+// needs neither keys nor ranks; the entry tests fold the best hit into the exit's minimum; child
+// references come with the planes instead of one scalar load per use. Camera walk of the 1080p
+// job of 64 frames: 11.35 -> 7.2 ms.
 #ifdef __HIP_DEVICE_COMPILE__
 typedef const __attribute__((address_space(4))) Node4F ConstNode4F;  // scalar-loadable: uniform address, never written by the walk
 typedef const __attribute__((address_space(4))) float4 ConstFloat4;
@@ -418,6 +474,20 @@ typedef const Node4F ConstNode4F;
 typedef const float4 ConstFloat4;
 typedef const TriMT ConstTriMT;
 #endif
+
+#ifdef __HIP_DEVICE_COMPILE__
+// v_writelane_b32: lane `at` of `old` replaced by a wave-uniform value (clang has no builtin for the intrinsic)
+extern "C" __device__ int32_t nova_writelane(int32_t value, int32_t at, int32_t old) __asm("llvm.amdgcn.writelane.i32");
+#else
+__device__ inline int32_t nova_writelane(int32_t, int32_t, int32_t old) { return old; }
+#endif
+
+// A wave-uniform value that is to be computed (loaded) here and not where it is used.
+__device__ __forceinline__ void keep_scalar(int32_t &v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+s"(v));
+#endif
+}
 
 constexpr int kWaveStack = 64;  // (node, mask) entries per wave, one per lane; usable when 3 * wide depth + 4 < kWaveStack
 
@@ -445,79 +515,83 @@ __device__ void coherent_walk(const TraceCtx &tc, TraceState &st, uint64_t lanes
     node = __builtin_amdgcn_readfirstlane(node);
     ConstNode4F &nd = nodes[node];
     const bool in = (mask >> lane) & 1u;
-    float key[4] = {kInf, kInf, kInf, kInf};
-    bool hit[4] = {false, false, false, false};
-    if (in) {
-      if (kCount) nodes_visited++;
-      if (uniform) {
-        ConstFloat4 *rows = (ConstFloat4 *)&nodes[node];
-        const float4 qnx = rows[rnx], qfx = rows[rfx], qny = rows[rny], qfy = rows[rfy], qnz = rows[rnz], qfz = rows[rfz];
-        const float nxs[4] = {qnx.x, qnx.y, qnx.z, qnx.w}, fxs[4] = {qfx.x, qfx.y, qfx.z, qfx.w};
-        const float nys[4] = {qny.x, qny.y, qny.z, qny.w}, fys[4] = {qfy.x, qfy.y, qfy.z, qfy.w};
-        const float nzs[4] = {qnz.x, qnz.y, qnz.z, qnz.w}, fzs[4] = {qfz.x, qfz.y, qfz.z, qfz.w};
+    if (kCount && in) nodes_visited++;
+    // Every lane tests its ray (the wave issues the instructions either way); the lanes outside
+    // the mask drop out of the ballots below.
+    float t0s[4];
+    bool hit[4];
+    // the child references with the planes, in one wait: left to itself the compiler loads each
+    // where it is first used, one scalar-memory latency after the other
+    int32_t child[4] = {nd.child[0], nd.child[1], nd.child[2], nd.child[3]};
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          const float tnx = (nxs[k] - st.o.x) * st.inv.x, tfx = (fxs[k] - st.o.x) * st.inv.x;
-          const float tny = (nys[k] - st.o.y) * st.inv.y, tfy = (fys[k] - st.o.y) * st.inv.y;
-          const float tnz = (nzs[k] - st.o.z) * st.inv.z, tfz = (fzs[k] - st.o.z) * st.inv.z;
-          const float t0 = fmaxf(fmaxf(tnx, tny), tnz);
-          const float t1 = fminf(fminf(tfx, tfy), tfz) * kUp;
-          hit[k] = nd.child[k] != -1 && t0 <= t1 && t1 >= 0.f && t0 <= st.tbest * kUp;
-          key[k] = hit[k] ? t0 : kInf;
-        }
-      } else {  // mixed signs or axis-parallel rays: both planes of each axis, then min/max (the same values)
+    for (int k = 0; k < 4; k++) keep_scalar(child[k]);
+    if (uniform) {
+      ConstFloat4 *rows = (ConstFloat4 *)&nodes[node];
+      const float4 qnx = rows[rnx], qfx = rows[rfx], qny = rows[rny], qfy = rows[rfy], qnz = rows[rnz], qfz = rows[rfz];
+      const float nxs[4] = {qnx.x, qnx.y, qnx.z, qnx.w}, fxs[4] = {qfx.x, qfx.y, qfx.z, qfx.w};
+      const float nys[4] = {qny.x, qny.y, qny.z, qny.w}, fys[4] = {qfy.x, qfy.y, qfy.z, qfy.w};
+      const float nzs[4] = {qnz.x, qnz.y, qnz.z, qnz.w}, fzs[4] = {qfz.x, qfz.y, qfz.z, qfz.w};
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          const float bmnx = nd.plane[0][0][k], bmxx = nd.plane[0][1][k];
-          const float bmny = nd.plane[1][0][k], bmxy = nd.plane[1][1][k];
-          const float bmnz = nd.plane[2][0][k], bmxz = nd.plane[2][1][k];
-          float tx1 = (bmnx - st.o.x) * st.inv.x, tx2 = (bmxx - st.o.x) * st.inv.x;
-          float ty1 = (bmny - st.o.y) * st.inv.y, ty2 = (bmxy - st.o.y) * st.inv.y;
-          float tz1 = (bmnz - st.o.z) * st.inv.z, tz2 = (bmxz - st.o.z) * st.inv.z;
-          if (st.px) {
-            const bool inside = bmnx <= st.o.x && st.o.x <= bmxx;
-            tx1 = -kInf;
-            tx2 = inside ? kInf : -kInf;
-          }
-          if (st.py) {
-            const bool inside = bmny <= st.o.y && st.o.y <= bmxy;
-            ty1 = -kInf;
-            ty2 = inside ? kInf : -kInf;
-          }
-          if (st.pz) {
-            const bool inside = bmnz <= st.o.z && st.o.z <= bmxz;
-            tz1 = -kInf;
-            tz2 = inside ? kInf : -kInf;
-          }
-          const float t0 = fmaxf(fmaxf(fminf(tx1, tx2), fminf(ty1, ty2)), fminf(tz1, tz2));
-          const float t1 = fminf(fminf(fmaxf(tx1, tx2), fmaxf(ty1, ty2)), fmaxf(tz1, tz2)) * kUp;
-          hit[k] = nd.child[k] != -1 && t0 <= t1 && t1 >= 0.f && t0 <= st.tbest * kUp;
-          key[k] = hit[k] ? t0 : kInf;
+      for (int k = 0; k < 4; k++) {
+        const float tnx = (nxs[k] - st.o.x) * st.inv.x, tfx = (fxs[k] - st.o.x) * st.inv.x;
+        const float tny = (nys[k] - st.o.y) * st.inv.y, tfy = (fys[k] - st.o.y) * st.inv.y;
+        const float tnz = (nzs[k] - st.o.z) * st.inv.z, tfz = (fzs[k] - st.o.z) * st.inv.z;
+        const float t0 = fmaxf(fmaxf(tnx, tny), tnz);
+        // the exit and the best hit, each widened by kUp, in one minimum (the product keeps order)
+        const float t1 = fminf(fminf(fminf(tfx, tfy), tfz), st.tbest) * kUp;
+        hit[k] = (t0 <= t1) & (t1 >= 0.f);
+        t0s[k] = t0;
+      }
+    } else {  // mixed signs or axis-parallel rays: both planes of each axis, then min/max (the same values)
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const float bmnx = nd.plane[0][0][k], bmxx = nd.plane[0][1][k];
+        const float bmny = nd.plane[1][0][k], bmxy = nd.plane[1][1][k];
+        const float bmnz = nd.plane[2][0][k], bmxz = nd.plane[2][1][k];
+        float tx1 = (bmnx - st.o.x) * st.inv.x, tx2 = (bmxx - st.o.x) * st.inv.x;
+        float ty1 = (bmny - st.o.y) * st.inv.y, ty2 = (bmxy - st.o.y) * st.inv.y;
+        float tz1 = (bmnz - st.o.z) * st.inv.z, tz2 = (bmxz - st.o.z) * st.inv.z;
+        if (st.px) {
+          const bool inside = bmnx <= st.o.x && st.o.x <= bmxx;
+          tx1 = -kInf;
+          tx2 = inside ? kInf : -kInf;
         }
+        if (st.py) {
+          const bool inside = bmny <= st.o.y && st.o.y <= bmxy;
+          ty1 = -kInf;
+          ty2 = inside ? kInf : -kInf;
+        }
+        if (st.pz) {
+          const bool inside = bmnz <= st.o.z && st.o.z <= bmxz;
+          tz1 = -kInf;
+          tz2 = inside ? kInf : -kInf;
+        }
+        const float t0 = fmaxf(fmaxf(fminf(tx1, tx2), fminf(ty1, ty2)), fminf(tz1, tz2));
+        const float t1 = fminf(fminf(fminf(fmaxf(tx1, tx2), fmaxf(ty1, ty2)), fmaxf(tz1, tz2)), st.tbest) * kUp;
+        hit[k] = (t0 <= t1) & (t1 >= 0.f);
+        t0s[k] = t0;
       }
     }
-    // The wave's view of each child: the lanes that enter it, and an ordering key -- the
-    // first lane's entry distance as an orderable integer with the child's index in its low
-    // two bits (so the four keys differ; order among near-equal keys does not matter).
-    const int leader = __builtin_ffsll((long long)mask) - 1;
+    // The wave's view of each child: the lanes that enter it. An empty slot (child -1) may be
+    // "entered" too; it is neither a leaf nor an inner node below.
     uint64_t m[4];
-    int32_t pk[4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      m[k] = __ballot(hit[k]);
-      const int32_t b = __builtin_amdgcn_readlane(__builtin_bit_cast(int32_t, key[k]), leader);
-      pk[k] = ((m[k] ? (b ^ ((b >> 31) & 0x7fffffff)) : 0x7fffffff) & ~3) | k;
-    }
+    for (int k = 0; k < 4; k++) m[k] = __ballot(hit[k]) & mask;
+    const int leader = __builtin_ffsll((long long)mask) - 1;
     // leaves, in child order, by the lanes that enter each leaf's box
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-      const int32_t c = nd.child[k];
+      const int32_t c = child[k];
       if (c > -2 || !m[k]) continue;
-      const bool mine = ((m[k] >> lane) & 1u) && key[k] <= st.tbest * kUp;
+      const bool mine = ((m[k] >> lane) & 1u) && t0s[k] <= st.tbest * kUp;
       const int32_t start = leaf_first(c);
-      const int32_t cnt = __builtin_bit_cast(int32_t, tris[start].b.w);
+      int32_t cnt = 1;  // the leaf size comes with its first record
       for (int32_t i = start; i < start + cnt; i++) {
         const TriMT tr = tris[i];
+        if (i == start) {
+          cnt = __builtin_bit_cast(int32_t, tr.b.w);
+          keep_scalar(cnt);
+        }
         if (!mine) continue;
         if (kCount) tri_tests++;
         float tt, uu, vv;
@@ -532,65 +606,57 @@ __device__ void coherent_walk(const TraceCtx &tc, TraceState &st, uint64_t lanes
       }
     }
     // Inner children entered by some lane: the nearest is visited next, the others go onto
-    // the stack far to near -- child k to slot sp + (entered inner children farther than k).
-    bool inner[4];
-    int ninner = 0;
+    // the stack far to near. One such child, the most frequent case, needs no order.
+    uint32_t inner = 0;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      inner[k] = nd.child[k] >= 0 && m[k] != 0;
-      ninner += inner[k] ? 1 : 0;
-    }
-    int32_t next = -1;
-    uint64_t next_mask = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      int farther = 0;
-#pragma unroll
-      for (int j = 0; j < 4; j++) farther += (j != k && inner[j] && pk[j] > pk[k]) ? 1 : 0;
-      const bool nearest = inner[k] && farther == ninner - 1;
-      next = nearest ? nd.child[k] : next;
-      next_mask = nearest ? m[k] : next_mask;
-      // pushed entries land at sp .. sp + ninner - 2; the others write the spare last slot
-      const int slot = (inner[k] && !nearest) ? sp + farther : kWaveStack - 1;
-      const bool here = (int)lane == slot;  // a lane write: compare and select
-      stk_node = here ? nd.child[k] : stk_node;
-      stk_lo = here ? (int32_t)(uint32_t)m[k] : stk_lo;
-      stk_hi = here ? (int32_t)(uint32_t)(m[k] >> 32) : stk_hi;
-    }
-    if (next >= 0) {
-      sp += ninner - 1;
-      node = next;
-      mask = next_mask;
+    for (int k = 0; k < 4; k++) inner |= (child[k] >= 0 && m[k] != 0) ? 1u << k : 0u;
+    if (inner == 0) {
+      if (sp == 0) break;
+      sp--;
+      node = __builtin_amdgcn_readlane(stk_node, sp);
+      mask = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(stk_hi, sp) << 32) | (uint32_t)__builtin_amdgcn_readlane(stk_lo, sp);
       continue;
     }
-    if (sp == 0) break;
-    sp--;
-    node = __builtin_amdgcn_readlane(stk_node, sp);
-    mask = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(stk_hi, sp) << 32) | (uint32_t)__builtin_amdgcn_readlane(stk_lo, sp);
+    if ((inner & (inner - 1)) == 0) {
+      node = (inner & 1) ? child[0] : (inner & 2) ? child[1] : (inner & 4) ? child[2] : child[3];
+      mask = (inner & 1) ? m[0] : (inner & 2) ? m[1] : (inner & 4) ? m[2] : m[3];
+      continue;
+    }
+    // The order: the first lane's entry distances (+inf where it misses) as orderable integers
+    // with the child's index in the low two bits (so they differ; order among near-equal keys
+    // does not matter); child k's rank is the number of entered inner children farther than it.
+    int32_t pk[4];
+    int farther[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int32_t t = __builtin_amdgcn_readlane(__builtin_bit_cast(int32_t, t0s[k]), leader);
+      const int32_t b = (m[k] >> leader) & 1u ? t : 0x7f800000;
+      pk[k] = (inner >> k) & 1u ? ((b ^ ((b >> 31) & 0x7fffffff)) & ~3) | k : (int32_t)0x80000000;  // not entered: before every key
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int k = j + 1; k < 4; k++) {
+        const bool gt = pk[j] > pk[k];
+        farther[k] += gt ? 1 : 0;
+        farther[j] += gt ? 0 : 1;
+      }
+    // entered child k goes to slot sp + farther[k]; the nearest (the highest) is taken off again
+    const int ninner = __builtin_popcount(inner);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (!((inner >> k) & 1u)) continue;
+      if (farther[k] == ninner - 1) {
+        node = child[k];
+        mask = m[k];
+      } else {  // an entry is written into its lane of the stack registers
+        stk_node = nova_writelane(child[k], sp + farther[k], stk_node);
+        stk_lo = nova_writelane((int32_t)(uint32_t)m[k], sp + farther[k], stk_lo);
+        stk_hi = nova_writelane((int32_t)(uint32_t)(m[k] >> 32), sp + farther[k], stk_hi);
+      }
+    }
+    sp += ninner - 1;
   }
 }
-
-#ifndef NOVA_LDS_STACK
-#define NOVA_LDS_STACK 16
-#endif
-constexpr int kTraceBlock = 256;
-constexpr int kLdsStack = NOVA_LDS_STACK;  // traversal stack levels held in LDS per lane
-
-// Traversal stack of one lane of a kTraceBlock-thread block: the first kLdsStack levels in
-// LDS (lane-interleaved), the rest in a global overflow area strided by the grid size.
-struct LdsStack {
-  uint32_t *lds;
-  uint32_t *gstack;
-  uint32_t gstride, gtid, lane;
-  __device__ __forceinline__ void push(int sp, uint32_t v) {
-    if (sp < kLdsStack)
-      lds[sp * kTraceBlock + lane] = v;
-    else
-      gstack[(size_t)(sp - kLdsStack) * gstride + gtid] = v;
-  }
-  __device__ __forceinline__ uint32_t at(int sp) const {
-    return sp < kLdsStack ? lds[sp * kTraceBlock + lane] : gstack[(size_t)(sp - kLdsStack) * gstride + gtid];
-  }
-};
 
 }  // namespace nova_hip
