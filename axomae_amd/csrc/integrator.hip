@@ -32,22 +32,62 @@ namespace nova_hip {
 
 // ------------------------------------------------------------------ kernels
 
-constexpr int kWorkCounter = 4;  // count[] slot of the extend work counter, zeroed before each extend
-constexpr int kTailSlot = 5;     // count[] slot: 0, or 1 + the bounce from which the batch's paths finish in tail_kernel
+constexpr int kTailSlot = 5;  // count[] slot: 0, or 1 + the bounce from which the batch's paths finish in tail_kernel
 
+// A ray queue is cut into 2^shard_bits shards. Workgroup b works on shard b mod 2^shard_bits: its
+// first rays and its claims come from that shard, its survivors go to the same shard of the
+// next queue, and each shard's counters have a cache line of their own. Atomics on one address
+// run at 11.4 ns each on this chip, whatever the number of waves: with one counter the claims
+// (one per 56 rays) bound the camera walk of a one-sample 1080p frame (0.50 -> 0.34 ms; the
+// frame 2.11 -> 1.90 ms, six frames at 1021x577 of a scene with many misses 2.33 -> 1.84), and
+// long walks could not refill more often (64 samples at 1080p: 47.5 -> 45.8 ms). One shard per
+// XCD: 16 take 46.1 ms there, 32 take 46.4.
+//
+// The first queue is linear (entry = path id): shard k holds every 2^shard_bits-th chunk of
+// kQueueChunk entries, so all shards move through the image together. Later queues give shard k
+// the entries [k * seg, (k + 1) * seg), seg being what the shard holds at the start.
+constexpr uint32_t kQueueChunk = 256;
+constexpr uint32_t kMaxShardBits = 3;
+constexpr uint32_t kCounterStride = 32;  // words between two shards' counters
 struct Queues {
   float *ray[2];      // 6 planes of cap floats each: ox oy oz dx dy dz
   int32_t *slot[2];
-  uint32_t *count;    // [0], [1]: queue sizes; [2]: segments traced
+  uint32_t *count;    // [0]: entries of the first queue; [2]: segments traced; [kTailSlot]
+  uint32_t *shard_n[2];  // entries per shard, kCounterStride words apart
+  uint32_t *work;        // rays claimed per shard beyond the lanes' first ones, zeroed before each extend
   unsigned long long *stats64;  // [0] node visits, [1] triangle tests, [2] escaped segments (camera-ray launches count into [4], [5]);
                                 // per-ray walk: [8] wave loop turns, [9] active lanes summed over turns, [10] wave rounds of the triangle loop;
                                 // tail_kernel: [16] segments, [17] node visits, [18] triangle tests
   float4 *hit;        // closest hit per queue entry: (prim id bits, t, u, v), one 16-byte record
-  float *T, *L, *A;   // path state by slot: T,L 3 planes of cap each; A alpha
+  float *T, *L, *A;   // path state by path id: T,L 3 planes of `paths` each; A alpha
   float *partial;     // frames x W x H x 4
-  uint32_t cap;
+  uint32_t cap;       // entries of a queue (plane stride)
+  uint32_t paths;     // paths of a batch (plane stride of the path state)
+  uint32_t shard_bits, seg;
 };
 
+// Entries of share k of S of a linear queue of n entries, its runs of kRun dealt out in turn.
+template <uint32_t kRun>
+NOVA_HD uint32_t linear_share_count(uint32_t n, uint32_t S, uint32_t k) {
+  const uint32_t runs = n / kRun, rest = n % kRun, last = runs % S;
+  return (runs / S + (k < last ? 1u : 0u)) * kRun + (k == last ? rest : 0u);
+}
+// Entry i of shard k of a linear queue.
+NOVA_HD uint32_t linear_shard_pos(uint32_t bits, uint32_t k, uint32_t i) { return (((i / kQueueChunk) << bits) + k) * kQueueChunk + i % kQueueChunk; }
+
+// The workgroup's shard and its place among the workgroups of that shard.
+__device__ __forceinline__ uint32_t block_shard(uint32_t bits) { return blockIdx.x & ((1u << bits) - 1); }
+__device__ __forceinline__ uint32_t shard_blocks(uint32_t bits, uint32_t k) { return (gridDim.x + (1u << bits) - 1 - k) >> bits; }
+
+// Entries of a whole queue, the same value in every lane.
+__device__ __forceinline__ uint32_t queue_total(const uint32_t *shard_n, uint32_t bits) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t mine = lane < (1u << bits) ? shard_n[lane * kCounterStride] : 0u;
+  uint32_t n = 0;
+#pragma unroll
+  for (int k = 0; k < (1 << kMaxShardBits); k++) n += (uint32_t)__builtin_amdgcn_readlane((int)mine, k);
+  return n;
+}
 
 // AbstractIntegrator::render per pixel (Integrator.h:53-95): one camera ray per path slot.
 // The first shade takes the path id from the queue position and starts every path at T = 1,
@@ -72,16 +112,22 @@ __global__ __launch_bounds__(256) void generate_kernel(FrameParams fp, const uin
     r[4 * (size_t)n + i] = d.y;
     r[5 * (size_t)n + i] = d.z;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    q.count[0] = active;
-    q.count[1] = 0;
-    q.count[kWorkCounter] = 0;
-    q.count[kTailSlot] = 0;
+  if (blockIdx.x == 0 && threadIdx.x < (1u << q.shard_bits)) {
+    const uint32_t k = threadIdx.x;
+    q.shard_n[0][k * kCounterStride] = linear_share_count<kQueueChunk>(active, 1u << q.shard_bits, k);
+    q.shard_n[1][k * kCounterStride] = 0;
+    q.work[k * kCounterStride] = 0;
+    if (k == 0) {
+      q.count[0] = active;
+      q.count[kTailSlot] = 0;
+    }
   }
 }
 
 #ifndef NOVA_TRACE_REFILL
-#define NOVA_TRACE_REFILL 56  // idle lanes that trigger a refill in the extend kernel (0: grid-stride, one ray per lane at a time)
+// idle lanes that trigger a refill of the per-ray walk (64 samples at 1080p: 48.3 ms at 60, 47.5
+// at 56, 46.2 at 40, 45.8 at 24, 47.2 at 8)
+#define NOVA_TRACE_REFILL 24
 #endif
 #ifndef NOVA_TRACE_WAVES
 #define NOVA_TRACE_WAVES 6  // waves per SIMD the extend kernel is compiled for (0: compiler's choice)
@@ -100,12 +146,92 @@ static_assert(kTraceBlock == 256, "the workgroups-per-CU count assumes one wave 
 #define NOVA_TRACE_OCCUPANCY
 #endif
 
+// The per-ray walk of a queue by a whole grid: one traversal step per loop turn; a lane whose
+// ray has ended takes the next unclaimed ray as soon as NOVA_TRACE_REFILL lanes of its wave are
+// idle (one atomic per refill for the wave), so lanes do not wait for the wave's longest ray.
+// The queue comes in shares with a claim counter each; a wave claims from its own share only
+// (the shares are statistically alike, and taking over another's rays cost the loop 18
+// registers). A share's first rays go one per lane by thread index, without an atomic: a launch
+// over a nearly empty queue (the last bounces) then makes no claims at all. fetch(p, o, d) gives
+// the ray at place p of the queue, store(p, st) takes its finished state.
+template <uint32_t kRun>
+struct WalkShare {
+  uint32_t n;            // its entries
+  uint32_t first, step;  // the place of its entry 0, and from a run of kRun entries to its next
+  uint32_t begin;        // the entry of this workgroup's first lane
+  uint32_t handed;       // entries handed out by thread index
+  __device__ __forceinline__ uint32_t pos(uint32_t i) const { return first + (i / kRun) * step + i % kRun; }
+};
+// The share of a bounce's queue that this workgroup works on, its shard: the first queue is linear.
+__device__ __forceinline__ WalkShare<kQueueChunk> queue_share(const Queues &q, int which, bool linear) {
+  const uint32_t k = block_shard(q.shard_bits), n = q.shard_n[which][k * kCounterStride];
+  return {n, linear ? k * kQueueChunk : k * q.seg, linear ? kQueueChunk << q.shard_bits : kQueueChunk,
+          (blockIdx.x >> q.shard_bits) * (uint32_t)kTraceBlock, shard_blocks(q.shard_bits, k) * (uint32_t)kTraceBlock};
+}
+// Every workgroup a share of its own of a linear queue: runs of a wave's entries dealt out in
+// turn, short ones so that a share mixes many parts of the queue (normals of the 1080p scene of
+// 1,048,576 triangles: 0.52 ms with runs of 256, 0.47 with 64, 0.53 with 32).
+constexpr uint32_t kShareRun = 64;
+__device__ __forceinline__ WalkShare<kShareRun> workgroup_share(uint32_t n) {
+  return {linear_share_count<kShareRun>(n, gridDim.x, blockIdx.x), blockIdx.x * kShareRun, kShareRun * gridDim.x, 0, kTraceBlock};
+}
+struct WalkCounts {
+  uint32_t nodes = 0, tests = 0, wave_turns = 0, lane_turns = 0, tri_rounds = 0;  // instrumented launches only
+};
+
+template <bool kCount, class Share, class Fetch, class Store>
+__device__ __forceinline__ void refill_walk(const TraceCtx &tc, LdsStack &stk, const Share &share, uint32_t *claims, Fetch fetch, Store store,
+                                            WalkCounts &c) {
+  const uint32_t lane = threadIdx.x & 63, n = share.n, handed = share.handed;
+  TraceState ts;
+  bool have = false, exhausted = handed >= n;
+  uint32_t ray = 0;
+  for (uint32_t turns = 0; turns < (1u << 30); turns++) {
+    const uint64_t idle = __ballot(!have);
+    uint32_t base = share.begin + threadIdx.x - lane;  // first turn: every lane idle, a ray per lane
+    bool fill = turns == 0;
+    if (!fill && !exhausted && __popcll(idle) >= NOVA_TRACE_REFILL) {
+      const int leader = __builtin_ffsll((long long)idle) - 1;
+      if ((int)lane == leader) base = handed + atomicAdd(claims, (uint32_t)__popcll(idle));
+      base = __shfl(base, leader, 64);
+      if (base >= n) exhausted = true;
+      fill = true;
+    }
+    if (fill && !have) {
+      const uint32_t i = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0));
+      if (i < n) {
+        const uint32_t p = share.pos(i);
+        f3 o, d;
+        fetch(p, o, d);
+        trace_init(ts, o, d);
+        ray = p;
+        have = true;
+      }
+    }
+    const uint64_t busy = __ballot(have);
+    if (busy == 0) break;
+    if (kCount && (threadIdx.x & 63) == 0) {
+      c.wave_turns++;
+      c.lane_turns += (uint32_t)__popcll(busy);
+    }
+    if (have && trace_step<kCount>(tc, stk, ts, 0.000001f, c.nodes, c.tests)) {
+      store(ray, ts);
+      have = false;
+      if (kCount) c.tri_rounds += ts.tri_rounds;
+    }
+  }
+}
+
+// A finished ray's record: (prim id bits, t, u, v).
+__device__ __forceinline__ float4 hit_record(const TraceState &st) {
+  return make_float4(__builtin_bit_cast(float, (int32_t)(st.best)), st.tbest, st.bu, st.bv);
+}
+
 template <bool kCount>
 __global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void extend_kernel(TraceCtx tc, Queues q, int which, int bounce, uint32_t tail_rays,
                                                                                   int tail_force) {
   __shared__ uint32_t lds[kLdsStack * kTraceBlock];
-  uint32_t nv = 0, nt = 0;
-  const uint32_t n = q.count[which];
+  const uint32_t n = queue_total(q.shard_n[which], q.shard_bits);
   const float *r = q.ray[which];
   const size_t cap = q.cap;
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -118,67 +244,19 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void extend_kerne
   }
   if (gtid == 0) q.count[2] += n;
   LdsStack stk{lds, tc.gstack, tc.gstride, gtid, threadIdx.x};
-#if NOVA_TRACE_REFILL > 0
-  // One traversal step per loop turn; a lane whose ray has ended takes the next unclaimed
-  // ray as soon as NOVA_TRACE_REFILL lanes of its wave are idle (one atomic per refill for
-  // the wave), so lanes do not wait for the wave's longest ray.
-  // The first rays go one per lane by thread index, without an atomic: a launch over a
-  // nearly empty queue (the last bounces) then makes no claims at all, where one claim per
-  // wave on the shared counter cost about 90 us per launch. Refills claim rays past those.
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t nthreads = gridDim.x * blockDim.x;
-  TraceState ts;
-  bool have = false, exhausted = nthreads >= n;
-  uint32_t ray = 0;
-  uint32_t wave_turns = 0, lane_turns = 0, tri_rounds = 0;  // instrumented launches only
-  for (uint32_t turns = 0; turns < (1u << 30); turns++) {
-    const uint64_t idle = __ballot(!have);
-    uint32_t base = gtid - lane;  // first turn: every lane idle, lane l takes ray gtid
-    bool fill = turns == 0;
-    if (!fill && !exhausted && __popcll(idle) >= NOVA_TRACE_REFILL) {
-      const int leader = __builtin_ffsll((long long)idle) - 1;
-      if ((int)lane == leader) base = nthreads + atomicAdd(&q.count[kWorkCounter], (uint32_t)__popcll(idle));
-      base = __shfl(base, leader, 64);
-      if (base >= n) exhausted = true;
-      fill = true;
-    }
-    if (fill && !have) {
-      const uint32_t i = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0));
-      if (i < n) {
-        trace_init(ts, mk3(r[i], r[cap + i], r[2 * cap + i]), mk3(r[3 * cap + i], r[4 * cap + i], r[5 * cap + i]));
-        ray = i;
-        have = true;
-      }
-    }
-    const uint64_t busy = __ballot(have);
-    if (busy == 0) break;
-    if (kCount && lane == 0) {
-      wave_turns++;
-      lane_turns += (uint32_t)__popcll(busy);
-    }
-    if (have && trace_step<kCount>(tc, stk, ts, 0.000001f, nv, nt)) {
-      q.hit[ray] = make_float4(__builtin_bit_cast(float, (int32_t)(ts.best)), ts.tbest, ts.bu, ts.bv);
-      have = false;
-      if (kCount) tri_rounds += ts.tri_rounds;
-    }
-  }
+  WalkCounts c;
+  auto fetch = [&](uint32_t p, f3 &o, f3 &d) {
+    o = mk3(r[p], r[cap + p], r[2 * cap + p]);
+    d = mk3(r[3 * cap + p], r[4 * cap + p], r[5 * cap + p]);
+  };
+  auto store = [&](uint32_t p, const TraceState &st) { q.hit[p] = hit_record(st); };
+  refill_walk<kCount>(tc, stk, queue_share(q, which, bounce == 0), q.work + block_shard(q.shard_bits) * kCounterStride, fetch, store, c);
   if (kCount) {
-    atomicAdd(&q.stats64[8], (unsigned long long)wave_turns);
-    atomicAdd(&q.stats64[9], (unsigned long long)lane_turns);
-    atomicAdd(&q.stats64[10], (unsigned long long)tri_rounds);
-  }
-#else
-  for (uint32_t i = gtid; i < n; i += gridDim.x * blockDim.x) {
-    const f3 o = mk3(r[i], r[cap + i], r[2 * cap + i]);
-    const f3 d = mk3(r[3 * cap + i], r[4 * cap + i], r[5 * cap + i]);
-    float t, u, v;
-    const int prim = trace_closest<kCount>(tc, stk, o, d, 0.000001f, t, u, v, nv, nt);
-    q.hit[i] = make_float4(__builtin_bit_cast(float, (int32_t)(prim)), t, u, v);
-  }
-#endif
-  if (kCount) {
-    atomicAdd(&q.stats64[0], (unsigned long long)nv);
-    atomicAdd(&q.stats64[1], (unsigned long long)nt);
+    atomicAdd(&q.stats64[8], (unsigned long long)c.wave_turns);
+    atomicAdd(&q.stats64[9], (unsigned long long)c.lane_turns);
+    atomicAdd(&q.stats64[10], (unsigned long long)c.tri_rounds);
+    atomicAdd(&q.stats64[0], (unsigned long long)c.nodes);
+    atomicAdd(&q.stats64[1], (unsigned long long)c.tests);
   }
 }
 
@@ -199,7 +277,7 @@ constexpr int kCoherentBlock = 256;
 template <bool kCount>
 __global__ __launch_bounds__(kCoherentBlock) NOVA_COHERENT_OCCUPANCY void extend_coherent_kernel(TraceCtx tc, Queues q, int which) {
   uint32_t nv = 0, nt = 0;
-  const uint32_t n = q.count[which];
+  const uint32_t n = q.count[0];  // the first queue: linear
   const float *r = q.ray[which];
   const size_t cap = q.cap;
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -288,28 +366,32 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
     if (threadIdx.x == 0) gcount[(it + 1u) & 1u] = 0;
   };
   const SobolNibbles sobn{sob_tab, sp.dim0};
-  const uint32_t n = q.count[which];
-  const size_t cap = q.cap;
+  const size_t cap = q.cap, paths = q.paths;
   const float *rin = q.ray[which];
   float *rout = q.ray[which ^ 1];
   int32_t *sout = q.slot[which ^ 1];
-  const uint32_t stride = gridDim.x * blockDim.x;
+  // the workgroup's shard of the queue; its survivors go to the same shard of the next one
+  const uint32_t shard = block_shard(q.shard_bits), n = q.shard_n[which][shard * kCounterStride];
+  const uint32_t stride = shard_blocks(q.shard_bits, shard) * blockDim.x;
+  const uint32_t out0 = shard * q.seg;
+  uint32_t *const out_n = &q.shard_n[which ^ 1][shard * kCounterStride];
   // every lane of a wave runs the same number of iterations so the ballot below is uniform
   const uint32_t iters = (n + stride - 1) / stride;
   uint32_t escapes = 0;  // wave-uniform count of escaped paths, added to the statistics once
   __shared__ uint32_t wave_cnt[2][kShadeBlock / 64], blk_base[2];
   for (uint32_t it = 0; it < iters; it++) {
-    const uint32_t i = it * stride + blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t e = it * stride + (blockIdx.x >> q.shard_bits) * blockDim.x + threadIdx.x;
     bool cont = false, escaped = false;
     f3 no = mk3(0, 0, 0), nd = mk3(0, 0, 0);
     int32_t pid = -1;
-    if (i < n) {
+    if (e < n) {
       const bool first = sp.bounce == 0;  // camera rays: path id = queue position, fresh path state
+      const uint32_t i = first ? linear_shard_pos(q.shard_bits, shard, e) : out0 + e;
       pid = first ? (int32_t)i : q.slot[which][i];
       const f3 o = mk3(rin[i], rin[cap + i], rin[2 * cap + i]);
       const f3 d = mk3(rin[3 * cap + i], rin[4 * cap + i], rin[5 * cap + i]);
-      f3 T = first ? mk3(1.f, 1.f, 1.f) : mk3(q.T[pid], q.T[cap + pid], q.T[2 * cap + pid]);
-      f3 L = first ? mk3(0.f, 0.f, 0.f) : mk3(q.L[pid], q.L[cap + pid], q.L[2 * cap + pid]);
+      f3 T = first ? mk3(1.f, 1.f, 1.f) : mk3(q.T[pid], q.T[paths + pid], q.T[2 * paths + pid]);
+      f3 L = first ? mk3(0.f, 0.f, 0.f) : mk3(q.L[pid], q.L[paths + pid], q.L[2 * paths + pid]);
       float A = first ? 0.f : q.A[pid];
       int prim;
       float ht, hu, hv;
@@ -344,14 +426,14 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
       cont = shade_path<kAdj>(sp, sc, sobn, path_slot(sp.fp, (uint32_t)pid), o, d, prim, ht, hu, hv, T, L, A, no, nd, escaped, &padj);
       const bool done = !cont;
       q.T[pid] = T.x;
-      q.T[cap + pid] = T.y;
-      q.T[2 * cap + pid] = T.z;
+      q.T[paths + pid] = T.y;
+      q.T[2 * paths + pid] = T.z;
       if (done) {
         if (!kAdj) write_partial(q, (uint32_t)pid, L.x, L.y, L.z, A);  // a replay reads the primal's
       } else {
         q.L[pid] = L.x;
-        q.L[cap + pid] = L.y;
-        q.L[2 * cap + pid] = L.z;
+        q.L[paths + pid] = L.y;
+        q.L[2 * paths + pid] = L.z;
         q.A[pid] = A;
       }
     }
@@ -359,10 +441,10 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
     // compact survivors into the next queue
     const uint64_t m = __ballot(cont);
     const uint32_t lane_rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-    const uint32_t base = block_reserve<kShadeBlock>(m, &q.count[which ^ 1], it, wave_cnt, blk_base);
+    const uint32_t base = block_reserve<kShadeBlock>(m, out_n, it, wave_cnt, blk_base);
     if (kAdj) flush_table(it);  // every lane has splatted this iteration (block_reserve waited)
     if (cont) {
-      const uint32_t j = base + lane_rank;
+      const uint32_t j = out0 + base + lane_rank;
       rout[j] = no.x;
       rout[cap + j] = no.y;
       rout[2 * cap + j] = no.z;
@@ -400,18 +482,20 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TAIL_OCCUPANCY void tail_kernel(T
   sobol_nibble_fill(sobol, sp.dim0, ndims, sob_tab, threadIdx.x, blockDim.x);
   __syncthreads();
   const SobolNibbles sobn{sob_tab, sp.dim0};
-  const uint32_t n = q.count[which];
+  const uint32_t shard = block_shard(q.shard_bits), n = q.shard_n[which][shard * kCounterStride];
   const float *rin = q.ray[which];
-  const size_t cap = q.cap;
+  const size_t cap = q.cap, paths = q.paths;
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   LdsStack stk{tail_lds, tc.gstack, tc.gstride, gtid, threadIdx.x};
   uint32_t nv = 0, nt = 0, segs = 0, escapes = 0;
-  for (uint32_t i = gtid; i < n; i += gridDim.x * blockDim.x) {
+  const uint32_t stride = shard_blocks(q.shard_bits, shard) * blockDim.x;
+  for (uint32_t e = (blockIdx.x >> q.shard_bits) * blockDim.x + threadIdx.x; e < n; e += stride) {
+    const uint32_t i = shard * q.seg + e;
     const int32_t pid = q.slot[which][i];
     f3 o = mk3(rin[i], rin[cap + i], rin[2 * cap + i]);
     f3 d = mk3(rin[3 * cap + i], rin[4 * cap + i], rin[5 * cap + i]);
-    f3 T = mk3(q.T[pid], q.T[cap + pid], q.T[2 * cap + pid]);
-    f3 L = mk3(q.L[pid], q.L[cap + pid], q.L[2 * cap + pid]);
+    f3 T = mk3(q.T[pid], q.T[paths + pid], q.T[2 * paths + pid]);
+    f3 L = mk3(q.L[pid], q.L[paths + pid], q.L[2 * paths + pid]);
     float A = q.A[pid];
     const uint32_t slot = path_slot(sp.fp, (uint32_t)pid);
     ShadeParams s = sp;
@@ -446,11 +530,13 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TAIL_OCCUPANCY void tail_kernel(T
   }
 }
 
-// Between an extend and a shade launch: the shade's output queue and the next extend's work
-// counter start at zero.
-__global__ void reset_count_kernel(uint32_t *count, int which) {
-  count[which] = 0;
-  count[kWorkCounter] = 0;
+// Between an extend and a shade launch: the shade's output queue and the next extend's claims
+// start at zero.
+__global__ void reset_count_kernel(Queues q, int which) {
+  if (threadIdx.x < (1u << q.shard_bits)) {
+    q.shard_n[which][threadIdx.x * kCounterStride] = 0;
+    q.work[threadIdx.x * kCounterStride] = 0;
+  }
 }
 
 // Engine::writeFramebuffer per frame, in frame order (engine.cpp:351-363); one thread per
@@ -565,35 +651,77 @@ __global__ __launch_bounds__(kTraceBlock) void closest_hit_kernel(TraceCtx tc, c
   }
 }
 
-// Render passes (NORMAL / DEPTH / EMISSIVE): one unjittered ray per pixel, the pass value
-// (pass_value) accumulated for every frame as the path integrator's frames are.
-__global__ __launch_bounds__(kTraceBlock) void pass_kernel(TraceCtx tc, ShadeCtx sc, const uint32_t *__restrict__ sobol, FrameParams fp, int pass,
-                                                           float z_near, float z_far, float *__restrict__ accum, float *__restrict__ final_out,
-                                                           float *__restrict__ partial_out) {
-  __shared__ uint32_t lds[kLdsStack * kTraceBlock];
-  const uint32_t npix = (uint32_t)fp.width * (uint32_t)fp.height;
+// The same for many rays per lane: lanes refill, and every workgroup has a share of the rays with
+// its claim counter in LDS (nothing for a caller to clear, no rate of a shared counter, and calls
+// on several streams share no claims). 3,000,000 rays into 100,480 triangles: 670 -> 515 us, into
+// 1,048,576: 888 -> 690 us.
+__global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void closest_hit_refill_kernel(TraceCtx tc, const float *__restrict__ rays, uint32_t n,
+                                                                                              int32_t *__restrict__ prim, float *__restrict__ tuv) {
+  __shared__ uint32_t lds[kLdsStack * kTraceBlock], claims;
+  if (threadIdx.x == 0) claims = 0;
+  __syncthreads();
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   LdsStack stk{lds, tc.gstack, tc.gstride, gtid, threadIdx.x};
-  for (uint32_t p = gtid; p < npix; p += gridDim.x * blockDim.x) {
-    f3 o, d;
-    camera_ray_pass(fp, p, o, d);
-    float t, u, v;
-    uint32_t nv = 0, nt = 0;
-    const int prim = trace_closest<false>(tc, stk, o, d, 0.000001f, t, u, v, nv, nt);
-    const float4 val = pass_value(pass, fp, sc, sobol, p, o, d, prim, t, u, v, z_near, z_far);
-    const uint32_t i = pixel_offset(fp, p);
-    float a[4] = {accum[i], accum[i + 1], accum[i + 2], accum[i + 3]}, fin[4] = {0.f, 0.f, 0.f, 0.f};
+  WalkCounts c;
+  refill_walk<false>(
+      tc, stk, workgroup_share(n), &claims,
+      [&](uint32_t i, f3 &o, f3 &d) {
+        const float *r = rays + (size_t)i * 6;
+        o = mk3(r[0], r[1], r[2]);
+        d = mk3(r[3], r[4], r[5]);
+      },
+      [&](uint32_t i, const TraceState &st) {
+        prim[i] = st.best;
+        float *o = tuv + (size_t)i * 3;
+        o[0] = st.best >= 0 ? st.tbest : 0.f;
+        o[1] = st.bu;
+        o[2] = st.bv;
+      },
+      c);
+}
+
+// Render passes (NORMAL / DEPTH / EMISSIVE): one unjittered ray per pixel, in two launches with
+// the hits in the pixels of the final image between them. The walk takes its rays in 8x8 tiles
+// and with lane refill, at its own register budget. One kernel that walked row by row and shaded
+// in place ran at 205 registers, two waves per SIMD, and computed a whole BSDF sample whatever
+// the pass: 1.08 ms for the normals of the 1,048,576-triangle scene at 1080p, these two 0.47.
+__global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void pass_trace_kernel(TraceCtx tc, FrameParams fp, float *__restrict__ hits) {
+  __shared__ uint32_t lds[kLdsStack * kTraceBlock], claims;
+  if (threadIdx.x == 0) claims = 0;
+  __syncthreads();
+  const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
+  LdsStack stk{lds, tc.gstack, tc.gstride, gtid, threadIdx.x};
+  WalkCounts c;
+  refill_walk<false>(
+      tc, stk, workgroup_share((uint32_t)fp.width * (uint32_t)fp.height), &claims,
+      [&](uint32_t i, f3 &o, f3 &d) { camera_ray_pass(fp, pixel_of_rank(fp, i), o, d); },
+      [&](uint32_t i, const TraceState &st) {
+        const float4 h = hit_record(st);
+        __builtin_memcpy(hits + pixel_offset(fp, pixel_of_rank(fp, i)), &h, sizeof(h));
+      },
+      c);
+}
+
+template <int kPass>
+__global__ __launch_bounds__(256) void pass_shade_kernel(ShadeCtx sc, const uint32_t *__restrict__ sobol, FrameParams fp, const float *hits, float z_near,
+                                                         float z_far, float *accum, float *final_out, float *partial_out) {
+  const uint32_t npix = (uint32_t)fp.width * (uint32_t)fp.height;
+  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < npix; k += gridDim.x * blockDim.x) {
+    const uint32_t p = pixel_of_rank(fp, k), i = pixel_offset(fp, p);
+    float h[4];
+    __builtin_memcpy(h, hits + i, sizeof(h));
+    f3 o = mk3(0.f, 0.f, 0.f), d = o;
+    if (kPass != PASS_DEPTH) camera_ray_pass(fp, p, o, d);
+    const float4 val = pass_value(kPass, fp, sc, sobol, p, o, d, __builtin_bit_cast(int32_t, h[0]), h[1], h[2], h[3], z_near, z_far);
     const float vv[4] = {val.x, val.y, val.z, val.w};
+    float a[4], fin[4];
+    __builtin_memcpy(a, accum + i, sizeof(a));
     for (int f = 0; f < fp.frames; f++)  // Engine::writeFramebuffer per frame, in frame order
-      for (int c = 0; c < 4; c++) {
-        a[c] += vv[c];
-        fin[c] = a[c] / float(fp.frame0 + f + 1);
-      }
-    for (int c = 0; c < 4; c++) {
-      accum[i + c] = a[c];
-      final_out[i + c] = fin[c];
-      if (partial_out) partial_out[i + c] = vv[c];
-    }
+      for (int c = 0; c < 4; c++) a[c] += vv[c];
+    for (int c = 0; c < 4; c++) fin[c] = a[c] / float(fp.frame0 + fp.frames);
+    __builtin_memcpy(accum + i, a, sizeof(a));
+    __builtin_memcpy(final_out + i, fin, sizeof(fin));
+    if (partial_out) __builtin_memcpy(partial_out + i, vv, sizeof(vv));
   }
 }
 
@@ -699,13 +827,34 @@ struct ScratchCarve {
   }
 };
 
+// How a batch's queues are cut: 2^bits shards of at least 4,096 paths each.
+struct QueueShape {
+  uint32_t bits, seg;
+  size_t entries;  // of one queue: the shards' room, a little more than the paths
+};
+static QueueShape queue_shape(size_t paths, uint32_t max_bits) {
+  QueueShape q{0, (uint32_t)paths, paths};
+  while (q.bits < max_bits && (paths >> (q.bits + 1)) >= 4096) q.bits++;
+  if (q.bits == 0) return q;
+  const size_t chunks = (paths + kQueueChunk - 1) / kQueueChunk, S = (size_t)1 << q.bits;
+  q.seg = (uint32_t)((chunks + S - 1) / S * kQueueChunk);
+  q.entries = (size_t)q.seg * S;
+  return q;
+}
+// Counters: a line of control words and statistics, then the two queues' and the claims' lines.
+// One shard keeps its three words in the first line.
+constexpr size_t kControlBytes = 256, kShardLineBytes = kCounterStride * sizeof(uint32_t);
+constexpr size_t kCounterBytes = kControlBytes + 3 * ((size_t)1 << kMaxShardBits) * kShardLineBytes;
+static size_t counter_bytes(uint32_t bits) { return bits == 0 ? kControlBytes : kCounterBytes; }
+
 // Bytes a batch of `cap` paths needs in the fixed array: the queues and path state (116 B
 // per path), the counters and the traversal overflow stacks of `threads` lanes.
-static size_t noalloc_bytes(size_t cap, uint32_t threads, uint32_t stack_bound) {
-  const size_t per_path[] = {cap * 12 * sizeof(float), cap * 2 * sizeof(int32_t), cap * 4 * sizeof(float), cap * 7 * sizeof(float),
-                             cap * 4 * sizeof(float)};
-  size_t total = 256 + 256;  // counters
-  for (size_t b : per_path) total += (b + 255) / 256 * 256;
+static size_t noalloc_bytes(size_t cap, uint32_t max_bits, uint32_t threads, uint32_t stack_bound) {
+  const QueueShape qs = queue_shape(cap, max_bits);
+  const size_t pieces[] = {qs.entries * 12 * sizeof(float), qs.entries * 2 * sizeof(int32_t), qs.entries * 4 * sizeof(float), cap * 7 * sizeof(float),
+                           cap * 4 * sizeof(float)};
+  size_t total = 256 + counter_bytes(qs.bits);
+  for (size_t b : pieces) total += (b + 255) / 256 * 256;
   const size_t g = stack_bound > (uint32_t)kLdsStack ? (size_t)(stack_bound - kLdsStack) * threads : 1;
   return total + (g * sizeof(uint32_t) + 255) / 256 * 256;
 }
@@ -720,12 +869,23 @@ extern "C" int nova_hip_closest_hit(nova_hip_ctx *ctx, const float *rays_dev, ui
   if (n == 0) return NOVA_HIP_SUCCESS;
   if (!rays_dev || !prim_dev || !tuv_dev) return set_error(ctx, NOVA_HIP_INVALID_ARGUMENT, "null buffer");
   NOVA_HIP_CHECK(ctx, hipSetDevice(ctx->device));
-  const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + kTraceBlock - 1) / kTraceBlock, (uint64_t)device_cus(ctx) * 8);
+  const uint64_t cus = (uint64_t)device_cus(ctx);
+  // From two rays per lane on, lanes refill (1,000,000 rays into 1,048,576 triangles: 396 -> 340 us);
+  // below that a refilled walk has nothing to win and its lanes take longer (262,147 rays: 127 against 135 us).
+  const bool refill = n >= 2 * cus * NOVA_TRACE_BLOCKS_PER_CU * kTraceBlock;
+  const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + kTraceBlock - 1) / kTraceBlock, cus * (refill ? NOVA_TRACE_BLOCKS_PER_CU : 8));
   const uint32_t threads = blocks * kTraceBlock;
   int st = ensure_gstack(ctx, threads);
   if (st) return st;
   TraceCtx tc{ctx->nodes4, ctx->tri_leaf, ctx->gstack, threads, ctx->tie};
-  hipLaunchKernelGGL(closest_hit_kernel, dim3(blocks), dim3(kTraceBlock), 0, (hipStream_t)stream, tc, rays_dev, n, prim_dev, tuv_dev);
+  if (refill) {
+    constexpr uint64_t kMost = 1u << 30;  // rays per launch: entries stay in 32 bits
+    for (uint64_t at = 0; at < n; at += kMost)
+      hipLaunchKernelGGL(closest_hit_refill_kernel, dim3(blocks), dim3(kTraceBlock), 0, (hipStream_t)stream, tc, rays_dev + at * 6,
+                         (uint32_t)std::min(n - at, kMost), prim_dev + at, tuv_dev + at * 3);
+  } else {
+    hipLaunchKernelGGL(closest_hit_kernel, dim3(blocks), dim3(kTraceBlock), 0, (hipStream_t)stream, tc, rays_dev, n, prim_dev, tuv_dev);
+  }
   NOVA_HIP_CHECK(ctx, hipGetLastError());
   return NOVA_HIP_SUCCESS;
 }
@@ -759,10 +919,19 @@ static int call_events(nova_hip_ctx *ctx, hipEvent_t *ev0, hipEvent_t *ev1) {
 static int render_pass(nova_hip_ctx *ctx, const nova_hip_render_params *p, int pass, float *accum_dev, float *final_dev, float *partial_dev,
                        hipStream_t s, bool async) {
   const uint32_t npix = (uint32_t)p->width * (uint32_t)p->height;
-  const uint32_t blocks = std::min<uint32_t>((npix + kTraceBlock - 1) / kTraceBlock, (uint32_t)device_cus(ctx) * 8);
+  const uint32_t cus = (uint32_t)device_cus(ctx);
+  const uint32_t blocks = std::min<uint32_t>((npix + kTraceBlock - 1) / kTraceBlock, cus * NOVA_TRACE_BLOCKS_PER_CU);
   const uint32_t threads = blocks * kTraceBlock;
   int st = ensure_gstack(ctx, threads);
   if (st) return st;
+  // the hits wait in the final image's pixels; an image that lies over the accumulated one leaves no room for them
+  float *hits = final_dev;
+  const uintptr_t bytes = (uintptr_t)npix * 4 * sizeof(float), a0 = (uintptr_t)accum_dev, f0 = (uintptr_t)final_dev;
+  if (a0 < f0 + bytes && f0 < a0 + bytes) {
+    hipError_t e = hipSuccess;
+    hits = (float *)ensure_scratch(ctx, 3, bytes, &e);
+    if (!hits) return check_hip(ctx, e, "hit alloc");
+  }
   TraceCtx tc{ctx->nodes4, ctx->tri_leaf, ctx->gstack, threads, ctx->tie};
   ShadeCtx sc{ctx->textures, ctx->tex_u32, ctx->tex_f32, ctx->materials, ctx->mesh_xf, ctx->shade, ctx->acos_lut, ctx->envmap, -1};
   FrameParams fp;
@@ -771,7 +940,7 @@ static int render_pass(nova_hip_ctx *ctx, const nova_hip_render_params *p, int p
   fp.frame0 = p->frame_start;
   fp.frames = p->frame_count;
   fp.frame_minor = 0;
-  fp.tiled = 0;
+  fp.tiled = 1;
   fp.offset = 0;
   fp.vinvert = p->vertical_invert;
   fp.policy = NOVA_HIP_INDEX_CPU;
@@ -779,19 +948,24 @@ static int render_pass(nova_hip_ctx *ctx, const nova_hip_render_params *p, int p
     fp.inv_P[i] = p->inv_P[i];
     fp.inv_V[i] = p->inv_V[i];
   }
-  if (async) {  // queued; statistics untouched
-    hipLaunchKernelGGL(pass_kernel, dim3(blocks), dim3(kTraceBlock), 0, s, tc, sc, ctx->sobol_table, fp, pass, p->z_near, p->z_far, accum_dev,
-                       final_dev, partial_dev);
-    NOVA_HIP_CHECK(ctx, hipGetLastError());
-    return NOVA_HIP_SUCCESS;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  if (!async) {  // queued calls leave the statistics untouched
+    if ((st = call_events(ctx, &ev0, &ev1))) return st;
+    NOVA_HIP_CHECK(ctx, hipEventRecord(ev0, s));
   }
-  hipEvent_t ev0, ev1;
-  int est = call_events(ctx, &ev0, &ev1);
-  if (est) return est;
-  NOVA_HIP_CHECK(ctx, hipEventRecord(ev0, s));
-  hipLaunchKernelGGL(pass_kernel, dim3(blocks), dim3(kTraceBlock), 0, s, tc, sc, ctx->sobol_table, fp, pass, p->z_near, p->z_far, accum_dev, final_dev,
-                     partial_dev);
+  hipLaunchKernelGGL(pass_trace_kernel, dim3(blocks), dim3(kTraceBlock), 0, s, tc, fp, hits);
+  const dim3 grid(std::min<uint32_t>((npix + 255) / 256, cus * 16));
+  auto shade = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, sc, ctx->sobol_table, fp, hits, p->z_near, p->z_far, accum_dev, final_dev, partial_dev);
+  };
+  if (pass == PASS_NORMAL)
+    shade(pass_shade_kernel<PASS_NORMAL>);
+  else if (pass == PASS_DEPTH)
+    shade(pass_shade_kernel<PASS_DEPTH>);
+  else
+    shade(pass_shade_kernel<PASS_EMISSIVE>);
   NOVA_HIP_CHECK(ctx, hipGetLastError());
+  if (async) return NOVA_HIP_SUCCESS;
   NOVA_HIP_CHECK(ctx, hipEventRecord(ev1, s));
   NOVA_HIP_CHECK(ctx, hipEventSynchronize(ev1));
   float ms = 0.f;
@@ -857,14 +1031,18 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
   auto trace_threads_of = [&](size_t c) {
     return (uint32_t)std::min<size_t>((c + kTraceBlock - 1) / kTraceBlock, (size_t)cus * NOVA_TRACE_BLOCKS_PER_CU) * kTraceBlock;
   };
+  uint32_t max_bits = kMaxShardBits;
   if (noalloc) {
-    // as many frames per batch as the fixed array holds
-    while (fb > 0 && noalloc_bytes(npix * fb, trace_threads_of(npix * fb), traversal_stack_bound(ctx)) > kNoAllocScratchBytes) fb--;
+    // as many frames per batch as the fixed array holds (one shard: the least memory)
+    auto bytes_of = [&](int frames, uint32_t max_bits) {
+      return noalloc_bytes(npix * frames, max_bits, trace_threads_of(npix * frames), traversal_stack_bound(ctx));
+    };
+    while (fb > 0 && bytes_of(fb, 0) > kNoAllocScratchBytes) fb--;
     if (fb == 0)
       return set_error(ctx, NOVA_HIP_INVALID_ARGUMENT,
-                       "image of " + std::to_string(npix) + " pixels needs " +
-                           std::to_string(noalloc_bytes(npix, trace_threads_of(npix), traversal_stack_bound(ctx))) +
+                       "image of " + std::to_string(npix) + " pixels needs " + std::to_string(bytes_of(1, 0)) +
                            " bytes of scratch per frame; the no-allocation entry point holds " + std::to_string(kNoAllocScratchBytes));
+    while (max_bits > 0 && bytes_of(fb, max_bits) > kNoAllocScratchBytes) max_bits--;
   }
   const size_t cap = npix * fb;
   if (cap >= (1u << 31)) return set_error(ctx, NOVA_HIP_INVALID_ARGUMENT, "image too large");
@@ -876,26 +1054,40 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
     if (!r) e = hipErrorOutOfMemory;
     return r;
   };
+  const QueueShape qs = queue_shape(cap, max_bits);
+  const size_t qn = qs.entries;
   Queues q;
-  q.cap = (uint32_t)cap;
-  float *rays = (float *)piece(0, cap * 12 * sizeof(float));
+  q.cap = (uint32_t)qn;
+  q.paths = (uint32_t)cap;
+  q.shard_bits = qs.bits;
+  q.seg = qs.seg;
+  float *rays = (float *)piece(0, qn * 12 * sizeof(float));
   if (!rays) return check_hip(ctx, e, "queue alloc");
-  int32_t *slots = (int32_t *)piece(1, cap * 2 * sizeof(int32_t));
+  int32_t *slots = (int32_t *)piece(1, qn * 2 * sizeof(int32_t));
   if (!slots) return check_hip(ctx, e, "queue alloc");
-  uint32_t *counts = (uint32_t *)piece(2, 256);
+  uint32_t *counts = (uint32_t *)piece(2, noalloc ? counter_bytes(qs.bits) : kCounterBytes);
   if (!counts) return check_hip(ctx, e, "counter alloc");
   unsigned long long *stats64 = (unsigned long long *)(counts + 8);
-  float *hits = (float *)piece(3, cap * 4 * sizeof(float));
+  float *hits = (float *)piece(3, qn * 4 * sizeof(float));
   if (!hits) return check_hip(ctx, e, "hit alloc");
   float *state = (float *)piece(4, cap * 7 * sizeof(float));
   if (!state) return check_hip(ctx, e, "state alloc");
   float *partial = (float *)piece(5, cap * 4 * sizeof(float));
   if (!partial) return check_hip(ctx, e, "partial alloc");
   q.ray[0] = rays;
-  q.ray[1] = rays + cap * 6;
+  q.ray[1] = rays + qn * 6;
   q.slot[0] = slots;
-  q.slot[1] = slots + cap;
+  q.slot[1] = slots + qn;
   q.count = counts;
+  if (qs.bits == 0) {  // words 48 and up of the first line: the statistics end there
+    q.shard_n[0] = counts + 48;
+    q.shard_n[1] = counts + 49;
+    q.work = counts + 50;
+  } else {
+    q.shard_n[0] = counts + kControlBytes / sizeof(uint32_t);
+    q.shard_n[1] = q.shard_n[0] + (kCounterStride << kMaxShardBits);
+    q.work = q.shard_n[1] + (kCounterStride << kMaxShardBits);
+  }
   q.stats64 = stats64;
   q.hit = reinterpret_cast<float4 *>(hits);
   q.T = state;
@@ -1040,7 +1232,7 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
                            tail_last ? 1 : 0);
       }
       if (timing && (st = stamp())) return st;
-      hipLaunchKernelGGL(reset_count_kernel, dim3(1), dim3(1), 0, s, counts, which ^ 1);
+      hipLaunchKernelGGL(reset_count_kernel, dim3(1), dim3(64), 0, s, q, which ^ 1);
       ShadeParams spp;
       spp.fp = fp;
       spp.bounce = k;
@@ -1056,9 +1248,11 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
       if (timing && (st = stamp())) return st;
       NOVA_HIP_CHECK(ctx, hipGetLastError());
       if (tail_here) {
-        // at most trace_threads lanes: the overflow stacks are sized for the extend grid
-        const uint32_t tblocks = std::min<uint32_t>({(uint32_t)((std::min<size_t>(tail_last ? cap : tail_rays, cap) + kTraceBlock - 1) / kTraceBlock),
-                                                     trace_blocks, (uint32_t)cus * 4});
+        // at most trace_threads lanes: the overflow stacks are sized for the extend grid. A
+        // workgroup per shard more than the rays need, since the shards differ a little
+        const uint32_t tblocks =
+            std::min<uint32_t>({(uint32_t)((std::min<size_t>(tail_last ? cap : tail_rays, cap) + kTraceBlock - 1) / kTraceBlock) + (1u << qs.bits),
+                                trace_blocks, (uint32_t)cus * 5});
         if (timing && (st = stamp())) return st;
         if (timing) kkind.push_back(3);
         if (counting)
