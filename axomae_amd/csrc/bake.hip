@@ -1,14 +1,18 @@
-// Batched environment-map bakes: one launch covers every output texel of every map.
+// Batched environment-map bakes: one call covers every output texel of every map.
 //  * diffuse irradiance: TextureOperations<float>::computeDiffuseIrradiance
 //    (TextureProcessing.cpp:9-64, TextureProcessing.h:253-301) - pgc3d-hashed cosine
 //    samples per texel, looked up with the nearest-texel rule uvSample degenerates to;
 //  * GGX prefiltered specular: envmap_prefilter.frag:1-116 on equirect, level 0;
-//  * the split-sum BRDF table: brdf_lookup_table_baker.frag:1-117.
-// Each output texel is one lane; samples are summed in the reference's order.
+//  * the split-sum BRDF table: brdf_lookup_table_baker.frag:1-117;
+//  * the GL viewer's cube capture and Riemann irradiance.
+// The samples of a texel lie across the lanes of a workgroup, and their sums are added in a
+// fixed tree (bake_kernel).
 #include <algorithm>
 #include <vector>
 
 #include "device_math.h"
+#include "device_path.h"
+#include "device_trig.h"
 #include "nova_internal.h"
 
 namespace nova_hip {
@@ -19,36 +23,45 @@ struct BakeMap {
   int32_t w, h, c, ow, oh;
   int32_t kind;  // NOVA_HIP_BAKE_*
   float roughness;
-  uint64_t first;  // first global texel index of this map
+  uint64_t first;  // first work item of this job: a group of texels in bake_kernel, a texel elsewhere
+  uint32_t block_row;  // bake_kernel: blocks of kGroupRun groups in a row of blocks; lut_kernel: waves of a row
 };
+
+// A texel of three or four channels. Maps lie in device global memory: through the global address
+// space the loads are global ones, not flat.
+#ifdef __HIP_DEVICE_COMPILE__
+typedef const __attribute__((address_space(1))) float GlobalFloat;
+typedef const __attribute__((address_space(1))) float4 GlobalFloat4;
+#else
+typedef const float GlobalFloat;
+typedef const float4 GlobalFloat4;
+#endif
+__device__ __forceinline__ f3 load_texel(const BakeMap &m, unsigned x, unsigned y) {
+  const size_t i = (size_t)y * (unsigned)m.w + x;
+  if (m.c == 4) {  // RGBA texels of a 16-byte aligned map: one vector load
+    float4 t;
+    __builtin_memcpy(&t, (GlobalFloat4 *)m.env + i, sizeof(t));
+    return mk3(t.x, t.y, t.z);
+  }
+  GlobalFloat *p = (GlobalFloat *)m.env + ((i << 1) + i);
+  return mk3(p[0], p[1], p[2]);
+}
 
 __device__ __forceinline__ unsigned uv_to_pixel(float coord, unsigned dim) { return (unsigned)(long long)(coord * (float)dim); }
 
 // sphericalToCartesian<float> (math_spherical.h:33-39)
 __device__ __forceinline__ f3 sph_to_cart(float phi, float theta) {
-  const float z = cos_f(theta);
-  const float x = sin_f(theta) * cos_f(phi);
-  const float y = sin_f(theta) * sin_f(phi);
-  return mk3(x, y, z);
+  float sp, cp, st, ct;
+  sincos_turns(phi, sp, cp);
+  sincos_turns(theta, st, ct);
+  return mk3(st * cp, st * sp, ct);
 }
 
-// discreteSample + uvSample (TextureProcessing.h:173-210)
-__device__ __forceinline__ f3 discrete(const BakeMap &m, int x, int y) {
-  int xc, yc;
-  x = x < 0 ? 0 : x;  // coordinates come from unsigned texel indices; a NaN direction must stay in bounds
-  y = y < 0 ? 0 : y;
-  if (x >= m.w) xc = x % m.w;
-  else if (x < 0) xc = m.w + (x % m.w);
-  else xc = x;
-  if (y >= m.h) yc = y % m.h;
-  else if (y < 0) yc = m.h + (y % m.h);
-  else yc = y;
-  const float *p = m.env + ((size_t)yc * m.w + xc) * m.c;
-  if (m.c == 4) {  // RGBA texels of a 16-byte aligned map: one vector load
-    const float4 t = *reinterpret_cast<const float4 *>(p);
-    return mk3(t.x, t.y, t.z);
-  }
-  return mk3(p[0], p[1], p[2]);
+// discreteSample + uvSample (TextureProcessing.h:173-210) at pixel coordinates of at most (w, h);
+// a coordinate of w or h wraps to 0
+__device__ __forceinline__ f3 discrete(const BakeMap &m, unsigned x, unsigned y) {
+  const unsigned xc = x == (unsigned)m.w ? 0u : x, yc = y == (unsigned)m.h ? 0u : y;
+  return load_texel(m, xc, yc);
 }
 
 // uvSample: the pixel coordinates px, py are whole numbers (an unsigned texel index turned
@@ -60,8 +73,9 @@ __device__ __forceinline__ f3 uv_sample(const BakeMap &m, float u, float v) {
   const float ui = floorf(u), vi = floorf(v);
   const float up = (u > 1. || u < 0.) ? u - ui : u;
   const float vp = (v > 1. || v < 0.) ? v - vi : v;
-  const unsigned px = min(uv_to_pixel(up, (unsigned)m.w), (unsigned)m.w), py = min(uv_to_pixel(vp, (unsigned)m.h), (unsigned)m.h);
-  return discrete(m, (int)px, (int)py);
+  // up and vp lie in [0, 1] (the coordinate 0 for a NaN): the conversion needs no 64 bits
+  const unsigned px = min((unsigned)(up * (float)m.w), (unsigned)m.w), py = min((unsigned)(vp * (float)m.h), (unsigned)m.h);
+  return discrete(m, px, py);
 }
 
 __device__ __forceinline__ f3 dir_sample(const BakeMap &m, const float *lut, f3 d) {
@@ -107,62 +121,6 @@ __device__ __forceinline__ int find_map(const BakeMap *maps, int count, uint64_t
   return lo;
 }
 
-// One irradiance texel. The reference draws its cosine samples from pgc3d of the texel's
-// recomputed pixel and the sample number; the Sobol variant takes Owen-scrambled Sobol
-// points (dims 0 and 1) at indices texel * samples + s, so each texel gets its own
-// stratified block of the sequence.
-__device__ __forceinline__ f3 irradiance_texel(const BakeMap &m, const float *__restrict__ lut, const uint32_t *__restrict__ sobol, unsigned i,
-                                               unsigned j, int samples) {
-  {
-    const float u = (float)((double)i / (double)m.ow), v = (float)((double)j / (double)m.oh);
-    const f3 nrm = sph_to_cart((float)(2 * 3.14159265358979323846 * u), (float)(3.14159265358979323846 * v));
-    const float aphi = atan2_approx(nrm.y, nrm.x), atheta = acos_lt(lut, nrm.z);
-    const double inv_2pi = 1.f / (2.f * 3.14159265358979323846), inv_pi = 1.f / 3.14159265358979323846;
-    const unsigned px = uv_to_pixel((float)(aphi * inv_2pi), (unsigned)m.ow), py = uv_to_pixel((float)(atheta * inv_pi), (unsigned)m.oh);
-    const f3 right = mk3(1.f, 0.f, 0.f);
-    const float dd = dot(right, nrm);
-    f3 tangent = mk3(0.f, 1.f, 0.f);
-    if (1.0 - fabs((double)dd) > 1e-6) tangent = normalize(cross(right, nrm));
-    const f3 bitangent = cross(nrm, tangent);
-    f3 irr = mk3(0.f, 0.f, 0.f);
-    const uint32_t base = (j * (uint32_t)m.ow + i) * (uint32_t)samples;
-    // Sobol points of consecutive indices: the gray code of idx differs from idx-1's in bit
-    // ctz(idx), so each sample XORs one direction number into the running values (equal to
-    // the direct gray-code sum bit for bit).
-    uint32_t ax = 0, ay = 0;
-    if (m.kind == NOVA_HIP_BAKE_IRRADIANCE_SOBOL) {
-      const uint32_t g0 = base ^ (base >> 1);
-      ax = sobol_xor(sobol, g0);
-      ay = sobol_xor(sobol + 32, g0);
-    }
-    for (int s = 0; s < samples; s++) {
-      float rx, ry;
-      if (m.kind == NOVA_HIP_BAKE_IRRADIANCE_SOBOL) {
-        if (s > 0) {
-          const uint32_t bit = (uint32_t)__builtin_ctz(base + (uint32_t)s);
-          ax ^= sobol[bit];
-          ay ^= sobol[32 + bit];
-        }
-        rx = u32_to_unit(owen_scramble(ax));
-        ry = u32_to_unit(owen_scramble(ay));
-      } else {
-        const f3 r = pgc3d(px, py, (unsigned)s);
-        rx = r.x;
-        ry = r.y;
-      }
-      // cosine sample at phi = 2 pi rx, theta = asin(sqrt(ry)) (TextureProcessing.h:270-276):
-      // sin(theta) = sqrt(ry), cos(theta) = sqrt(1 - ry)
-      float sp, cp;
-      sincos_2pi(rx, sp, cp);
-      const float st = sqrtf(ry), ct = sqrtf(1.f - ry);
-      f3 c = mk3(st * cp, st * sp, ct);
-      c = c.x * tangent + c.y * bitangent + c.z * nrm;
-      irr = irr + dir_sample(m, lut, c);
-    }
-    return irr / (float)samples;
-  }
-}
-
 __device__ __forceinline__ float radical_inverse(unsigned bits) {
   bits = (bits << 16u) | (bits >> 16u);
   bits = ((bits & 0x55555555u) << 1u) | ((bits & 0xAAAAAAAAu) >> 1u);
@@ -172,81 +130,13 @@ __device__ __forceinline__ float radical_inverse(unsigned bits) {
   return (float)bits * 2.3283064365386963e-10f;
 }
 
-// One prefiltered-specular texel: N = V = R, Hammersley GGX half vectors, NdotL weights.
-__device__ __forceinline__ f3 prefilter_texel(const BakeMap &m, const float *__restrict__ lut, unsigned i, unsigned j, int samples) {
-  {
-    const float u = (float)((double)i / (double)m.ow), v = (float)((double)j / (double)m.oh);
-    const f3 N = normalize(sph_to_cart((float)(2 * 3.14159265358979323846 * u), (float)(3.14159265358979323846 * v)));
-    f3 col = mk3(0.f, 0.f, 0.f);
-    if (m.roughness == 0.f) {
-      col = dir_sample(m, lut, N);
-    } else {
-      float total_w = 0.f;
-      const float a = m.roughness * m.roughness;
-      const f3 up = fabsf(N.z) < 0.999f ? mk3(0.f, 0.f, 1.f) : mk3(1.f, 0.f, 0.f);
-      const f3 t = normalize(cross(up, N));
-      const f3 b = cross(N, t);
-      for (int s = 0; s < samples; s++) {
-        const float xi0 = (float)s / (float)samples, xi1 = radical_inverse((unsigned)s);
-        const float ct = sqrtf((1.0f - xi1) / (1.0f + (a * a - 1.0f) * xi1));
-        const float st = sqrtf(1.0f - ct * ct);
-        float sp, cp;
-        sincos_2pi(xi0, sp, cp);
-        const f3 H = normalize(t * (cp * st) + b * (sp * st) + N * ct);
-        const f3 L = reflect(-N, H);
-        const float ndl = fmaxf(dot(N, L), 0.f);
-        if (ndl > 0.f) {
-          col = col + dir_sample(m, lut, L) * ndl;
-          total_w += ndl;
-        }
-      }
-      col = col / total_w;
-    }
-    return col;
-  }
-}
-
-// computeLut (brdf_lookup_table_baker.frag:74-113) at texel (i, j): NdotV = (i + 0.5) / ow,
-// roughness = (j + 0.5) / oh; the split-sum scale A and bias B over `samples` Hammersley GGX
-// half vectors about N = +z, with GeometrySmith's k = roughness^2 / 2.
+// GeometrySmith's k = roughness^2 / 2
 __device__ __forceinline__ float schlick_ggx_ibl(float ndotv, float roughness) {
   const float a = roughness;
   const float k = (a * a) / 2.0f;
-  return ndotv / (ndotv * (1.0f - k) + k);
+  return div_mid(ndotv, ndotv * (1.0f - k) + k);
 }
 
-__device__ __forceinline__ float2 brdf_lut_texel(const BakeMap &m, unsigned i, unsigned j, int samples) {
-  const float ndotv = ((float)i + 0.5f) / (float)m.ow, roughness = ((float)j + 0.5f) / (float)m.oh;
-  const f3 V = mk3(sqrtf(1.0f - ndotv * ndotv), 0.0f, ndotv);
-  const f3 N = mk3(0.f, 0.f, 1.f);
-  const float a = roughness * roughness;
-  const f3 up = fabsf(N.z) < 0.999f ? mk3(0.f, 0.f, 1.f) : mk3(1.f, 0.f, 0.f);
-  const f3 t = normalize(cross(up, N));
-  const f3 b = cross(N, t);
-  const float gv = schlick_ggx_ibl(fmaxf(dot(N, V), 0.0f), roughness);
-  float A = 0.f, B = 0.f;
-  for (int s = 0; s < samples; s++) {
-    const float xi0 = (float)s / (float)samples, xi1 = radical_inverse((unsigned)s);
-    const float ct = sqrtf((1.0f - xi1) / (1.0f + (a * a - 1.0f) * xi1));
-    const float st = sqrtf(1.0f - ct * ct);
-    float sp, cp;
-    sincos_2pi(xi0, sp, cp);
-    const f3 H = normalize(t * (cp * st) + b * (sp * st) + N * ct);
-    const f3 L = normalize(H * (2.0f * dot(V, H)) - V);
-    const float ndl = fmaxf(L.z, 0.0f), ndh = fmaxf(H.z, 0.0f), vdh = fmaxf(dot(V, H), 0.0f);
-    if (ndl > 0.0f) {
-      const float G = schlick_ggx_ibl(ndl, roughness) * gv;
-      const float g_vis = (G * vdh) / (ndh * ndotv);
-      const float fc = pow5(1.0f - vdh);
-      A += (1.0f - fc) * g_vis;
-      B += fc * g_vis;
-    }
-  }
-  return make_float2(A / (float)samples, B / (float)samples);
-}
-
-// Every texel of every job in one grid-stride launch; jobs are laid out back to back, so a
-// wave almost always works on a single map and kind.
 // ----------------------------------------------- GL viewer bakes on equirect maps
 // envmap_bake.frag:10-24 with the capture views of RenderPipeline.cpp:14-26, and
 // irradiance_baker.frag:15-39. Lookup rule: the equirect texture's GL sampler state (the
@@ -254,33 +144,28 @@ __device__ __forceinline__ float2 brdf_lut_texel(const BakeMap &m, unsigned i, u
 // REPEAT wrap), level 0 with GL_LINEAR filtering: texel centres at (i + 0.5) / w, bilinear
 // weights, indices modulo the map size. atan and acos in double, rounded once.
 __device__ __forceinline__ f3 gl_normalize(f3 v) {
-  const float inv = 1.f / sqrtf((v.x * v.x + v.y * v.y) + v.z * v.z);
+  const float inv = inv_sqrt_mid((v.x * v.x + v.y * v.y) + v.z * v.z);
   return mk3(v.x * inv, v.y * inv, v.z * inv);
 }
 
-__device__ __forceinline__ f3 gl_texel(const BakeMap &m, int x, int y) {
-  x %= m.w;
-  if (x < 0) x += m.w;
-  y %= m.h;
-  if (y < 0) y += m.h;
-  const float *p = m.env + ((size_t)y * m.w + x) * m.c;
-  if (m.c == 4) {
-    const float4 t = *reinterpret_cast<const float4 *>(p);
-    return mk3(t.x, t.y, t.z);
-  }
-  return mk3(p[0], p[1], p[2]);
+// A texel index into [0, n): at most one turn away, since a direction's coordinates lie within one
+// texel of the map. A NaN direction's index is 0.
+__device__ __forceinline__ unsigned gl_wrap(int x, int n) {
+  const int y = x < 0 ? x + n : x >= n ? x - n : x;
+  return min((unsigned)y, (unsigned)n - 1u);
 }
 
 // texture(environment_map, sphericalToUv(d)) for a unit direction d
 __device__ __forceinline__ f3 gl_lookup(const BakeMap &m, f3 d) {
   const float PI = 3.14159265359f;
-  const float theta = (float)atan2(-(double)d.z, (double)d.x), phi = (float)acos((double)d.y);
-  const float u = theta / (2.0f * PI), v = phi / PI;
+  const float theta = (float)atan2_moderate(-(double)d.z, (double)d.x), phi = (float)acos_moderate(d.y);
+  const float u = div_mid(theta, 2.0f * PI), v = div_mid(phi, PI);
   const float x = u * (float)m.w - 0.5f, y = v * (float)m.h - 0.5f;
   const float fx = floorf(x), fy = floorf(y);
   const float a = x - fx, b = y - fy;
   const int i0 = (int)fx, j0 = (int)fy;
-  const f3 t00 = gl_texel(m, i0, j0), t10 = gl_texel(m, i0 + 1, j0), t01 = gl_texel(m, i0, j0 + 1), t11 = gl_texel(m, i0 + 1, j0 + 1);
+  const unsigned x0 = gl_wrap(i0, m.w), x1 = gl_wrap(i0 + 1, m.w), y0 = gl_wrap(j0, m.h), y1 = gl_wrap(j0 + 1, m.h);
+  const f3 t00 = load_texel(m, x0, y0), t10 = load_texel(m, x1, y0), t01 = load_texel(m, x0, y1), t11 = load_texel(m, x1, y1);
   const float w00 = (1.f - a) * (1.f - b), w10 = a * (1.f - b), w01 = (1.f - a) * b, w11 = a * b;
   return ((w00 * t00 + w10 * t10) + w01 * t01) + w11 * t11;
 }
@@ -310,45 +195,256 @@ __device__ __forceinline__ f3 equirect_texel_direction(int i, int j, int w, int 
   return mk3((float)(cos(az) * sin(po)), (float)cos(po), (float)(-sin(az) * sin(po)));
 }
 
+// The sampled bakes. A group of 2x2 output texels belongs to one workgroup of kBakeWaves waves, a
+// lane takes every (64 kBakeWaves)-th sample of all four. What bounds it is texel gathers:
+// neighbouring samples of a narrow lobe, and neighbouring texels' lobes, meet the same lines of
+// the map, and with a workgroup per 2x2 texels the few texels that an XCD works on at one time
+// stay within a part of the map that its L2 holds. One texel per lane, its samples in a loop, had
+// a whole mip in flight at once (each sample a line from beyond L2) and, with 12,960 texels per
+// map, 1.6 waves per SIMD. The samples' azimuth and elevation are computed once for the four
+// texels. The sums over lanes follow a fixed tree, whatever else is in the call. 8 maps (4096x2048
+// to 1024x512, 1,024 samples, 64x32 irradiance and 5 mips from 128x64): 3.0 -> 1.21 ms; with 2
+// waves per group 1.34, with 8 1.28, with 16 1.80.
+//
+// Groups are numbered in blocks of 8x4 groups (kGroupRun, 16x8 texels) row by row.
+constexpr unsigned kBakeWaves = 4;
+constexpr unsigned kBakeThreads = 64 * kBakeWaves;
+constexpr unsigned kGroupRun = 32;
 constexpr unsigned kBakeBlock = 256;
-// Workgroups go to the MI355X's 8 XCDs (each with its own L2) round robin. Workgroup b works
-// on texel block (b % 8) * (grid / 8) + b / 8 instead of b, so each XCD's L2 sees a
-// contiguous run of texels -- one or two maps at a time -- rather than every eighth block
-// of all of them. The grid is a multiple of 8, so this is a permutation of the blocks.
+// Workgroups go to the MI355X's 8 XCDs (each with its own L2) round robin. Of every 8 kGroupRun
+// workgroups, those of XCD x (x, x + 8, ..) take the x-th block of kGroupRun groups: an XCD's L2
+// sees neighbouring texels, and jobs of unlike cost spread over all XCDs.
 constexpr unsigned kXcds = 8;
-__global__ __launch_bounds__(kBakeBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) void bake_kernel(const BakeMap *__restrict__ maps, int count, uint64_t total, const float *__restrict__ lut,
-                            const uint32_t *__restrict__ sobol, int samples) {
-  const uint64_t block = (uint64_t)(blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
-  for (uint64_t g = block * blockDim.x + threadIdx.x; g < total; g += (uint64_t)gridDim.x * blockDim.x) {
+
+struct TexelFrame {
+  f3 n, t, b;
+};
+
+__device__ __forceinline__ float from_lane(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+// Lane `lane`'s frame, in scalar registers.
+__device__ __forceinline__ TexelFrame frame_of(const TexelFrame &f, int lane) {
+  return {mk3(from_lane(f.n.x, lane), from_lane(f.n.y, lane), from_lane(f.n.z, lane)),
+          mk3(from_lane(f.t.x, lane), from_lane(f.t.y, lane), from_lane(f.t.z, lane)),
+          mk3(from_lane(f.b.x, lane), from_lane(f.b.y, lane), from_lane(f.b.z, lane))};
+}
+
+// Sums of v[0..16) over the wave, the sum of v[k] in lanes 4k .. 4k+3: each step exchanges half
+// of what is left with the lane across one bit, 17 exchanges where a tree for each value has 96.
+__device__ __forceinline__ float wave_sums_16(float (&v)[16]) {
+  const unsigned lane = __lane_id();
+#pragma unroll
+  for (int half = 8; half >= 1; half >>= 1) {
+    const bool up = (lane & (4u * half)) != 0;
+#pragma unroll
+    for (int k = 0; k < half; k++) {
+      const float send = up ? v[k] : v[k + half], keep = up ? v[k + half] : v[k];
+      v[k] = keep + __shfl_xor(send, 4 * half, 64);
+    }
+  }
+  float r = v[0];
+  r += __shfl_xor(r, 2, 64);
+  r += __shfl_xor(r, 1, 64);
+  return r;
+}
+
+// The four texels of a group: the group's corner plus (q & 1, q >> 1); texels outside the output
+// repeat the corner and are not written.
+__global__ __launch_bounds__(kBakeThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void bake_kernel(const BakeMap *__restrict__ maps, int count,
+                                                                                                       uint64_t total, const float *__restrict__ lut,
+                                                                                                       const uint32_t *__restrict__ sobol, int samples) {
+  __shared__ uint32_t sob_tab[2 * 128];
+  __shared__ float red[2][kBakeWaves][16];
+  sobol_nibble_fill(sobol, 0, 2, sob_tab, threadIdx.x, blockDim.x);
+  __syncthreads();
+  const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t rounds = (total + gridDim.x - 1) / gridDim.x;  // the grid is a multiple of kXcds kGroupRun
+  unsigned done = 0;
+  for (uint64_t it = 0; it < rounds; it++) {
+    const uint64_t w = it * gridDim.x + blockIdx.x, span = w / (kXcds * kGroupRun);
+    const unsigned r = (unsigned)(w % (kXcds * kGroupRun));
+    const uint64_t g = (span * kXcds + r % kXcds) * kGroupRun + r / kXcds;
+    if (g >= total) continue;  // the same in the whole workgroup
     const BakeMap m = maps[find_map(maps, count, g)];
     const uint64_t local = g - m.first;
-    const unsigned i = (unsigned)(local % (unsigned)m.ow), j = (unsigned)(local / (unsigned)m.ow);
-    if (m.kind == NOVA_HIP_BAKE_BRDF_LUT) {
-      const float2 ab = brdf_lut_texel(m, i, j, samples);
-      float *o = m.out + ((size_t)j * m.ow + i) * 2;
-      o[0] = ab.x;
-      o[1] = ab.y;
-      continue;
+    const unsigned in_block = (unsigned)(local % kGroupRun);
+    const uint64_t block = local / kGroupRun;
+    const unsigned x0 = ((unsigned)(block % m.block_row) * 8u + in_block % 8u) * 2u, y0 = ((unsigned)(block / m.block_row) * 4u + in_block / 8u) * 2u;
+    if (x0 >= (unsigned)m.ow || y0 >= (unsigned)m.oh) continue;
+    // lane q (mod 4) prepares texel q
+    const unsigned i = x0 + (lane & 1u) < (unsigned)m.ow ? x0 + (lane & 1u) : x0;
+    const unsigned j = y0 + ((lane >> 1) & 1u) < (unsigned)m.oh ? y0 + ((lane >> 1) & 1u) : y0;
+    float acc[16];  // texel q: colour and weight at 4q .. 4q+3
+#pragma unroll
+    for (int k = 0; k < 16; k++) acc[k] = 0.f;
+    const float u = (float)((double)i / (double)m.ow), v = (float)((double)j / (double)m.oh);
+    TexelFrame mine;
+    mine.n = sph_to_cart((float)(2 * 3.14159265358979323846 * u), (float)(3.14159265358979323846 * v));
+    if (m.kind == NOVA_HIP_BAKE_PREFILTER) {
+      // N = V = R, Hammersley GGX half vectors, NdotL weights
+      mine.n = normalize(mine.n);
+      const f3 up = fabsf(mine.n.z) < 0.999f ? mk3(0.f, 0.f, 1.f) : mk3(1.f, 0.f, 0.f);
+      mine.t = normalize(cross(up, mine.n));
+      mine.b = cross(mine.n, mine.t);
+      const TexelFrame f[4] = {frame_of(mine, 0), frame_of(mine, 1), frame_of(mine, 2), frame_of(mine, 3)};
+      const float a = m.roughness * m.roughness;
+      for (unsigned s = threadIdx.x; s < (unsigned)samples; s += kBakeThreads) {
+        const float xi0 = (float)s / (float)samples, xi1 = radical_inverse(s);
+        const float ct = sqrtf((1.0f - xi1) / (1.0f + (a * a - 1.0f) * xi1));
+        const float st = sqrtf(1.0f - ct * ct);
+        float sp, cp;
+        sincos_2pi(xi0, sp, cp);
+        const float hx = cp * st, hy = sp * st;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const f3 H = normalize_mid(f[q].t * hx + f[q].b * hy + f[q].n * ct);
+          const f3 L = reflect(-f[q].n, H);
+          const float ndl = fmaxf(dot(f[q].n, L), 0.f);
+          if (ndl > 0.f) {
+            const f3 c = dir_sample(m, lut, L) * ndl;
+            acc[4 * q] += c.x;
+            acc[4 * q + 1] += c.y;
+            acc[4 * q + 2] += c.z;
+            acc[4 * q + 3] += ndl;
+          }
+        }
+      }
+    } else {
+      // The reference draws its cosine samples from pgc3d of the texel's recomputed pixel and
+      // the sample number; the Sobol variant takes Owen-scrambled Sobol points (dims 0 and 1)
+      // at indices texel * samples + s, so each texel gets its own stratified block of the
+      // sequence.
+      const bool is_sobol = m.kind == NOVA_HIP_BAKE_IRRADIANCE_SOBOL;
+      const float aphi = atan2_approx(mine.n.y, mine.n.x), atheta = acos_lt(lut, mine.n.z);
+      const double inv_2pi = 1.f / (2.f * 3.14159265358979323846), inv_pi = 1.f / 3.14159265358979323846;
+      const unsigned px_l = uv_to_pixel((float)(aphi * inv_2pi), (unsigned)m.ow), py_l = uv_to_pixel((float)(atheta * inv_pi), (unsigned)m.oh);
+      const f3 right = mk3(1.f, 0.f, 0.f);
+      const float dd = dot(right, mine.n);
+      mine.t = mk3(0.f, 1.f, 0.f);
+      if (1.0 - fabs((double)dd) > 1e-6) mine.t = normalize(cross(right, mine.n));
+      mine.b = cross(mine.n, mine.t);
+      const TexelFrame f[4] = {frame_of(mine, 0), frame_of(mine, 1), frame_of(mine, 2), frame_of(mine, 3)};
+      const uint32_t base_l = (j * (uint32_t)m.ow + i) * (uint32_t)samples;
+      uint32_t px[4], py[4], base[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        px[q] = (uint32_t)__builtin_amdgcn_readlane((int)px_l, q);
+        py[q] = (uint32_t)__builtin_amdgcn_readlane((int)py_l, q);
+        base[q] = (uint32_t)__builtin_amdgcn_readlane((int)base_l, q);
+      }
+      for (unsigned s = threadIdx.x; s < (unsigned)samples; s += kBakeThreads) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          float rx, ry;
+          if (is_sobol) {
+            const uint32_t idx = base[q] + s, gray = idx ^ (idx >> 1);
+            rx = u32_to_unit(owen_scramble(sobol_nibble_xor(sob_tab, gray)));
+            ry = u32_to_unit(owen_scramble(sobol_nibble_xor(sob_tab + 128, gray)));
+          } else {
+            const f3 rnd = pgc3d(px[q], py[q], s);
+            rx = rnd.x;
+            ry = rnd.y;
+          }
+          // cosine sample at phi = 2 pi rx, theta = asin(sqrt(ry)) (TextureProcessing.h:270-276):
+          // sin(theta) = sqrt(ry), cos(theta) = sqrt(1 - ry)
+          float sp, cp;
+          sincos_2pi(rx, sp, cp);
+          const float st = sqrt_mid(ry), ct = sqrt_mid(1.f - ry);
+          const f3 c = (st * cp) * f[q].t + (st * sp) * f[q].b + ct * f[q].n;
+          const f3 e = dir_sample(m, lut, c);
+          acc[4 * q] += e.x;
+          acc[4 * q + 1] += e.y;
+          acc[4 * q + 2] += e.z;
+        }
+      }
     }
-    const f3 col = m.kind == NOVA_HIP_BAKE_PREFILTER ? prefilter_texel(m, lut, i, j, samples) : irradiance_texel(m, lut, sobol, i, j, samples);
-    float *o = m.out + ((size_t)j * m.ow + i) * m.c;
-    o[0] = col.x;
-    o[1] = col.y;
-    o[2] = col.z;
-    for (int k = 3; k < m.c; k++) o[k] = 0.f;
+    const float sum = wave_sums_16(acc);
+    float(*const part)[16] = red[done++ & 1];  // the next group's sums go to the other half: one barrier a group
+    if ((lane & 3u) == 0) part[wave][lane >> 2] = sum;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+      const unsigned q = threadIdx.x >> 2, ch = threadIdx.x & 3u;
+      float val = 0.f, weight = 0.f;
+      for (unsigned k = 0; k < kBakeWaves; k++) {
+        val += part[k][threadIdx.x];
+        weight += part[k][threadIdx.x | 3u];
+      }
+      const unsigned x = x0 + (q & 1u), y = y0 + (q >> 1);
+      if (x < (unsigned)m.ow && y < (unsigned)m.oh && ch < (unsigned)m.c) {
+        float *o = m.out + ((size_t)y * (unsigned)m.ow + x) * (unsigned)m.c;
+        o[ch] = ch == 3u ? 0.f : m.kind == NOVA_HIP_BAKE_PREFILTER ? val / weight : val / (float)samples;
+      }
+    }
   }
 }
 
-// The Riemann irradiance of irradiance_baker.frag, one workgroup per output texel: lane t
-// sums the zenith loop of azimuth steps t, t + 256, ... (the steps' cos and sin, stepped in
-// float as GLSL steps them, come from host tables), then the lanes' sums are added in a
-// fixed tree. The shader keeps one running sum; the sum here is regrouped by azimuth,
-// which moves the result by float rounding only.
+// BRDF tables: computeLut (brdf_lookup_table_baker.frag:74-113) at texel (i, j): NdotV =
+// (i + 0.5) / ow, roughness = (j + 0.5) / oh; the split-sum scale A and bias B over `samples`
+// Hammersley GGX half vectors. A wave takes 64 columns of one row, so its roughness and with it
+// every half vector are the same in all lanes: lane l computes the half vector of each 64
+// samples' l-th once and the wave reads it into scalar registers. The sums stay one by one in
+// sample order (a tree moves them by 1.5e-5 from the shader's). What bounds it is the one wave per
+// SIMD that 256x256 texels give; four samples' arithmetic is interleaved (256x256, 1,024 samples:
+// 565 -> 261 us).
+__global__ __launch_bounds__(64) void lut_kernel(const BakeMap *__restrict__ maps, int count, uint64_t total, int samples) {
+  const unsigned lane = threadIdx.x;
+  for (uint64_t g = blockIdx.x; g < total; g += gridDim.x) {
+    const BakeMap m = maps[find_map(maps, count, g)];
+    const uint64_t local = g - m.first;
+    const unsigned i = (unsigned)(local % m.block_row) * 64u + lane, j = (unsigned)(local / m.block_row);
+    const float ndotv = ((float)i + 0.5f) / (float)m.ow, roughness = ((float)j + 0.5f) / (float)m.oh;
+    // with N = +z and up = +x the tangent is -y and the bitangent +x
+    const f3 V = mk3(sqrtf(1.0f - ndotv * ndotv), 0.0f, ndotv);
+    const float a = roughness * roughness;
+    const float gv = schlick_ggx_ibl(fmaxf(ndotv, 0.0f), roughness);
+    float A = 0.f, B = 0.f;
+    for (int s0 = 0; s0 < samples; s0 += 64) {
+      const int s = s0 + (int)lane < samples ? s0 + (int)lane : samples - 1, n = min(64, samples - s0);
+      const float xi0 = (float)s / (float)samples, xi1 = radical_inverse((unsigned)s);
+      const float ct = sqrtf((1.0f - xi1) / (1.0f + (a * a - 1.0f) * xi1));
+      const float st = sqrtf(1.0f - ct * ct);
+      float sp, cp;
+      sincos_2pi(xi0, sp, cp);
+      const f3 half = normalize(mk3(sp * st, -(cp * st), ct));
+      for (int k0 = 0; k0 < n; k0 += 4)  // four samples' arithmetic side by side
+#pragma unroll
+      for (int k = k0; k < k0 + 4; k++) {
+        const f3 H = mk3(from_lane(half.x, k), from_lane(half.y, k), from_lane(half.z, k));
+        const f3 L = normalize_mid(H * (2.0f * dot(V, H)) - V);
+        const float ndl = fmaxf(L.z, 0.0f), ndh = fmaxf(H.z, 0.0f), vdh = fmaxf(dot(V, H), 0.0f);
+        const float G = schlick_ggx_ibl(ndl, roughness) * gv;
+        const float g_vis = div_mid(G * vdh, ndh * ndotv);
+        const float fc = pow5(1.0f - vdh);
+        const bool counts = (ndl > 0.0f) & (k < n);
+        A = counts ? A + (1.0f - fc) * g_vis : A;
+        B = counts ? B + fc * g_vis : B;
+      }
+    }
+    if (i < (unsigned)m.ow) {
+      float *o = m.out + ((size_t)j * (unsigned)m.ow + i) * 2;
+      o[0] = A / (float)samples;
+      o[1] = B / (float)samples;
+    }
+  }
+}
+
+// The Riemann irradiance of irradiance_baker.frag, kRiemannParts workgroups per output texel,
+// each with a run of the azimuth steps (the steps' cos and sin, stepped in float as GLSL steps
+// them, come from host tables): the lanes' sums are added in a fixed tree and riemann_finish adds
+// the parts'. The shader keeps one running sum; the regrouping moves the result by float rounding
+// only. A texel reads half the map, so what counts beside the two angles in double
+// (device_trig.h) is that lanes meet the same lines: a wave takes 8x8 patches of (azimuth,
+// zenith) steps and its workgroup 16x16 ones, and 4 waves per SIMD thrash L1 less than 8. 512
+// texels of a 3-channel 2048x1024 map: 1.38 ms with a lane per azimuth step, 1.93 with lanes along
+// the zenith, 1.01 with patches at 8 waves per SIMD, 0.89 at 4.
 constexpr unsigned kRiemannBlock = 256;
-__global__ __launch_bounds__(kRiemannBlock) void riemann_kernel(const BakeMap *__restrict__ maps, int count, const float2 *__restrict__ phi_tab,
-                                                               int nphi, const float2 *__restrict__ theta_tab, int ntheta) {
-  __shared__ float red[3][kRiemannBlock];
+constexpr unsigned kRiemannParts = 8;
+__global__ __launch_bounds__(kRiemannBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) void riemann_kernel(const BakeMap *__restrict__ maps, int count, const float2 *__restrict__ phi_tab,
+                                                               int nphi, const float2 *__restrict__ theta_tab, int ntheta, float *__restrict__ parts) {
+  __shared__ float red[3][kRiemannBlock / 64];
   const uint64_t g = blockIdx.x;
+  const unsigned part = blockIdx.y;
   const BakeMap m = maps[find_map(maps, count, g)];
   const uint64_t local = g - m.first;
   const int i = (int)(local % (unsigned)m.ow), j = (int)(local / (unsigned)m.ow);
@@ -356,29 +452,48 @@ __global__ __launch_bounds__(kRiemannBlock) void riemann_kernel(const BakeMap *_
   const f3 right = gl_normalize(cross(mk3(0.f, 1.f, 0.f), n));
   const f3 up = gl_normalize(cross(n, right));
   f3 acc = mk3(0.f, 0.f, 0.f);
-  for (int k = threadIdx.x; k < nphi; k += kRiemannBlock) {
-    const float2 ph = phi_tab[k];
-    for (int t = 0; t < ntheta; t++) {
-      const float2 th = theta_tab[t];  // (cos, sin)
+  const int begin = (int)((uint64_t)nphi * part / kRiemannParts), end = (int)((uint64_t)nphi * (part + 1) / kRiemannParts);
+  const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int k1 = (int)((wave & 1u) * 8u + (lane & 7u)), t1 = (int)((wave >> 1) * 8u + (lane >> 3));
+  for (int k0 = begin; k0 < end; k0 += 16)
+    for (int t0 = 0; t0 < ntheta; t0 += 16) {
+      const int k = k0 + k1, t = t0 + t1;
+      if (k >= end || t >= ntheta) continue;
+      const float2 ph = phi_tab[k], th = theta_tab[t];  // (cos, sin)
       const float x = ph.x * th.y, y = th.y * ph.y, z = th.x;
       const f3 sv = (x * right + y * up) + z * n;
       acc = acc + (gl_lookup(m, gl_normalize(sv)) * th.x) * th.y;
     }
+  for (int w = 32; w > 0; w >>= 1) {
+    acc.x += __shfl_down(acc.x, w, 64);
+    acc.y += __shfl_down(acc.y, w, 64);
+    acc.z += __shfl_down(acc.z, w, 64);
   }
-  red[0][threadIdx.x] = acc.x;
-  red[1][threadIdx.x] = acc.y;
-  red[2][threadIdx.x] = acc.z;
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = acc.x;
+    red[1][threadIdx.x >> 6] = acc.y;
+    red[2][threadIdx.x >> 6] = acc.z;
+  }
   __syncthreads();
-  for (unsigned w = kRiemannBlock / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w)
-      for (int c = 0; c < 3; c++) red[c][threadIdx.x] += red[c][threadIdx.x + w];
-    __syncthreads();
+  if (threadIdx.x < 3) {
+    float sum = red[threadIdx.x][0];
+    for (unsigned w = 1; w < kRiemannBlock / 64; w++) sum += red[threadIdx.x][w];
+    parts[(g * kRiemannParts + part) * 3 + threadIdx.x] = sum;
   }
-  if (threadIdx.x == 0) {
+}
+
+__global__ __launch_bounds__(256) void riemann_finish(const BakeMap *__restrict__ maps, int count, uint64_t total, const float *__restrict__ parts,
+                                                      int steps) {
+  for (uint64_t g = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; g < total; g += (uint64_t)gridDim.x * blockDim.x) {
+    const BakeMap m = maps[find_map(maps, count, g)];
     const float PI = 3.14159265358f;
-    const float inv = 1.f / (float)(nphi * ntheta);
-    float *o = m.out + ((size_t)j * m.ow + i) * m.c;
-    for (int c = 0; c < 3; c++) o[c] = (PI * red[c][0]) * inv;
+    const float inv = 1.f / (float)steps;
+    float *o = m.out + (g - m.first) * (unsigned)m.c;
+    for (int c = 0; c < 3; c++) {
+      float sum = 0.f;
+      for (unsigned k = 0; k < kRiemannParts; k++) sum += parts[(g * kRiemannParts + k) * 3 + c];
+      o[c] = (PI * sum) * inv;
+    }
     for (int c = 3; c < m.c; c++) o[c] = 0.f;
   }
 }
@@ -390,15 +505,21 @@ static void riemann_steps(float bound, std::vector<float2> &tab) {
   for (float a = 0.f; a <= bound; a += 0.0075f) tab.push_back(make_float2((float)std::cos((double)a), (float)std::sin((double)a)));
 }
 
-// Cube-map captures, one texel per lane: six faces of ow x ow, face-major, rows bottom-up.
-// A kernel of its own: its double-precision atan and acos would raise the register budget of
-// the sampled bakes.
-__global__ __launch_bounds__(kBakeBlock) void cubemap_kernel(const BakeMap *__restrict__ maps, int count, uint64_t total) {
+// Outputs of one lookup per texel, one texel per lane: cube-map captures (six faces of ow x ow,
+// face-major, rows bottom-up) and prefilter levels of roughness 0.
+__global__ __launch_bounds__(kBakeBlock) void lookup_kernel(const BakeMap *__restrict__ maps, int count, uint64_t total, const float *__restrict__ lut) {
   for (uint64_t g = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; g < total; g += (uint64_t)gridDim.x * blockDim.x) {
     const BakeMap m = maps[find_map(maps, count, g)];
     const uint64_t local = g - m.first;
-    const unsigned S = (unsigned)m.ow, face = (unsigned)(local / ((uint64_t)S * S)), r = (unsigned)(local % ((uint64_t)S * S));
-    const f3 col = gl_lookup(m, cube_texel_direction((int)face, (int)(r % S), (int)(r / S), (int)S));
+    f3 col;
+    if (m.kind == NOVA_HIP_BAKE_CUBEMAP) {
+      const unsigned S = (unsigned)m.ow, face = (unsigned)(local / ((uint64_t)S * S)), r = (unsigned)(local % ((uint64_t)S * S));
+      col = gl_lookup(m, cube_texel_direction((int)face, (int)(r % S), (int)(r / S), (int)S));
+    } else {
+      const unsigned i = (unsigned)(local % (unsigned)m.ow), j = (unsigned)(local / (unsigned)m.ow);
+      const float u = (float)((double)i / (double)m.ow), v = (float)((double)j / (double)m.oh);
+      col = dir_sample(m, lut, normalize(sph_to_cart((float)(2 * 3.14159265358979323846 * u), (float)(3.14159265358979323846 * v))));
+    }
     float *o = m.out + local * m.c;
     o[0] = col.x;
     o[1] = col.y;
@@ -410,8 +531,9 @@ __global__ __launch_bounds__(kBakeBlock) void cubemap_kernel(const BakeMap *__re
 static int launch_batch(const nova_hip_bake_job *jobs, uint32_t count, int32_t samples, hipStream_t s) {
   if (count == 0) return NOVA_HIP_SUCCESS;
   if (!jobs || samples <= 0) return NOVA_HIP_INVALID_ARGUMENT;
-  std::vector<BakeMap> maps, cube, riemann;  // sampled bakes; cube captures; Riemann jobs (a workgroup per texel)
-  uint64_t total = 0, cube_total = 0, riemann_total = 0;
+  // sampled bakes (in groups of texels); one lookup per texel; BRDF tables (in waves); Riemann jobs (kRiemannParts workgroups per texel)
+  std::vector<BakeMap> maps, direct, luts, riemann;
+  uint64_t total = 0, direct_total = 0, lut_total = 0, riemann_total = 0;
   for (uint32_t i = 0; i < count; i++) {
     const nova_hip_bake_job &jb = jobs[i];
     if (jb.kind == NOVA_HIP_BAKE_BRDF_LUT) {  // no environment map; two output channels
@@ -429,13 +551,18 @@ static int launch_batch(const nova_hip_bake_job *jobs, uint32_t count, int32_t s
     if (jb.kind == NOVA_HIP_BAKE_IRRADIANCE_SOBOL && (uint64_t)jb.out_width * jb.out_height * (uint64_t)samples > 0xFFFFFFFFull)
       return NOVA_HIP_INVALID_ARGUMENT;
     const uint64_t texels = (uint64_t)jb.out_width * jb.out_height * (jb.kind == NOVA_HIP_BAKE_CUBEMAP ? 6u : 1u);
-    const bool is_cube = jb.kind == NOVA_HIP_BAKE_CUBEMAP, is_riemann = jb.kind == NOVA_HIP_BAKE_IRRADIANCE_RIEMANN;
-    uint64_t &first = is_riemann ? riemann_total : is_cube ? cube_total : total;
-    (is_riemann ? riemann : is_cube ? cube : maps)
-        .push_back(BakeMap{jb.env, jb.out, jb.width, jb.height, jb.channels, jb.out_width, jb.out_height, jb.kind, jb.roughness, first});
-    first += texels;
+    const bool is_riemann = jb.kind == NOVA_HIP_BAKE_IRRADIANCE_RIEMANN;
+    const bool is_direct = jb.kind == NOVA_HIP_BAKE_CUBEMAP || (jb.kind == NOVA_HIP_BAKE_PREFILTER && jb.roughness == 0.f);
+    const bool is_lut = jb.kind == NOVA_HIP_BAKE_BRDF_LUT;
+    const uint32_t block_row = is_lut ? ((uint32_t)jb.out_width + 63) / 64 : ((uint32_t)jb.out_width + 15) / 16;
+    uint64_t &first = is_riemann ? riemann_total : is_direct ? direct_total : is_lut ? lut_total : total;
+    (is_riemann ? riemann : is_direct ? direct : is_lut ? luts : maps)
+        .push_back(BakeMap{jb.env, jb.out, jb.width, jb.height, jb.channels, jb.out_width, jb.out_height, jb.kind, jb.roughness, first, block_row});
+    first += is_riemann || is_direct ? texels
+             : is_lut                ? (uint64_t)block_row * (uint32_t)jb.out_height
+                                     : (uint64_t)block_row * (((uint32_t)jb.out_height + 7) / 8) * kGroupRun;
   }
-  if (riemann_total > 0x7FFFFFFFull) return NOVA_HIP_INVALID_ARGUMENT;  // one workgroup per texel
+  if (riemann_total > 0x7FFFFFFFull) return NOVA_HIP_INVALID_ARGUMENT;  // a column of workgroups per texel
   const uint32_t *sobol = device_sobol_table();
   if (!sobol) return NOVA_HIP_OUT_OF_MEMORY;
   // acos table: one device copy per process and device
@@ -457,33 +584,39 @@ static int launch_batch(const nova_hip_bake_job *jobs, uint32_t count, int32_t s
     riemann_steps(azimuth_max, phi_tab);
     riemann_steps(zenith_max, theta_tab);
   }
-  const size_t maps_bytes = maps.size() * sizeof(BakeMap), cube_bytes = cube.size() * sizeof(BakeMap), riemann_bytes = riemann.size() * sizeof(BakeMap);
-  const size_t tab_bytes = (phi_tab.size() + theta_tab.size()) * sizeof(float2);
+  const size_t tab_bytes = (phi_tab.size() + theta_tab.size()) * sizeof(float2), parts_bytes = riemann_total * kRiemannParts * 3 * sizeof(float);
+  const size_t n_maps = maps.size(), n_direct = direct.size(), n_luts = luts.size(), n_riemann = riemann.size();
+  for (const std::vector<BakeMap> *v : {&direct, &luts, &riemann}) maps.insert(maps.end(), v->begin(), v->end());
+  const size_t maps_bytes = maps.size() * sizeof(BakeMap);
   char *buf = nullptr;
-  if (hipMalloc(&buf, maps_bytes + cube_bytes + riemann_bytes + tab_bytes + 16) != hipSuccess) return NOVA_HIP_OUT_OF_MEMORY;
-  BakeMap *d_maps = reinterpret_cast<BakeMap *>(buf), *d_cube = reinterpret_cast<BakeMap *>(buf + maps_bytes);
-  BakeMap *d_riemann = reinterpret_cast<BakeMap *>(buf + maps_bytes + cube_bytes);
-  float2 *d_phi = reinterpret_cast<float2 *>(buf + maps_bytes + cube_bytes + riemann_bytes), *d_theta = d_phi + phi_tab.size();
-  hipError_t e = hipSuccess;
-  if (maps_bytes) e = hipMemcpyAsync(d_maps, maps.data(), maps_bytes, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess && cube_bytes) e = hipMemcpyAsync(d_cube, cube.data(), cube_bytes, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess && riemann_bytes) e = hipMemcpyAsync(d_riemann, riemann.data(), riemann_bytes, hipMemcpyHostToDevice, s);
+  if (hipMalloc(&buf, maps_bytes + tab_bytes + parts_bytes + 16) != hipSuccess) return NOVA_HIP_OUT_OF_MEMORY;
+  BakeMap *d_maps = reinterpret_cast<BakeMap *>(buf), *d_direct = d_maps + n_maps, *d_luts = d_direct + n_direct, *d_riemann = d_luts + n_luts;
+  float2 *d_phi = reinterpret_cast<float2 *>(buf + maps_bytes), *d_theta = d_phi + phi_tab.size();
+  float *d_parts = reinterpret_cast<float *>(d_theta + theta_tab.size());
+  hipError_t e = hipMemcpyAsync(d_maps, maps.data(), maps_bytes, hipMemcpyHostToDevice, s);
   if (e == hipSuccess && !phi_tab.empty()) e = hipMemcpyAsync(d_phi, phi_tab.data(), phi_tab.size() * sizeof(float2), hipMemcpyHostToDevice, s);
   if (e == hipSuccess && !theta_tab.empty()) e = hipMemcpyAsync(d_theta, theta_tab.data(), theta_tab.size() * sizeof(float2), hipMemcpyHostToDevice, s);
   if (e == hipSuccess && total > 0) {
-    const unsigned block = kBakeBlock;
-    const unsigned grid = (unsigned)std::min<uint64_t>(((total + block - 1) / block + kXcds - 1) / kXcds * kXcds, 1u << 20);  // a multiple of kXcds
-    hipLaunchKernelGGL(bake_kernel, dim3(grid), dim3(block), 0, s, d_maps, (int)maps.size(), total, d_lut, sobol, samples);
+    // a multiple of the workgroups that share a run of blocks over the XCDs
+    constexpr uint64_t kSpan = kXcds * kGroupRun;
+    const unsigned grid = (unsigned)std::min<uint64_t>((total + kSpan - 1) / kSpan * kSpan, 1u << 20);
+    hipLaunchKernelGGL(bake_kernel, dim3(grid), dim3(kBakeThreads), 0, s, d_maps, (int)n_maps, total, d_lut, sobol, samples);
     e = hipGetLastError();
   }
-  if (e == hipSuccess && cube_total > 0) {
-    const unsigned grid = (unsigned)std::min<uint64_t>((cube_total + kBakeBlock - 1) / kBakeBlock, 1u << 20);
-    hipLaunchKernelGGL(cubemap_kernel, dim3(grid), dim3(kBakeBlock), 0, s, d_cube, (int)cube.size(), cube_total);
+  if (e == hipSuccess && direct_total > 0) {
+    const unsigned grid = (unsigned)std::min<uint64_t>((direct_total + kBakeBlock - 1) / kBakeBlock, 1u << 20);
+    hipLaunchKernelGGL(lookup_kernel, dim3(grid), dim3(kBakeBlock), 0, s, d_direct, (int)n_direct, direct_total, d_lut);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess && lut_total > 0) {
+    hipLaunchKernelGGL(lut_kernel, dim3((unsigned)std::min<uint64_t>(lut_total, 1u << 20)), dim3(64), 0, s, d_luts, (int)n_luts, lut_total, samples);
     e = hipGetLastError();
   }
   if (e == hipSuccess && riemann_total > 0) {
-    hipLaunchKernelGGL(riemann_kernel, dim3((unsigned)riemann_total), dim3(kRiemannBlock), 0, s, d_riemann, (int)riemann.size(), d_phi,
-                       (int)phi_tab.size(), d_theta, (int)theta_tab.size());
+    hipLaunchKernelGGL(riemann_kernel, dim3((unsigned)riemann_total, kRiemannParts), dim3(kRiemannBlock), 0, s, d_riemann, (int)n_riemann, d_phi,
+                       (int)phi_tab.size(), d_theta, (int)theta_tab.size(), d_parts);
+    hipLaunchKernelGGL(riemann_finish, dim3((unsigned)std::min<uint64_t>((riemann_total + 255) / 256, 4096)), dim3(256), 0, s, d_riemann,
+                       (int)n_riemann, riemann_total, d_parts, (int)(phi_tab.size() * theta_tab.size()));
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(s);

@@ -1,0 +1,126 @@
+// Arithmetic at the precision the render and bake paths ask for in fewer instructions than the
+// general operators and library functions: correctly rounded float square roots and quotients
+// inside the exponent range; sine, cosine, arc tangent and arc cosine in double for arguments
+// that are floats and results that are rounded to float once.
+#pragma once
+#include "device_math.h"
+
+namespace nova_hip {
+
+// Square roots, reciprocals and quotients of numbers well inside the exponent range (2^-60 to 2^60
+// by magnitude, or 0 under a root and over a fraction), bit for bit those of the IEEE operators,
+// which also scale and fix up denormal and extreme operands: 1 / sqrt(x) in 8 instructions where
+// the operators' expansion has about 35. Square roots from v_rsq_f32 and reciprocals from
+// v_rcp_f32 with one fused correction each are exact for every mantissa of both exponent
+// parities; quotients then by Markstein's theorem (a zero's sign is not kept). The caller knows
+// the range: a test here would cost what is saved, in instructions and in scheduling.
+#ifdef __HIP_DEVICE_COMPILE__
+__device__ __forceinline__ float rcp_mid(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.f), r, r);
+}
+__device__ __forceinline__ float sqrt_mid(float x) {
+  const float r = __builtin_amdgcn_rsqf(fmaxf(x, 1e-30f)), s = x * r;
+  return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * r, s);
+}
+__device__ __forceinline__ float inv_sqrt_mid(float x) {
+  const float r = __builtin_amdgcn_rsqf(x), s = x * r;
+  return rcp_mid(__builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * r, s));
+}
+__device__ __forceinline__ float div_mid(float n, float d) {
+  const float r = rcp_mid(d), q = n * r;
+  return __builtin_fmaf(__builtin_fmaf(-d, q, n), r, q);
+}
+#else
+NOVA_HD float sqrt_mid(float x) { return sqrtf(x); }
+NOVA_HD float inv_sqrt_mid(float x) { return 1.f / sqrtf(x); }
+NOVA_HD float div_mid(float n, float d) { return n / d; }
+#endif
+// normalize() of a vector of moderate length
+NOVA_HD f3 normalize_mid(f3 v) { return v * inv_sqrt_mid(dot(v, v)); }
+
+// sin and cos of a float of at most a few turns, each computed in double and rounded once. One
+// reduction by pi/2 (two fused steps) and both Taylor sums; the general library functions reduce
+// each for arguments of any size, in about 250 instructions for the pair against 45 here. The
+// error before the rounding is below 3e-16, so a result differs from the correctly rounded one
+// for about one argument in 10^8.
+__host__ __device__ __forceinline__ void sincos_turns(float xf, float &s_out, float &c_out) {
+  const double x = (double)xf;
+  const double n = rint(x * 0.6366197723675814);
+  double r = fma(n, -1.5707963267948966, x);
+  r = fma(n, -6.123233995736766e-17, r);
+  const double z = r * r;
+  // 1/3!, 1/5!, .. and 1/2!, 1/4!, ..: |r| <= pi/4, the first terms left out are below 5e-17
+  double s = fma(z, -1.0 / 1307674368000.0, 1.0 / 6227020800.0);
+  s = fma(z, s, -1.0 / 39916800.0);
+  s = fma(z, s, 1.0 / 362880.0);
+  s = fma(z, s, -1.0 / 5040.0);
+  s = fma(z, s, 1.0 / 120.0);
+  s = fma(z, s, -1.0 / 6.0);
+  s = fma(r * z, s, r);
+  double c = fma(z, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
+  c = fma(z, c, 1.0 / 479001600.0);
+  c = fma(z, c, -1.0 / 3628800.0);
+  c = fma(z, c, 1.0 / 40320.0);
+  c = fma(z, c, -1.0 / 720.0);
+  c = fma(z, c, 1.0 / 24.0);
+  c = fma(z, c, -0.5);
+  c = fma(z, c, 1.0);
+  const float sf = (float)s, cf = (float)c;
+  const int q = (int)n;
+  const float a = (q & 1) ? cf : sf, b = (q & 1) ? sf : cf;
+  s_out = xf == 0.f ? xf : (q & 2) ? -a : a;
+  c_out = ((q + 1) & 2) ? -b : b;
+}
+
+// num / den in double to 5e-15 (v_rcp_f64 gives 5e-8), for a normal den of moderate size.
+__host__ __device__ __forceinline__ double quick_div(double num, double den) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const double r = __builtin_amdgcn_rcp(den);
+  return num * fma(fma(-den, r, 1.0), r, r);
+#else
+  return num / den;
+#endif
+}
+
+// atan2(y, x) for x and y of moderate size (zeros with their signs included). The smaller
+// over the larger magnitude, moved below tan(pi/8) by one subtraction of angles, then a
+// polynomial of atan through the Chebyshev nodes of [0, tan^2(pi/8)] (its error below 4e-15).
+// A NaN comes out as one.
+__host__ __device__ __forceinline__ double atan2_moderate(double y, double x) {
+  const double ax = fabs(x), ay = fabs(y);
+  const bool swap = ay > ax;
+  const double lo = swap ? ax : ay, hi = swap ? ay : ax;
+  const bool upper = lo > 0.4142135623730951 * hi;
+  const double t = quick_div(upper ? lo - hi : lo, upper ? lo + hi : hi == 0.0 ? 1.0 : hi);
+  const double z = t * t;
+  double p = fma(z, -0.02723288223178155, 0.051688348206153534);
+  p = fma(z, p, -0.0655090727849726);
+  p = fma(z, p, 0.0768104519901944);
+  p = fma(z, p, -0.09090255952436734);
+  p = fma(z, p, 0.11111089649202319);
+  p = fma(z, p, -0.14285713930378444);
+  p = fma(z, p, 0.19999999997724888);
+  p = fma(z, p, -0.3333333333333093);
+  double a = fma(t * z, p, t);
+  a = upper ? 0.7853981633974483 + a : a;
+  a = swap ? 1.5707963267948966 - a : a;
+  a = copysign(1.0, x) < 0.0 ? 3.141592653589793 - a : a;
+  return copysign(a, y);
+}
+
+// acos of a float; NaN outside [-1, 1].
+__host__ __device__ __forceinline__ double acos_moderate(float xf) {
+  const double x = (double)xf, s2 = (1.0 - x) * (1.0 + x);
+#ifdef __HIP_DEVICE_COMPILE__
+  // s2 is 0 or above 1e-8
+  const double r = __builtin_amdgcn_rsq(s2 == 0.0 ? 1.0 : s2);  // to 5e-8; NaN below 0
+  const double q = s2 * r;
+  const double s = fma(fma(-q, r, 1.0), 0.5 * q, q);
+#else
+  const double s = sqrt(s2);
+#endif
+  return atan2_moderate(s, x);
+}
+
+}  // namespace nova_hip
