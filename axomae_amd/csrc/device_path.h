@@ -295,9 +295,9 @@ NOVA_HD void sample_surface(const ShadeParams &sp, const ShadeCtx &sc, Sobol sob
     float4 t4 = sample_u32(sc, mat.normal, h.u, h.v);
     nrm = mk3(t4.x * ONE_255, t4.y * ONE_255, t4.z * ONE_255);
   }
-  const f3 ns = normalize(mul(h.frame, nrm * 2.f - 1.f));
+  const f3 ns = normalize_mid(mul(h.frame, nrm * 2.f - 1.f));
   out.ns = ns;
-  const f3 wo = normalize(-d);
+  const f3 wo = normalize_mid(-d);
   BsdfIn bi;
   bi.ns = ns;
   bi.ng = h.ng;
@@ -335,10 +335,10 @@ NOVA_HD void sample_surface(const ShadeParams &sp, const ShadeCtx &sc, Sobol sob
   Principled b;
   b.configure(bi);
   b.construct(uc);
-  float r_sampling = b.roughness;
-  if (sc.sampling_roughness >= 0 && mat.roughness_f32 >= 0) r_sampling = sample_f32_bilinear(sc, sc.sampling_roughness, h.u, h.v).x;
-  const VNDF ggx(b.anisotropy, r_sampling);  // samples and weights by its pdf
   const VNDF ggx_e(b.anisotropy, b.roughness);  // BSDF value
+  VNDF ggx = ggx_e;  // samples and weights by its pdf
+  const bool detached = sc.sampling_roughness >= 0 && mat.roughness_f32 >= 0;
+  if (detached) ggx = VNDF(b.anisotropy, sample_f32_bilinear(sc, sc.sampling_roughness, h.u, h.v).x);
   if ((b.flags(ggx) & (BX_GLOSSY | BX_REFLECTION)) && bi.wo_dot_ng >= 0) {
     // the corrected shading normal reconfigures the frame; the chosen lobe and its weights stay
     bi.ns = normalize(correct_specular_shading_normal(bi.ng, wo, bi.ns));
@@ -356,17 +356,21 @@ NOVA_HD void sample_surface(const ShadeParams &sp, const ShadeCtx &sc, Sobol sob
   out.dlna = mk3(0.f, 0.f, 0.f);
   out.dlnr = 0.f;
   if (b.lobe != LOBE_NONE) {
-    const f3 lwo = normalize(mul_t(b.frame, wo));
+    const f3 lwo = normalize_mid(mul_t(b.frame, wo));
     if ((b.flags(ggx) & (BX_REFLECTION | BX_TRANSMISSION)) && lwo.z != 0.f) {
-      if (b.lobe == LOBE_DIFFUSE)
-        ok = sample_disney(b, lwo, u0, u1, smp);
-      else if (b.lobe == LOBE_SPECULAR)
-        ok = sample_specular(b, ggx, ggx_e, lwo, u0, u1, smp);
-      else
-        ok = sample_dielectric(b, ggx, ggx_e, lwo, uc2, u0, u1, smp);
+      const bool diffuse = b.lobe == LOBE_DIFFUSE;
+      float r, ang, sn, cs;
+      if (diffuse) {
+        shirley_chiu(u0, u1, r, ang);
+      } else {
+        r = sqrt_mid(u0);
+        ang = (float)(2.0 * 3.14159265358979323846 * (double)u1);
+      }
+      sincos_turns(ang, sn, cs);
+      ok = diffuse ? sample_disney(b, lwo, r * cs, r * sn, smp) : sample_microfacet(b, ggx, ggx_e, !detached, lwo, uc2, r * cs, r * sn, smp);
       if (ok && ((smp.f.x == 0.f && smp.f.y == 0.f && smp.f.z == 0.f) || smp.pdf == 0.f || smp.wi.z == 0.f)) ok = false;
       if (kAdj && ok) bsdf_log_derivatives(b, ggx_e, lwo, smp, out.dlna, out.dlnr);
-      if (ok) smp.wi = normalize(mul(b.frame, smp.wi));
+      if (ok) smp.wi = normalize_mid(mul(b.frame, smp.wi));
     }
   }
   out.smp = smp;
@@ -451,7 +455,7 @@ NOVA_HD bool shade_path(const ShadeParams &sp, const ShadeCtx &sc, Sobol sobol, 
   T = T * c;
   // Ray::spawn (Ray.h:22-27)
   const f3 wi = smp.wi;
-  nd = normalize(wi);
+  nd = normalize_mid(wi);
   no = h.pos + h.ng * (1e-3f + 1e-3f * gsign(dot(h.ng, wi)));
   if (sp.last) {  // depth budget spent: V = envmap(direction) without traversal
     const float4 env = sample_envmap(sc, nd);
