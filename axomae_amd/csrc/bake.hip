@@ -12,6 +12,7 @@
 
 #include "device_math.h"
 #include "device_path.h"
+#include "device_queue.h"
 #include "device_trig.h"
 #include "nova_internal.h"
 
@@ -228,25 +229,6 @@ __device__ __forceinline__ TexelFrame frame_of(const TexelFrame &f, int lane) {
   return {mk3(from_lane(f.n.x, lane), from_lane(f.n.y, lane), from_lane(f.n.z, lane)),
           mk3(from_lane(f.t.x, lane), from_lane(f.t.y, lane), from_lane(f.t.z, lane)),
           mk3(from_lane(f.b.x, lane), from_lane(f.b.y, lane), from_lane(f.b.z, lane))};
-}
-
-// Sums of v[0..16) over the wave, the sum of v[k] in lanes 4k .. 4k+3: each step exchanges half
-// of what is left with the lane across one bit, 17 exchanges where a tree for each value has 96.
-__device__ __forceinline__ float wave_sums_16(float (&v)[16]) {
-  const unsigned lane = __lane_id();
-#pragma unroll
-  for (int half = 8; half >= 1; half >>= 1) {
-    const bool up = (lane & (4u * half)) != 0;
-#pragma unroll
-    for (int k = 0; k < half; k++) {
-      const float send = up ? v[k] : v[k + half], keep = up ? v[k + half] : v[k];
-      v[k] = keep + __shfl_xor(send, 4 * half, 64);
-    }
-  }
-  float r = v[0];
-  r += __shfl_xor(r, 2, 64);
-  r += __shfl_xor(r, 1, 64);
-  return r;
 }
 
 // The four texels of a group: the group's corner plus (q & 1, q >> 1); texels outside the output

@@ -205,40 +205,15 @@ struct AdjointCtx {
   float4 *hit_cache;
   uint32_t cache_paths;    // paths per bounce in the cache
   uint32_t cache_bounces;  // bounces 0 .. cache_bounces-1 are cached
-  // The replay kernel's LDS table (kGradSlots keys, 3 values each) that sums its workgroup's
-  // texel gradients before they go to device memory; null: straight to device memory.
-  uint32_t *table_keys = nullptr;
-  float *table_vals = nullptr;
-  uint16_t *table_list = nullptr;   // slots taken since the last flush, in claim order
-  uint32_t *table_count = nullptr;  // entries of table_list
 };
 
-// Texel-gradient table of a replay workgroup: neighbouring pixels' paths splat mostly onto
-// the same texels, so each distinct texel gets one device atomic per channel and workgroup
-// iteration instead of one per lane. Open addressing on the texel's index in the gradient
-// pool; kGradEmpty marks a free slot.
-constexpr int kGradSlots = 2048;
-constexpr uint32_t kGradEmpty = 0xFFFFFFFFu;
-#ifdef __HIP_DEVICE_COMPILE__
-// Adds v[0..n) at `key` to the table, listing a newly taken slot; false when no slot was
-// found within the probe limit (the caller then adds to device memory).
-__device__ __forceinline__ bool grad_table_add(const AdjointCtx *adj, uint32_t key, const float *v, int n) {
-  uint32_t *keys = adj->table_keys;
-  float *vals = adj->table_vals;
-  uint32_t h = (key * 2654435761u) >> 21;  // 11 bits: kGradSlots
-  for (int probe = 0; probe < 32; probe++) {
-    const uint32_t old = atomicCAS(&keys[h], kGradEmpty, key);
-    if (old == kGradEmpty) adj->table_list[atomicAdd(adj->table_count, 1u)] = (uint16_t)h;
-    if (old == kGradEmpty || old == key) {
-      for (int c = 0; c < n; c++)
-        if (v[c] != 0.f) atomicAdd(&vals[h * 3 + c], v[c]);
-      return true;
-    }
-    h = (h + 1) & (kGradSlots - 1);
-  }
-  return false;
-}
-#endif
+// The texel gradients of one replayed scatter: the loss gradient with respect to the albedo and
+// roughness lookups of `material` at (u, v).
+struct SplatRec {
+  bool on;
+  int32_t material;
+  float u, v, albedo[3], roughness;
+};
 
 NOVA_HD void add_grad(float *p, float v) {
 #ifdef __HIP_DEVICE_COMPILE__
@@ -249,7 +224,7 @@ NOVA_HD void add_grad(float *p, float v) {
 }
 
 // Adds g[ch] * (bilinear weight) to the gradient of channel ch of the four texels an FP32
-// texture lookup blended (through the workgroup's table when the replay gives one).
+// texture lookup blended.
 NOVA_HD void splat_texture_grad(const ShadeCtx &sc, const AdjointCtx *adj, int tex, float u, float v, const float *g, int nch) {
   unsigned idx[4];
   float w[4];
@@ -258,14 +233,14 @@ NOVA_HD void splat_texture_grad(const ShadeCtx &sc, const AdjointCtx *adj, int t
   const int nc = nch < t.channels ? nch : t.channels;  // at most 3
   for (int k = 0; k < 4; k++) {
     const uint64_t key = t.offset + (uint64_t)idx[k] * (uint32_t)t.channels;  // the texel's channel 0 in the pool
-    float val[3] = {0.f, 0.f, 0.f};
-    for (int ch = 0; ch < nc; ch++) val[ch] = w[k] * g[ch];
-#ifdef __HIP_DEVICE_COMPILE__
-    if (adj->table_keys && key < kGradEmpty && grad_table_add(adj, (uint32_t)key, val, nc)) continue;
-#endif
     for (int ch = 0; ch < nc; ch++)
-      if (g[ch] != 0.f) add_grad(adj->grad + key + ch, val[ch]);
+      if (g[ch] != 0.f) add_grad(adj->grad + key + ch, w[k] * g[ch]);
   }
+}
+NOVA_HD void splat_grads(const ShadeCtx &sc, const AdjointCtx *adj, const SplatRec &r) {
+  const MatRec &mat = sc.mats[r.material];
+  if (mat.albedo_f32 >= 0) splat_texture_grad(sc, adj, mat.albedo_f32, r.u, r.v, r.albedo, 3);
+  if (mat.roughness_f32 >= 0) splat_texture_grad(sc, adj, mat.roughness_f32, r.u, r.v, &r.roughness, 1);
 }
 
 // The surface half of PrincipledMaterial::scatter (NovaMaterials.h:89-137) at a hit: the
@@ -393,11 +368,11 @@ NOVA_HD f3 emitted(const ShadeCtx &sc, const MatRec &mat, float u, float v) {
 // its radiance and alpha.
 // With kAdj the segment is replayed: after a scatter the radiance still to come,
 // R = L_path - L (everything after this vertex, T c V_next), gives the loss gradient of
-// the vertex's weight c; it is pushed to the albedo and roughness texels through
-// d ln c / d(param) and the bilinear weights.
+// the vertex's weight c; through d ln c / d(param) it goes to the albedo and roughness
+// texels (to *splat, for the caller to add, where one is given).
 template <bool kAdj = false, class Sobol = const uint32_t *>
 NOVA_HD bool shade_path(const ShadeParams &sp, const ShadeCtx &sc, Sobol sobol, uint32_t slot, f3 o, f3 d, int prim, float ht, float hu,
-                        float hv, f3 &T, f3 &L, float &A, f3 &no, f3 &nd, bool &escaped, const AdjointCtx *adj = nullptr) {
+                        float hv, f3 &T, f3 &L, float &A, f3 &no, f3 &nd, bool &escaped, const AdjointCtx *adj = nullptr, SplatRec *splat = nullptr) {
   escaped = false;
   if (prim < 0) {  // Li on a miss: envmap(ray.direction) (Integrator.cpp:93-97)
     escaped = true;
@@ -449,8 +424,11 @@ NOVA_HD bool shade_path(const ShadeParams &sp, const ShadeCtx &sc, Sobol sobol, 
       ga[rr_channel] -= (G[0] + G[1] + G[2]) * dm[rr_channel];
       gr[0] = 0.f;
     }
-    if (mat.albedo_f32 >= 0) splat_texture_grad(sc, adj, mat.albedo_f32, h.u, h.v, ga, 3);
-    if (mat.roughness_f32 >= 0) splat_texture_grad(sc, adj, mat.roughness_f32, h.u, h.v, gr, 1);
+    const SplatRec rec{mat.albedo_f32 >= 0 || mat.roughness_f32 >= 0, ss.material, h.u, h.v, {ga[0], ga[1], ga[2]}, gr[0]};
+    if (splat)
+      *splat = rec;
+    else
+      splat_grads(sc, adj, rec);
   }
   T = T * c;
   // Ray::spawn (Ray.h:22-27)

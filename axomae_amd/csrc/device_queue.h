@@ -1,4 +1,4 @@
-// Queue compaction shared by the wavefront kernels.
+// Queue compaction and sums over a wave shared by the kernels.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
@@ -28,6 +28,25 @@ __device__ __forceinline__ uint32_t block_reserve(uint64_t m, uint32_t *count, u
   uint32_t base = blk_base[buf];
   for (uint32_t k = 0; k < wv; k++) base += wave_cnt[buf][k];
   return base;
+}
+
+// Sums of v[0..16) over the wave, the sum of v[k] in lanes 4k .. 4k+3: each step exchanges half
+// of what is left with the lane across one bit, 17 exchanges where a tree for each value has 96.
+__device__ __forceinline__ float wave_sums_16(float (&v)[16]) {
+  const unsigned lane = __lane_id();
+#pragma unroll
+  for (int half = 8; half >= 1; half >>= 1) {
+    const bool up = (lane & (4u * half)) != 0;
+#pragma unroll
+    for (int k = 0; k < half; k++) {
+      const float send = up ? v[k] : v[k + half], keep = up ? v[k + half] : v[k];
+      v[k] = keep + __shfl_xor(send, 4 * half, 64);
+    }
+  }
+  float r = v[0];
+  r += __shfl_xor(r, 2, 64);
+  r += __shfl_xor(r, 1, 64);
+  return r;
 }
 
 }  // namespace nova_hip

@@ -19,6 +19,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "device_math.h"
@@ -26,6 +27,7 @@
 #include "device_queue.h"
 #include "device_shading.h"
 #include "device_trace.h"
+#include "device_walk.h"
 #include "nova_internal.h"
 
 namespace nova_hip {
@@ -34,21 +36,6 @@ namespace nova_hip {
 
 constexpr int kTailSlot = 5;  // count[] slot: 0, or 1 + the bounce from which the batch's paths finish in tail_kernel
 
-// A ray queue is cut into 2^shard_bits shards. Workgroup b works on shard b mod 2^shard_bits: its
-// first rays and its claims come from that shard, its survivors go to the same shard of the
-// next queue, and each shard's counters have a cache line of their own. Atomics on one address
-// run at 11.4 ns each on this chip, whatever the number of waves: with one counter the claims
-// (one per 56 rays) bound the camera walk of a one-sample 1080p frame (0.50 -> 0.34 ms; the
-// frame 2.11 -> 1.90 ms, six frames at 1021x577 of a scene with many misses 2.33 -> 1.84), and
-// long walks could not refill more often (64 samples at 1080p: 47.5 -> 45.8 ms). One shard per
-// XCD: 16 take 46.1 ms there, 32 take 46.4.
-//
-// The first queue is linear (entry = path id): shard k holds every 2^shard_bits-th chunk of
-// kQueueChunk entries, so all shards move through the image together. Later queues give shard k
-// the entries [k * seg, (k + 1) * seg), seg being what the shard holds at the start.
-constexpr uint32_t kQueueChunk = 256;
-constexpr uint32_t kMaxShardBits = 3;
-constexpr uint32_t kCounterStride = 32;  // words between two shards' counters
 struct Queues {
   float *ray[2];      // 6 planes of cap floats each: ox oy oz dx dy dz
   int32_t *slot[2];
@@ -65,29 +52,6 @@ struct Queues {
   uint32_t paths;     // paths of a batch (plane stride of the path state)
   uint32_t shard_bits, seg;
 };
-
-// Entries of share k of S of a linear queue of n entries, its runs of kRun dealt out in turn.
-template <uint32_t kRun>
-NOVA_HD uint32_t linear_share_count(uint32_t n, uint32_t S, uint32_t k) {
-  const uint32_t runs = n / kRun, rest = n % kRun, last = runs % S;
-  return (runs / S + (k < last ? 1u : 0u)) * kRun + (k == last ? rest : 0u);
-}
-// Entry i of shard k of a linear queue.
-NOVA_HD uint32_t linear_shard_pos(uint32_t bits, uint32_t k, uint32_t i) { return (((i / kQueueChunk) << bits) + k) * kQueueChunk + i % kQueueChunk; }
-
-// The workgroup's shard and its place among the workgroups of that shard.
-__device__ __forceinline__ uint32_t block_shard(uint32_t bits) { return blockIdx.x & ((1u << bits) - 1); }
-__device__ __forceinline__ uint32_t shard_blocks(uint32_t bits, uint32_t k) { return (gridDim.x + (1u << bits) - 1 - k) >> bits; }
-
-// Entries of a whole queue, the same value in every lane.
-__device__ __forceinline__ uint32_t queue_total(const uint32_t *shard_n, uint32_t bits) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t mine = lane < (1u << bits) ? shard_n[lane * kCounterStride] : 0u;
-  uint32_t n = 0;
-#pragma unroll
-  for (int k = 0; k < (1 << kMaxShardBits); k++) n += (uint32_t)__builtin_amdgcn_readlane((int)mine, k);
-  return n;
-}
 
 // AbstractIntegrator::render per pixel (Integrator.h:53-95): one camera ray per path slot.
 // The first shade takes the path id from the queue position and starts every path at T = 1,
@@ -124,11 +88,6 @@ __global__ __launch_bounds__(256) void generate_kernel(FrameParams fp, const uin
   }
 }
 
-#ifndef NOVA_TRACE_REFILL
-// idle lanes that trigger a refill of the per-ray walk (64 samples at 1080p: 48.3 ms at 60, 47.5
-// at 56, 46.2 at 40, 45.8 at 24, 47.2 at 8)
-#define NOVA_TRACE_REFILL 24
-#endif
 #ifndef NOVA_TRACE_WAVES
 #define NOVA_TRACE_WAVES 6  // waves per SIMD the extend kernel is compiled for (0: compiler's choice)
 #endif
@@ -145,87 +104,6 @@ static_assert(kTraceBlock == 256, "the workgroups-per-CU count assumes one wave 
 #else
 #define NOVA_TRACE_OCCUPANCY
 #endif
-
-// The per-ray walk of a queue by a whole grid: one traversal step per loop turn; a lane whose
-// ray has ended takes the next unclaimed ray as soon as NOVA_TRACE_REFILL lanes of its wave are
-// idle (one atomic per refill for the wave), so lanes do not wait for the wave's longest ray.
-// The queue comes in shares with a claim counter each; a wave claims from its own share only
-// (the shares are statistically alike, and taking over another's rays cost the loop 18
-// registers). A share's first rays go one per lane by thread index, without an atomic: a launch
-// over a nearly empty queue (the last bounces) then makes no claims at all. fetch(p, o, d) gives
-// the ray at place p of the queue, store(p, st) takes its finished state.
-template <uint32_t kRun>
-struct WalkShare {
-  uint32_t n;            // its entries
-  uint32_t first, step;  // the place of its entry 0, and from a run of kRun entries to its next
-  uint32_t begin;        // the entry of this workgroup's first lane
-  uint32_t handed;       // entries handed out by thread index
-  __device__ __forceinline__ uint32_t pos(uint32_t i) const { return first + (i / kRun) * step + i % kRun; }
-};
-// The share of a bounce's queue that this workgroup works on, its shard: the first queue is linear.
-__device__ __forceinline__ WalkShare<kQueueChunk> queue_share(const Queues &q, int which, bool linear) {
-  const uint32_t k = block_shard(q.shard_bits), n = q.shard_n[which][k * kCounterStride];
-  return {n, linear ? k * kQueueChunk : k * q.seg, linear ? kQueueChunk << q.shard_bits : kQueueChunk,
-          (blockIdx.x >> q.shard_bits) * (uint32_t)kTraceBlock, shard_blocks(q.shard_bits, k) * (uint32_t)kTraceBlock};
-}
-// Every workgroup a share of its own of a linear queue: runs of a wave's entries dealt out in
-// turn, short ones so that a share mixes many parts of the queue (normals of the 1080p scene of
-// 1,048,576 triangles: 0.52 ms with runs of 256, 0.47 with 64, 0.53 with 32).
-constexpr uint32_t kShareRun = 64;
-__device__ __forceinline__ WalkShare<kShareRun> workgroup_share(uint32_t n) {
-  return {linear_share_count<kShareRun>(n, gridDim.x, blockIdx.x), blockIdx.x * kShareRun, kShareRun * gridDim.x, 0, kTraceBlock};
-}
-struct WalkCounts {
-  uint32_t nodes = 0, tests = 0, wave_turns = 0, lane_turns = 0, tri_rounds = 0;  // instrumented launches only
-};
-
-template <bool kCount, class Share, class Fetch, class Store>
-__device__ __forceinline__ void refill_walk(const TraceCtx &tc, LdsStack &stk, const Share &share, uint32_t *claims, Fetch fetch, Store store,
-                                            WalkCounts &c) {
-  const uint32_t lane = threadIdx.x & 63, n = share.n, handed = share.handed;
-  TraceState ts;
-  bool have = false, exhausted = handed >= n;
-  uint32_t ray = 0;
-  for (uint32_t turns = 0; turns < (1u << 30); turns++) {
-    const uint64_t idle = __ballot(!have);
-    uint32_t base = share.begin + threadIdx.x - lane;  // first turn: every lane idle, a ray per lane
-    bool fill = turns == 0;
-    if (!fill && !exhausted && __popcll(idle) >= NOVA_TRACE_REFILL) {
-      const int leader = __builtin_ffsll((long long)idle) - 1;
-      if ((int)lane == leader) base = handed + atomicAdd(claims, (uint32_t)__popcll(idle));
-      base = __shfl(base, leader, 64);
-      if (base >= n) exhausted = true;
-      fill = true;
-    }
-    if (fill && !have) {
-      const uint32_t i = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0));
-      if (i < n) {
-        const uint32_t p = share.pos(i);
-        f3 o, d;
-        fetch(p, o, d);
-        trace_init(ts, o, d);
-        ray = p;
-        have = true;
-      }
-    }
-    const uint64_t busy = __ballot(have);
-    if (busy == 0) break;
-    if (kCount && (threadIdx.x & 63) == 0) {
-      c.wave_turns++;
-      c.lane_turns += (uint32_t)__popcll(busy);
-    }
-    if (have && trace_step<kCount>(tc, stk, ts, 0.000001f, c.nodes, c.tests)) {
-      store(ray, ts);
-      have = false;
-      if (kCount) c.tri_rounds += ts.tri_rounds;
-    }
-  }
-}
-
-// A finished ray's record: (prim id bits, t, u, v).
-__device__ __forceinline__ float4 hit_record(const TraceState &st) {
-  return make_float4(__builtin_bit_cast(float, (int32_t)(st.best)), st.tbest, st.bu, st.bv);
-}
 
 template <bool kCount>
 __global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void extend_kernel(TraceCtx tc, Queues q, int which, int bounce, uint32_t tail_rays,
@@ -250,7 +128,7 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void extend_kerne
     d = mk3(r[3 * cap + p], r[4 * cap + p], r[5 * cap + p]);
   };
   auto store = [&](uint32_t p, const TraceState &st) { q.hit[p] = hit_record(st); };
-  refill_walk<kCount>(tc, stk, queue_share(q, which, bounce == 0), q.work + block_shard(q.shard_bits) * kCounterStride, fetch, store, c);
+  refill_walk<kCount>(tc, stk, shard_share(q.shard_n[which], q.shard_bits, q.seg, bounce == 0), q.work + block_shard(q.shard_bits) * kCounterStride, fetch, store, c);
   if (kCount) {
     atomicAdd(&q.stats64[8], (unsigned long long)c.wave_turns);
     atomicAdd(&q.stats64[9], (unsigned long long)c.lane_turns);
@@ -315,8 +193,11 @@ __device__ __forceinline__ void write_partial(const Queues &q, uint32_t pid, flo
 #define NOVA_SHADE_WAVES 4  // waves per SIMD the shade kernel is compiled for (0: compiler's choice, 135 VGPRs and 3 waves;
                             // 4 waves spill one VGPR and shade 11% faster)
 #endif
+#ifndef NOVA_REPLAY_WAVES
+#define NOVA_REPLAY_WAVES 3  // the replay's (720p, 32 frames, 100,480 triangles: 6.8 ms; with 4 waves and 38 spilled VGPRs 7.3)
+#endif
 #if NOVA_SHADE_WAVES > 0
-#define NOVA_SHADE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(NOVA_SHADE_WAVES, NOVA_SHADE_WAVES)))
+#define NOVA_SHADE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(kAdj ? NOVA_REPLAY_WAVES : NOVA_SHADE_WAVES, kAdj ? NOVA_REPLAY_WAVES : NOVA_SHADE_WAVES)))
 #else
 #define NOVA_SHADE_OCCUPANCY
 #endif
@@ -325,6 +206,142 @@ __device__ __forceinline__ void write_partial(const Queues &q, uint32_t pid, flo
 #endif
 constexpr int kShadeBlock = 256;  // 512 and 1024 measured slower (barrier waits)
 
+// Texel-gradient table of a replay workgroup: what its paths' scatters of one iteration add to
+// the same texels is summed in LDS, and each entry goes to device memory once. An entry is a
+// lookup's place: the pool indices of the first of its four texels in the albedo and the
+// roughness texture (kNoTexel: no such texture) and 4 texels x (3 albedo channels, roughness)
+// sums. At most 256 lookups an iteration leave half of the slots free, so probes are short and
+// always end; a table of single texels had 8 entries per lookup, and where paths had scattered
+// its 2,048 slots were full.
+constexpr uint32_t kNoTexel = 0xFFFFFFFFu;
+constexpr unsigned long long kGradEmpty = ~0ull;
+constexpr int kGradSlots = 2 * kShadeBlock, kGradVals = 16;
+static_assert(kGradSlots == 512, "9 hash bits");
+struct GradTable {
+  unsigned long long keys[kGradSlots];
+  float vals[kGradVals][kGradSlots];  // value-major: the lanes' slots spread over the banks
+  uint16_t material[kGradSlots];      // a material with the entry's textures
+};
+__device__ __forceinline__ int grad_slot(GradTable &t, unsigned long long key, uint32_t material) {
+  uint32_t h = ((uint32_t)(key >> 32) * 2654435761u ^ (uint32_t)key * 2246822519u) >> 23;
+#pragma unroll 1
+  for (int probe = 0; probe < kGradSlots; probe++) {
+    const unsigned long long old = atomicCAS(&t.keys[h], kGradEmpty, key);
+    if (old == kGradEmpty) t.material[h] = (uint16_t)material;
+    if (old == kGradEmpty || old == key) return (int)h;
+    h = (h + 1) & (kGradSlots - 1);
+  }
+  return -1;  // not reached: at most kShadeBlock keys
+}
+#ifndef NOVA_GRAD_GROUP
+#define NOVA_GRAD_GROUP 8  // lookups of a wave at one place from which they are summed in registers first
+#endif
+// The wave's splats into the table; every lane calls it. Camera rays of one pixel's frames
+// mostly meet the same four texels: atomics on one LDS address take the lanes in turn, so a
+// place that many lanes share is summed over the wave first (first bounce of a 720p replay of 32
+// frames: 3.3 -> 2.9 ms). The replay's kernels of that job took 8.4 ms with single texels in the
+// table and unrolled probes, 21,298 instructions for a 64 KB instruction cache; now 6.8.
+__device__ __forceinline__ void splat_to_table(const ShadeCtx &sc, const AdjointCtx &adj, GradTable &t, const SplatRec &rec) {
+  const uint32_t lane = threadIdx.x & 63;
+  uint32_t ka = kNoTexel, kr = kNoTexel, material = 0;
+  float v[kGradVals];
+#pragma unroll
+  for (int k = 0; k < kGradVals; k++) v[k] = 0.f;
+  bool on = rec.on;
+  if (on) {
+    const MatRec &mat = sc.mats[rec.material];
+    material = (uint32_t)rec.material;
+    bool fits = material < 65536u;
+    unsigned idx[4];
+    float w[4];
+    if (mat.albedo_f32 >= 0) {
+      const TexRec tex = sc.tex[mat.albedo_f32];
+      bilinear_taps(sc, mat.albedo_f32, rec.u, rec.v, idx, w);
+      const uint64_t first = tex.offset + (uint64_t)idx[0] * (uint32_t)tex.channels;
+      fits = fits && first < kNoTexel;
+      ka = (uint32_t)first;
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int ch = 0; ch < 3; ch++) v[4 * k + ch] = ch < tex.channels && rec.albedo[ch] != 0.f ? w[k] * rec.albedo[ch] : 0.f;
+    }
+    if (mat.roughness_f32 >= 0) {
+      const TexRec tex = sc.tex[mat.roughness_f32];
+      bilinear_taps(sc, mat.roughness_f32, rec.u, rec.v, idx, w);
+      const uint64_t first = tex.offset + (uint64_t)idx[0] * (uint32_t)tex.channels;
+      fits = fits && first < kNoTexel;
+      kr = (uint32_t)first;
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[4 * k + 3] = rec.roughness != 0.f ? w[k] * rec.roughness : 0.f;
+    }
+    if (!fits) {
+      splat_grads(sc, &adj, rec);
+      on = false;
+    }
+  }
+  uint64_t pending = __ballot(on), single = 0;
+  for (int round = 0; round < 4 && pending != 0; round++) {
+    const int leader = __builtin_ffsll((long long)pending) - 1;
+    const uint32_t la = (uint32_t)__builtin_amdgcn_readlane((int)ka, leader), lr = (uint32_t)__builtin_amdgcn_readlane((int)kr, leader);
+    const uint64_t m = __ballot(ka == la && kr == lr) & pending;
+    pending &= ~m;
+    if (__popcll(m) < NOVA_GRAD_GROUP) {
+      single |= m;
+      continue;
+    }
+    float s[kGradVals];
+    const bool in = (m >> lane) & 1u;
+#pragma unroll
+    for (int k = 0; k < kGradVals; k++) s[k] = in ? v[k] : 0.f;
+    const float sum = wave_sums_16(s);
+    int slot = -1;
+    if ((int)lane == leader) slot = grad_slot(t, (unsigned long long)la << 32 | lr, material);
+    slot = __builtin_amdgcn_readlane(slot, leader);
+    if ((lane & 3u) == 0 && slot >= 0 && sum != 0.f) atomicAdd(&t.vals[lane >> 2][slot], sum);
+  }
+  single |= pending;
+  if ((single >> lane) & 1u) {
+    const int slot = grad_slot(t, (unsigned long long)ka << 32 | kr, material);
+    if (slot >= 0) {
+#pragma unroll
+      for (int k = 0; k < kGradVals; k++)
+        if (v[k] != 0.f) atomicAdd(&t.vals[k][slot], v[k]);
+    }
+  }
+}
+// The table's sums to device memory, and the table empty again. A wave takes 64 slots at a time,
+// 16 lanes an entry.
+__device__ __forceinline__ void flush_grads(const ShadeCtx &sc, float *grad, GradTable &t) {
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, k = lane & 15;
+  for (uint32_t s0 = wave * 64; s0 < kGradSlots; s0 += kShadeBlock) {
+    const bool used = t.keys[s0 + lane] != kGradEmpty;
+    uint64_t m = __ballot(used);
+    while (m != 0) {
+      int slot = -1;  // of the lane's group of 16: the group's turn among the next four entries
+#pragma unroll
+      for (uint32_t grp = 0; grp < 4; grp++) {
+        const int first = m != 0 ? __builtin_ffsll((long long)m) - 1 : -1;
+        if ((lane >> 4) == grp) slot = first;
+        m &= m - 1;  // 0 stays 0
+      }
+      if (slot < 0) continue;
+      const uint32_t e = s0 + (uint32_t)slot;
+      const float v = t.vals[k][e];
+      if (v != 0.f) {
+        const unsigned long long key = t.keys[e];
+        const MatRec &mat = sc.mats[t.material[e]];
+        const uint32_t ch = k & 3, tap = k >> 2;
+        const TexRec tex = sc.tex[ch < 3 ? mat.albedo_f32 : mat.roughness_f32];
+        const uint64_t first = ch < 3 ? (uint32_t)(key >> 32) : (uint32_t)key;
+        const uint64_t at = first + (uint64_t)((tap & 1) + (tap >> 1) * (uint32_t)tex.width) * (uint32_t)tex.channels + (ch < 3 ? ch : 0u);
+        add_grad(grad + at, v);
+        t.vals[k][e] = 0.f;
+      }
+    }
+    if (used) t.keys[s0 + lane] = kGradEmpty;
+  }
+}
+
 template <bool kAdj>
 __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel(ShadeParams sp, ShadeCtx sc, const uint32_t *__restrict__ sobol, Queues q, int which,
                                                     AdjointCtx adj) {
@@ -332,39 +349,12 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
   // nibble tables of this scatter's sampler dimensions (dim0 .. dim0+4)
   __shared__ uint32_t sob_tab[5 * 128];
   sobol_nibble_fill(sobol, sp.dim0, 5, sob_tab, threadIdx.x, blockDim.x);
-  // the replay's texel-gradient table (an array of one element in the primal kernel)
-  __shared__ uint32_t gkeys[kAdj ? kGradSlots : 1];
-  __shared__ float gvals[kAdj ? 3 * kGradSlots : 1];
-  __shared__ uint16_t glist[kAdj ? kGradSlots : 1];
-  __shared__ uint32_t gcount[2];  // list lengths of even and odd iterations
-  if (kAdj) {
-    for (int e = threadIdx.x; e < kGradSlots; e += blockDim.x) {
-      gkeys[e] = kGradEmpty;
-      gvals[3 * e] = gvals[3 * e + 1] = gvals[3 * e + 2] = 0.f;
-    }
-    if (threadIdx.x < 2) gcount[threadIdx.x] = 0;
-    adj.table_keys = gkeys;
-    adj.table_vals = gvals;
-    adj.table_list = glist;
+  __shared__ typename std::conditional<kAdj, GradTable, char>::type table;
+  if constexpr (kAdj) {
+    for (int e = threadIdx.x; e < kGradSlots; e += blockDim.x) table.keys[e] = kGradEmpty;
+    for (int e = threadIdx.x; e < kGradSlots * kGradVals; e += blockDim.x) table.vals[0][e] = 0.f;
   }
   __syncthreads();
-  // Iteration it's taken slots go to device memory (one atomic per texel channel) and are
-  // cleared; the next iteration's count starts at zero (it was read in iteration it - 1,
-  // before that iteration's closing barrier).
-  auto flush_table = [&](uint32_t it) {
-    const uint32_t used = gcount[it & 1u];
-    for (uint32_t e = threadIdx.x; e < used; e += blockDim.x) {
-      const uint32_t h = glist[e];
-      const uint32_t key = gkeys[h];
-      for (int c = 0; c < 3; c++) {
-        const float v = gvals[3 * h + c];
-        if (v != 0.f) add_grad(adj.grad + key + c, v);
-        gvals[3 * h + c] = 0.f;
-      }
-      gkeys[h] = kGradEmpty;
-    }
-    if (threadIdx.x == 0) gcount[(it + 1u) & 1u] = 0;
-  };
   const SobolNibbles sobn{sob_tab, sp.dim0};
   const size_t cap = q.cap, paths = q.paths;
   const float *rin = q.ray[which];
@@ -384,6 +374,7 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
     bool cont = false, escaped = false;
     f3 no = mk3(0, 0, 0), nd = mk3(0, 0, 0);
     int32_t pid = -1;
+    SplatRec splat{};
     if (e < n) {
       const bool first = sp.bounce == 0;  // camera rays: path id = queue position, fresh path state
       const uint32_t i = first ? linear_shard_pos(q.shard_bits, shard, e) : out0 + e;
@@ -396,7 +387,6 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
       int prim;
       float ht, hu, hv;
       AdjointCtx padj = adj;
-      padj.table_count = &gcount[it & 1u];
       if (kAdj) {  // this path's primal radiance (and hits), left by pass 0 under the same path id
         const size_t pid0 = (uint32_t)pid;
         padj.ltot = adj.ltot + pid0 * 4;
@@ -423,7 +413,7 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
         if (adj.hit_cache && (uint32_t)sp.bounce < adj.cache_bounces)
           adj.hit_cache[(size_t)sp.bounce * adj.cache_paths + pid] = make_float4(__builtin_bit_cast(float, prim), ht, hu, hv);
       }
-      cont = shade_path<kAdj>(sp, sc, sobn, path_slot(sp.fp, (uint32_t)pid), o, d, prim, ht, hu, hv, T, L, A, no, nd, escaped, &padj);
+      cont = shade_path<kAdj>(sp, sc, sobn, path_slot(sp.fp, (uint32_t)pid), o, d, prim, ht, hu, hv, T, L, A, no, nd, escaped, &padj, &splat);
       const bool done = !cont;
       q.T[pid] = T.x;
       q.T[paths + pid] = T.y;
@@ -437,12 +427,13 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
         q.A[pid] = A;
       }
     }
+    if constexpr (kAdj) splat_to_table(sc, adj, table, splat);
     escapes += (uint32_t)__popcll(__ballot(escaped));
     // compact survivors into the next queue
     const uint64_t m = __ballot(cont);
     const uint32_t lane_rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
     const uint32_t base = block_reserve<kShadeBlock>(m, out_n, it, wave_cnt, blk_base);
-    if (kAdj) flush_table(it);  // every lane has splatted this iteration (block_reserve waited)
+    if constexpr (kAdj) flush_grads(sc, adj.grad, table);  // every lane has splatted this iteration (block_reserve waited)
     if (cont) {
       const uint32_t j = out0 + base + lane_rank;
       rout[j] = no.x;
@@ -827,20 +818,6 @@ struct ScratchCarve {
   }
 };
 
-// How a batch's queues are cut: 2^bits shards of at least 4,096 paths each.
-struct QueueShape {
-  uint32_t bits, seg;
-  size_t entries;  // of one queue: the shards' room, a little more than the paths
-};
-static QueueShape queue_shape(size_t paths, uint32_t max_bits) {
-  QueueShape q{0, (uint32_t)paths, paths};
-  while (q.bits < max_bits && (paths >> (q.bits + 1)) >= 4096) q.bits++;
-  if (q.bits == 0) return q;
-  const size_t chunks = (paths + kQueueChunk - 1) / kQueueChunk, S = (size_t)1 << q.bits;
-  q.seg = (uint32_t)((chunks + S - 1) / S * kQueueChunk);
-  q.entries = (size_t)q.seg * S;
-  return q;
-}
 // Counters: a line of control words and statistics, then the two queues' and the claims' lines.
 // One shard keeps its three words in the first line.
 constexpr size_t kControlBytes = 256, kShardLineBytes = kCounterStride * sizeof(uint32_t);
