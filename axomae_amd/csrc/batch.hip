@@ -22,6 +22,7 @@
 #include "device_queue.h"
 #include "device_shading.h"
 #include "device_trace.h"
+#include "device_walk.h"
 #include "nova_internal.h"
 
 namespace nova_hip {
@@ -55,10 +56,11 @@ struct Segment {
 
 struct BatchState {
   uint32_t wave;
-  uint32_t count[2];  // queue sizes
-  uint32_t work;      // rays of the current queue claimed by the extend launch
   uint32_t do_accum;
   unsigned long long segments;  // rays traced
+  // per shard of the queues, a cache line apart: entries; rays of the current queue claimed by the extend launch
+  uint32_t shard_n[2][kCounterStride << kMaxShardBits];
+  uint32_t work[kCounterStride << kMaxShardBits];
 };
 
 struct BatchQueues {
@@ -68,7 +70,8 @@ struct BatchQueues {
   float4 *hit;        // closest hit per queue entry: (prim id bits, t, u, v), one 16-byte record
   float *T, *L, *A;
   float *partial;  // wave-relative slot x 4
-  uint32_t cap;
+  uint32_t cap;    // paths of a wave (plane stride of the path state)
+  uint32_t entries, shard_bits, seg;  // of a queue: plane stride; its shards
 };
 
 __device__ __forceinline__ int find_scene(const BatchScene *__restrict__ scenes, int n, uint64_t g) {
@@ -90,7 +93,7 @@ __global__ __launch_bounds__(256) void batch_generate(const BatchScene *__restri
   __syncthreads();
   const SobolNibbles sobn{sob_tab, 0};
   const WaveDesc w = waves[st->wave];
-  const size_t n = q.cap;
+  const size_t n = q.cap, qn = q.entries;
   for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < w.count; r += gridDim.x * blockDim.x) {
     const uint64_t g = w.start + r;
     const int s = find_scene(scenes, nscenes, g);
@@ -99,79 +102,58 @@ __global__ __launch_bounds__(256) void batch_generate(const BatchScene *__restri
     camera_ray(scenes[s].fp, sobn, path_slot(scenes[s].fp, l), o, d);
     float *ray = q.ray[0];
     ray[r] = o.x;
-    ray[n + r] = o.y;
-    ray[2 * n + r] = o.z;
-    ray[3 * n + r] = d.x;
-    ray[4 * n + r] = d.y;
-    ray[5 * n + r] = d.z;
+    ray[qn + r] = o.y;
+    ray[2 * qn + r] = o.z;
+    ray[3 * qn + r] = d.x;
+    ray[4 * qn + r] = d.y;
+    ray[5 * qn + r] = d.z;
     q.slot[0][r] = (int32_t)r;
     q.sid[0][r] = s;
     q.T[r] = q.T[n + r] = q.T[2 * n + r] = 1.f;
     q.L[r] = q.L[n + r] = q.L[2 * n + r] = 0.f;
     q.A[r] = 0.f;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    st->count[0] = w.count;
-    st->count[1] = 0;
-    st->work = 0;
+  if (blockIdx.x == 0 && threadIdx.x < (1u << q.shard_bits)) {
+    const uint32_t k = threadIdx.x;
+    st->shard_n[0][k * kCounterStride] = linear_share_count<kQueueChunk>(w.count, 1u << q.shard_bits, k);
+    st->shard_n[1][k * kCounterStride] = 0;
+    st->work[k * kCounterStride] = 0;
   }
 }
 
-// Closest hits of the queue with the single-scene kernel's lane refill: a lane whose ray
-// has ended takes the next unclaimed ray once kBatchRefill lanes of its wave are idle.
-constexpr uint32_t kBatchRefill = 56;
 // Tie tables of a lane's scene: an address computed from the scene index, not a pointer
 // loaded from the scene record at every leaf.
 struct SceneTie {
   const BatchScene *scenes;
-  int32_t sid;
-  __device__ const TieTables *operator()(const TraceCtx &) const { return &scenes[sid].tie; }
+  const int32_t *sid;
+  __device__ const TieTables *operator()(const TraceCtx &) const { return &scenes[*sid].tie; }
 };
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6, 6))) void batch_extend(
-    const BatchScene *__restrict__ scenes, BatchState *st, BatchQueues q, int which, uint32_t *gstack, uint32_t gstride) {
+// Closest hits of the queue: the single-scene renderer's walk, each lane's scene loaded when it
+// takes a ray (not at every step). The scene pointers take its registers past the budget of 6
+// waves per SIMD; at 5 nothing spills. 16 scenes, 55 M paths: 10.5 ms with one claim counter for
+// the chip, refills at 56 idle lanes and 6 waves; 8.8 with shards and refills at 24; 8.4 at 5.
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5, 5))) void batch_extend(
+    const BatchScene *__restrict__ scenes, BatchState *st, BatchQueues q, int which, int bounce, uint32_t *gstack, uint32_t gstride) {
   __shared__ uint32_t lds[kLdsStack * kTraceBlock];
-  const uint32_t n = st->count[which];
+  const uint32_t n = queue_total(st->shard_n[which], q.shard_bits);
   const float *r = q.ray[which];
-  const size_t cap = q.cap;
+  const size_t qn = q.entries;
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   if (gtid == 0) st->segments += n;
   LdsStack stk{lds, gstack, gstride, gtid, threadIdx.x};
-  // first rays by thread index, refills claimed past them (as extend_kernel)
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t nthreads = gridDim.x * blockDim.x;
-  TraceState ts;
-  bool have = false, exhausted = nthreads >= n;
-  uint32_t ray = 0;
+  TraceCtx tc{nullptr, nullptr, nullptr, 0, nullptr};
   int32_t sid = 0;
-  TraceCtx tc{nullptr, nullptr, nullptr, 0, nullptr};  // the lane's scene, loaded when it takes a ray (not at every step)
-  uint32_t nv = 0, nt = 0;
-  for (uint32_t turns = 0; turns < (1u << 30); turns++) {
-    const uint64_t idle = __ballot(!have);
-    uint32_t base = gtid - lane;  // first turn: lane l takes ray gtid
-    bool fill = turns == 0;
-    if (!fill && !exhausted && (uint32_t)__popcll(idle) >= kBatchRefill) {
-      const int leader = __builtin_ffsll((long long)idle) - 1;
-      if ((int)lane == leader) base = nthreads + atomicAdd(&st->work, (uint32_t)__popcll(idle));
-      base = __shfl(base, leader, 64);
-      if (base >= n) exhausted = true;
-      fill = true;
-    }
-    if (fill && !have) {
-      const uint32_t i = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0));
-      if (i < n) {
-        trace_init(ts, mk3(r[i], r[cap + i], r[2 * cap + i]), mk3(r[3 * cap + i], r[4 * cap + i], r[5 * cap + i]));
-        ray = i;
-        sid = q.sid[which][i];
-        tc = scenes[sid].tc;
-        have = true;
-      }
-    }
-    if (__ballot(have) == 0) break;
-    if (have && trace_step<false>(tc, stk, ts, 0.000001f, nv, nt, SceneTie{scenes, sid})) {
-      q.hit[ray] = make_float4(__builtin_bit_cast(float, (int32_t)(ts.best)), ts.tbest, ts.bu, ts.bv);
-      have = false;
-    }
-  }
+  WalkCounts c;
+  refill_walk<false>(
+      tc, stk, shard_share(st->shard_n[which], q.shard_bits, q.seg, bounce == 0), st->work + block_shard(q.shard_bits) * kCounterStride,
+      [&](uint32_t p, f3 &o, f3 &d) {
+        o = mk3(r[p], r[qn + p], r[2 * qn + p]);
+        d = mk3(r[3 * qn + p], r[4 * qn + p], r[5 * qn + p]);
+        sid = q.sid[which][p];
+        tc.nodes = scenes[sid].tc.nodes;
+        tc.tris = scenes[sid].tc.tris;
+      },
+      [&](uint32_t p, const TraceState &ts) { q.hit[p] = hit_record(ts); }, c, SceneTie{scenes, &sid});
 }
 
 // Camera rays (queue 0 right after batch_generate, in slot order) walked once per wave of 64
@@ -181,9 +163,9 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6, 
 constexpr int kBatchCoherentBlock = 256;
 constexpr uint32_t kBatchCoherentBlocksPerCu = 64;  // grid-stride over the packets, as the single-scene walk
 __global__ __launch_bounds__(kBatchCoherentBlock) void batch_extend_coherent(const BatchScene *__restrict__ scenes, BatchState *st, BatchQueues q) {
-  const uint32_t n = st->count[0];
+  const uint32_t n = queue_total(st->shard_n[0], q.shard_bits);
   const float *r = q.ray[0];
-  const size_t cap = q.cap;
+  const size_t cap = q.entries;
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if (blockIdx.x == 0 && threadIdx.x == 0) st->segments += n;
   uint32_t nv = 0, nt = 0;
@@ -206,8 +188,8 @@ __global__ __launch_bounds__(kBatchCoherentBlock) void batch_extend_coherent(con
 // Between an extend and a shade launch: the shade's output queue and the next extend's work
 // counter start at zero.
 __global__ void batch_reset(BatchState *st, int which) {
-  st->count[which] = 0;
-  st->work = 0;
+  st->shard_n[which][threadIdx.x * kCounterStride] = 0;
+  st->work[threadIdx.x * kCounterStride] = 0;
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void batch_shade(const BatchScene *__restrict__ scenes, const WaveDesc *__restrict__ waves, BatchState *st,
@@ -217,28 +199,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   sobol_nibble_fill(sobol, dim0, 5, sob_tab, threadIdx.x, blockDim.x);
   __syncthreads();
   const SobolNibbles sobn{sob_tab, dim0};
-  const uint32_t n = st->count[which];
   const uint64_t wstart = waves[st->wave].start;
-  const size_t cap = q.cap;
+  const size_t cap = q.cap, qn = q.entries;
   const float *rin = q.ray[which];
   float *rout = q.ray[which ^ 1];
-  const uint32_t stride = gridDim.x * blockDim.x;
-  const uint32_t iters = (n + stride - 1) / stride;  // uniform over the grid: the compaction below needs every thread
+  // the workgroup's shard of the queue; its survivors go to the same shard of the next one
+  const uint32_t shard = block_shard(q.shard_bits), n = st->shard_n[which][shard * kCounterStride], out0 = shard * q.seg;
+  const uint32_t stride = shard_blocks(q.shard_bits, shard) * blockDim.x;
+  const uint32_t iters = (n + stride - 1) / stride;  // uniform over the workgroup: the compaction below needs every thread
   __shared__ uint32_t wave_cnt[2][4], blk_base[2];
   for (uint32_t it = 0; it < iters; it++) {
-    const uint32_t i = it * stride + blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t e = it * stride + (blockIdx.x >> q.shard_bits) * blockDim.x + threadIdx.x;
     bool cont = false, escaped = false;
     f3 no = mk3(0, 0, 0), nd = mk3(0, 0, 0);
     int32_t slot = -1, sid = 0;
-    if (i < n) {
+    if (e < n) {
+      const uint32_t i = bounce == 0 ? linear_shard_pos(q.shard_bits, shard, e) : out0 + e;
       slot = q.slot[which][i];
       sid = q.sid[which][i];
-      const BatchScene &S = scenes[sid];
-      const f3 o = mk3(rin[i], rin[cap + i], rin[2 * cap + i]);
-      const f3 d = mk3(rin[3 * cap + i], rin[4 * cap + i], rin[5 * cap + i]);
+      const f3 o = mk3(rin[i], rin[qn + i], rin[2 * qn + i]);
+      const f3 d = mk3(rin[3 * qn + i], rin[4 * qn + i], rin[5 * qn + i]);
       f3 T = mk3(q.T[slot], q.T[cap + slot], q.T[2 * cap + slot]);
       f3 L = mk3(q.L[slot], q.L[cap + slot], q.L[2 * cap + slot]);
       float A = q.A[slot];
+      const float4 h = q.hit[i];
+      const BatchScene &S = scenes[sid];
       ShadeParams sp;
       sp.fp = S.fp;
       sp.bounce = bounce;
@@ -246,7 +231,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       sp.rr = rr;
       sp.dim0 = dim0;
       const uint32_t l = (uint32_t)(wstart + (uint64_t)slot - S.first);
-      const float4 h = q.hit[i];
       cont = shade_path(sp, S.sc, sobn, path_slot(S.fp, l), o, d, __builtin_bit_cast(int32_t, h.x), h.y, h.z, h.w, T, L, A, no, nd, escaped);
       q.T[slot] = T.x;
       q.T[cap + slot] = T.y;
@@ -262,15 +246,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     }
     const uint64_t m = __ballot(cont);
     const uint32_t lane_rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-    const uint32_t base = block_reserve<256>(m, &st->count[which ^ 1], it, wave_cnt, blk_base);
+    const uint32_t base = block_reserve<256>(m, &st->shard_n[which ^ 1][shard * kCounterStride], it, wave_cnt, blk_base);
     if (cont) {
-      const uint32_t j = base + lane_rank;
+      const uint32_t j = out0 + base + lane_rank;
       rout[j] = no.x;
-      rout[cap + j] = no.y;
-      rout[2 * cap + j] = no.z;
-      rout[3 * cap + j] = nd.x;
-      rout[4 * cap + j] = nd.y;
-      rout[5 * cap + j] = nd.z;
+      rout[qn + j] = no.y;
+      rout[2 * qn + j] = no.z;
+      rout[3 * qn + j] = nd.x;
+      rout[4 * qn + j] = nd.y;
+      rout[5 * qn + j] = nd.z;
       q.slot[which ^ 1][j] = slot;
       q.sid[which ^ 1][j] = sid;
     }
@@ -316,9 +300,7 @@ __global__ void batch_advance(BatchState *st) { st->wave += 1; }
 __global__ void batch_set(BatchState *st, uint32_t wave, uint32_t do_accum) {
   st->wave = wave;
   st->do_accum = do_accum;
-  st->count[0] = st->count[1] = 0;
-  st->work = 0;
-  st->segments = 0;
+  st->segments = 0;  // batch_generate sets the queue counters
 }
 
 __global__ void batch_zero(float *__restrict__ p, size_t n) {
@@ -386,23 +368,28 @@ struct BatchBuffers {
 static int alloc_buffers(nova_hip_ctx *ex, const BatchPlan &bp, const WavePlan &wp, uint32_t cap, uint32_t trace_threads, BatchBuffers &B,
                          hipStream_t s) {
   hipError_t e;
-  char *qbuf = (char *)ensure_scratch(ex, 6, (size_t)cap * (12 + 2 + 2 + 4 + 7 + 4) * 4, &e);
+  const QueueShape qs = queue_shape(cap, kMaxShardBits);
+  const size_t qn = qs.entries;  // a multiple of 256, as cap is: every piece stays 16-byte aligned
+  char *qbuf = (char *)ensure_scratch(ex, 6, (qn * (12 + 2 + 2 + 4) + (size_t)cap * (7 + 4)) * 4, &e);
   if (!qbuf) return check_hip(ex, e, "batch queue alloc");
   float *f = (float *)qbuf;
   B.q.cap = cap;
+  B.q.entries = (uint32_t)qn;
+  B.q.shard_bits = qs.bits;
+  B.q.seg = qs.seg;
   B.q.ray[0] = f;
-  B.q.ray[1] = f + (size_t)cap * 6;
-  int32_t *ip = (int32_t *)(f + (size_t)cap * 12);
+  B.q.ray[1] = f + qn * 6;
+  int32_t *ip = (int32_t *)(f + qn * 12);
   B.q.slot[0] = ip;
-  B.q.slot[1] = ip + cap;
-  B.q.sid[0] = ip + 2 * (size_t)cap;
-  B.q.sid[1] = ip + 3 * (size_t)cap;
-  B.q.hit = reinterpret_cast<float4 *>(ip + 4 * (size_t)cap);  // 16-byte aligned: cap is a multiple of 256
-  float *hf = (float *)(ip + 8 * (size_t)cap);
+  B.q.slot[1] = ip + qn;
+  B.q.sid[0] = ip + 2 * qn;
+  B.q.sid[1] = ip + 3 * qn;
+  B.q.hit = reinterpret_cast<float4 *>(ip + 4 * qn);
+  float *hf = (float *)(ip + 8 * qn);
   B.q.T = hf;
   B.q.L = hf + 3 * (size_t)cap;
   B.q.A = hf + 6 * (size_t)cap;
-  B.q.partial = hf + 7 * (size_t)cap;  // 4 floats per slot, 16-byte aligned (cap is a multiple of 256)
+  B.q.partial = hf + 7 * (size_t)cap;  // 4 floats per slot
   B.scenes = (BatchScene *)ensure_scratch(ex, 7, bp.scenes.size() * sizeof(BatchScene), &e);
   if (!B.scenes) return check_hip(ex, e, "batch scene table alloc");
   B.waves = (WaveDesc *)ensure_scratch(ex, 8, std::max<size_t>(1, wp.waves.size()) * sizeof(WaveDesc), &e);
@@ -437,9 +424,9 @@ static void launch_wave(const BatchPlan &bp, const BatchBuffers &B, const nova_h
       hipLaunchKernelGGL(batch_extend_coherent, dim3(std::min<uint32_t>((cap + kBatchCoherentBlock - 1) / kBatchCoherentBlock, (uint32_t)cus * kBatchCoherentBlocksPerCu)),
                          dim3(kBatchCoherentBlock), 0, s, B.scenes, B.state, B.q);
     else
-      hipLaunchKernelGGL(batch_extend, dim3(trace_blocks), dim3(kTraceBlock), 0, s, B.scenes, B.state, B.q, which, B.gstack,
+      hipLaunchKernelGGL(batch_extend, dim3(trace_blocks), dim3(kTraceBlock), 0, s, B.scenes, B.state, B.q, which, k, B.gstack,
                          trace_blocks * (uint32_t)kTraceBlock);
-    hipLaunchKernelGGL(batch_reset, dim3(1), dim3(1), 0, s, B.state, which ^ 1);
+    hipLaunchKernelGGL(batch_reset, dim3(1), dim3(1u << kMaxShardBits), 0, s, B.state, which ^ 1);
     const int rr = (bp.rr_start >= 0 && k >= bp.rr_start) ? 1 : 0;
     hipLaunchKernelGGL(batch_shade, dim3(shade_blocks), dim3(256), 0, s, B.scenes, B.waves, B.state, sobol, B.q, which, k,
                        k == bp.max_depth ? 1 : 0, rr, dim);
