@@ -137,6 +137,7 @@ struct nova_hip_ctx {
   uint32_t bnode_count = 0;
   nova_hip::Node4 *nodes4 = nullptr;
   nova_hip::Node4F *nodes4f = nullptr;        // the nodes with decoded planes (wave-coherent walk)
+  size_t wide_capacity = 0;                  // entries of nodes4 and nodes4f
   nova_hip::TriMT *tri_leaf = nullptr;       // MT records in leaf order (prim id in a.w)
   int32_t *bparent = nullptr;                // binary tree parent (-1 at the root)
   int32_t *bdepth = nullptr;                 // binary tree depth
