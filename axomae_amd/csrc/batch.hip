@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void batch_generate(const BatchScene *__restri
     const int s = find_scene(scenes, nscenes, g);
     const uint32_t l = (uint32_t)(g - scenes[s].first);
     f3 o, d;
-    camera_ray(scenes[s].fp, sobn, path_slot(scenes[s].fp, l), o, d);
+    camera_ray(scenes[s].fp, sobn, path_pixel(scenes[s].fp, l), o, d);
     float *ray = q.ray[0];
     ray[r] = o.x;
     ray[qn + r] = o.y;
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       sp.rr = rr;
       sp.dim0 = dim0;
       const uint32_t l = (uint32_t)(wstart + (uint64_t)slot - S.first);
-      cont = shade_path(sp, S.sc, sobn, path_slot(S.fp, l), o, d, __builtin_bit_cast(int32_t, h.x), h.y, h.z, h.w, T, L, A, no, nd, escaped);
+      cont = shade_path(sp, S.sc, sobn, path_pixel(S.fp, l), o, d, __builtin_bit_cast(int32_t, h.x), h.y, h.z, h.w, T, L, A, no, nd, escaped);
       q.T[slot] = T.x;
       q.T[cap + slot] = T.y;
       q.T[2 * cap + slot] = T.z;

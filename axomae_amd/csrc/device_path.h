@@ -25,8 +25,9 @@ struct ShadeParams {
 
 // Output offset of pixel p (floats): AbstractIntegrator::generateImageOffset (Integrator.h:38-42)
 NOVA_HD uint32_t pixel_offset(const FrameParams &fp, uint32_t p) {
+  if (!fp.vinvert) return p * 4u;
   const uint32_t x = p % (uint32_t)fp.width, y = p / (uint32_t)fp.width;
-  return fp.vinvert ? (((uint32_t)fp.height - 1 - y) * (uint32_t)fp.width + x) * 4u : (y * (uint32_t)fp.width + x) * 4u;
+  return (((uint32_t)fp.height - 1 - y) * (uint32_t)fp.width + x) * 4u;
 }
 
 // Pixel of rank r in the order the paths take them. Row by row, or with fp.tiled: each band
@@ -58,12 +59,29 @@ NOVA_HD uint32_t path_slot(const FrameParams &fp, uint32_t pid) {
   return (pid % (uint32_t)fp.frames) * npix + pixel_of_rank(fp, pid / (uint32_t)fp.frames);
 }
 
-// Sampler index of a path slot (frame-major slots), u32 wraparound. CPU policy:
+// A path's frame (from frame0 on) and pixel: what its slot holds, without the division that takes
+// a slot apart again. The stages below take either.
+struct PathPixel {
+  uint32_t frame, pixel;
+};
+NOVA_HD PathPixel path_pixel(const FrameParams &fp, uint32_t pid) {
+  if (fp.frame_minor) return {pid % (uint32_t)fp.frames, pixel_of_rank(fp, pid / (uint32_t)fp.frames)};
+  const uint32_t npix = (uint32_t)fp.width * (uint32_t)fp.height;
+  return {pid / npix, pid % npix};
+}
+NOVA_HD PathPixel slot_pixel(const FrameParams &, PathPixel p) { return p; }
+NOVA_HD PathPixel slot_pixel(const FrameParams &fp, uint32_t slot) {
+  const uint32_t npix = (uint32_t)fp.width * (uint32_t)fp.height;
+  return {slot / npix, slot % npix};
+}
+
+// Sampler index of a path (its slot or its frame and pixel), u32 wraparound. CPU policy:
 // idx * frame + renderer_max_samples with idx = 4 * pixel (Integrator.h:80). OptiX policy:
 // (x * H + y) * sample_max + frame (integrator_optix.cu:43).
-NOVA_HD uint32_t sample_index(const FrameParams &fp, uint32_t slot) {
-  const uint32_t npix = (uint32_t)fp.width * (uint32_t)fp.height;
-  const uint32_t f = (uint32_t)fp.frame0 + slot / npix, p = slot % npix;
+template <class Slot>
+NOVA_HD uint32_t sample_index(const FrameParams &fp, Slot slot) {
+  const PathPixel pp = slot_pixel(fp, slot);
+  const uint32_t f = (uint32_t)fp.frame0 + pp.frame, p = pp.pixel;
   if (fp.policy == NOVA_HIP_INDEX_OPTIX) return ((p % (uint32_t)fp.width) * (uint32_t)fp.height + p / (uint32_t)fp.width) * fp.offset + f;
   return pixel_offset(fp, p) * f + fp.offset;
 }
@@ -121,10 +139,10 @@ NOVA_HD void camera_ray_ndc(const FrameParams &fp, float nx, float ny, f3 &o, f3
 }
 
 // Sob: the direction table (const uint32_t *) or nibble tables holding dims 0-1 (SobolNibbles).
-template <class Sob>
-NOVA_HD void camera_ray(const FrameParams &fp, const Sob &sobol, uint32_t slot, f3 &o, f3 &d) {
-  const uint32_t npix = (uint32_t)fp.width * (uint32_t)fp.height;
-  const uint32_t p = slot % npix;
+template <class Sob, class Slot>
+NOVA_HD void camera_ray(const FrameParams &fp, const Sob &sobol, Slot slot_of, f3 &o, f3 &d) {
+  const PathPixel slot = slot_pixel(fp, slot_of);
+  const uint32_t p = slot.pixel;
   const int x = (int)(p % (uint32_t)fp.width), y = (int)(p / (uint32_t)fp.width);
   const uint32_t idx = sample_index(fp, slot);
   const uint32_t g = idx ^ (idx >> 1);
@@ -256,8 +274,8 @@ struct SurfaceSample {
   float dlnr;      // with kAdj: d ln c / d roughness
 };
 
-template <bool kAdj = false, class Sobol = const uint32_t *>
-NOVA_HD void sample_surface(const ShadeParams &sp, const ShadeCtx &sc, Sobol sobol, uint32_t slot, f3 o, f3 d, int prim, float ht, float hu, float hv,
+template <bool kAdj = false, class Sobol = const uint32_t *, class Slot = uint32_t>
+NOVA_HD void sample_surface(const ShadeParams &sp, const ShadeCtx &sc, Sobol sobol, Slot slot, f3 o, f3 d, int prim, float ht, float hu, float hv,
                             SurfaceSample &out) {
   const ShadeTri &tr = sc.shade[prim];
   out.h = make_hit(sc, tr, o, d, ht, hu, hv);
@@ -305,34 +323,27 @@ NOVA_HD void sample_surface(const ShadeParams &sp, const ShadeCtx &sc, Sobol sob
   const uint32_t idx = sample_index(sp.fp, slot);
   const uint32_t g = idx ^ (idx >> 1);
   const float uc = sobol_dim(sobol, sp.dim0, g);
-  const float u0 = sobol_dim(sobol, sp.dim0 + 1, g);
-  const float u1 = sobol_dim(sobol, sp.dim0 + 2, g);
   Principled b;
   b.configure(bi);
+  b.orient(bi);
   b.construct(uc);
-  const VNDF ggx_e(b.anisotropy, b.roughness);  // BSDF value
-  VNDF ggx = ggx_e;  // samples and weights by its pdf
   const bool detached = sc.sampling_roughness >= 0 && mat.roughness_f32 >= 0;
-  if (detached) ggx = VNDF(b.anisotropy, sample_f32_bilinear(sc, sc.sampling_roughness, h.u, h.v).x);
-  if ((b.flags(ggx) & (BX_GLOSSY | BX_REFLECTION)) && bi.wo_dot_ng >= 0) {
-    // the corrected shading normal reconfigures the frame; the chosen lobe and its weights stay
-    bi.ns = normalize(correct_specular_shading_normal(bi.ng, wo, bi.ns));
-    const int lobe = b.lobe;
-    const float lw = b.lobe_weight, lp = b.lobe_prob;
-    b.configure(bi);
-    b.lobe = lobe;
-    b.lobe_weight = lw;
-    b.lobe_prob = lp;
-  }
-  const float uc2 = sobol_dim(sobol, sp.dim0 + 3, g);
+  const float r_sampling = detached ? sample_f32_bilinear(sc, sc.sampling_roughness, h.u, h.v).x : b.roughness;
+  // a glossy or reflecting lobe (every lobe but a delta transmission and none)
+  const bool no_reflection = b.lobe == LOBE_NONE || (b.lobe == LOBE_DIELECTRIC && b.eta.x == 1.f && VNDF(b.anisotropy, r_sampling).full_specular());
+  // the corrected shading normal moves the frame; the chosen lobe and its weights do not depend on it
+  if (!no_reflection && bi.wo_dot_ng >= 0) bi.ns = normalize(correct_specular_shading_normal(bi.ng, wo, bi.ns));
+  if (!no_reflection && bi.wo_dot_ng >= 0) b.orient(bi);
   // PrincipledBSDF::sample_f (BSDF.h:107-130)
+  const float u0 = sobol_dim(sobol, sp.dim0 + 1, g);
+  const float u1 = sobol_dim(sobol, sp.dim0 + 2, g);
   BsdfSample smp{};
   bool ok = false;
   out.dlna = mk3(0.f, 0.f, 0.f);
   out.dlnr = 0.f;
   if (b.lobe != LOBE_NONE) {
     const f3 lwo = normalize_mid(mul_t(b.frame, wo));
-    if ((b.flags(ggx) & (BX_REFLECTION | BX_TRANSMISSION)) && lwo.z != 0.f) {
+    if (lwo.z != 0.f) {
       const bool diffuse = b.lobe == LOBE_DIFFUSE;
       float r, ang, sn, cs;
       if (diffuse) {
@@ -342,9 +353,17 @@ NOVA_HD void sample_surface(const ShadeParams &sp, const ShadeCtx &sc, Sobol sob
         ang = (float)(2.0 * 3.14159265358979323846 * (double)u1);
       }
       sincos_turns(ang, sn, cs);
-      ok = diffuse ? sample_disney(b, lwo, r * cs, r * sn, smp) : sample_microfacet(b, ggx, ggx_e, !detached, lwo, uc2, r * cs, r * sn, smp);
+      if (diffuse) {
+        ok = sample_disney(b, lwo, r * cs, r * sn, smp);
+        if (kAdj && ok) bsdf_log_derivatives(b, VNDF(b.anisotropy, b.roughness), lwo, smp, out.dlna, out.dlnr);
+      } else {
+        const VNDF ggx_e(b.anisotropy, b.roughness);  // BSDF value
+        VNDF ggx = ggx_e;                             // samples and weights by its pdf
+        if (detached) ggx = VNDF(b.anisotropy, r_sampling);
+        ok = sample_microfacet(b, ggx, ggx_e, !detached, lwo, [&]() { return sobol_dim(sobol, sp.dim0 + 3, g); }, r * cs, r * sn, smp);
+        if (kAdj && ok) bsdf_log_derivatives(b, ggx_e, lwo, smp, out.dlna, out.dlnr);
+      }
       if (ok && ((smp.f.x == 0.f && smp.f.y == 0.f && smp.f.z == 0.f) || smp.pdf == 0.f || smp.wi.z == 0.f)) ok = false;
-      if (kAdj && ok) bsdf_log_derivatives(b, ggx_e, lwo, smp, out.dlna, out.dlnr);
       if (ok) smp.wi = normalize_mid(mul(b.frame, smp.wi));
     }
   }
@@ -370,8 +389,8 @@ NOVA_HD f3 emitted(const ShadeCtx &sc, const MatRec &mat, float u, float v) {
 // R = L_path - L (everything after this vertex, T c V_next), gives the loss gradient of
 // the vertex's weight c; through d ln c / d(param) it goes to the albedo and roughness
 // texels (to *splat, for the caller to add, where one is given).
-template <bool kAdj = false, class Sobol = const uint32_t *>
-NOVA_HD bool shade_path(const ShadeParams &sp, const ShadeCtx &sc, Sobol sobol, uint32_t slot, f3 o, f3 d, int prim, float ht, float hu,
+template <bool kAdj = false, class Sobol = const uint32_t *, class Slot = uint32_t>
+NOVA_HD bool shade_path(const ShadeParams &sp, const ShadeCtx &sc, Sobol sobol, Slot slot, f3 o, f3 d, int prim, float ht, float hu,
                         float hv, f3 &T, f3 &L, float &A, f3 &no, f3 &nd, bool &escaped, const AdjointCtx *adj = nullptr, SplatRec *splat = nullptr) {
   escaped = false;
   if (prim < 0) {  // Li on a miss: envmap(ray.direction) (Integrator.cpp:93-97)
@@ -411,8 +430,7 @@ NOVA_HD bool shade_path(const ShadeParams &sp, const ShadeCtx &sc, Sobol sobol, 
   if (kAdj) {
     const f3 dlna = ss.dlna;
     const float dlnr = ss.dlnr;
-    const uint32_t npix = (uint32_t)sp.fp.width * (uint32_t)sp.fp.height;
-    const uint32_t px = pixel_offset(sp.fp, slot % npix);
+    const uint32_t px = pixel_offset(sp.fp, slot_pixel(sp.fp, slot).pixel);
     const float *lt = adj->ltot;  // the path's primal radiance: the caller points ltot at it
     const float *di = adj->dimg + px;
     // loss gradient of this vertex's weight, per channel: dimg * (L_path - L)

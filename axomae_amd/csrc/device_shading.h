@@ -349,7 +349,6 @@ struct VNDF {
   NOVA_HD float dlnG_da(f3 wo, f3 wi) const { return -(dlambda_da(wo) + dlambda_da(wi)) / (1.f + lambda(wo) + lambda(wi)); }
 };
 
-enum : unsigned { BX_REFLECTION = 1, BX_TRANSMISSION = 2, BX_DIFFUSE = 4, BX_GLOSSY = 8, BX_SPECULAR = 16 };
 enum : int { LOBE_NONE = 0, LOBE_DIFFUSE = 1, LOBE_SPECULAR = 2, LOBE_DIELECTRIC = 3 };
 
 struct BsdfIn {
@@ -368,19 +367,15 @@ struct Principled {
 
   // configureBSDFParams + generateWeightsFromParam (BSDF.h:43-97); subsurface 1, sheen 0,
   // clearcoat 0, specular 1, thin_surface false (BxDF.h:22-39 defaults).
+  // All but the frame, which orient() makes once the shading normal is final: the weights do not
+  // depend on it.
   NOVA_HD void configure(const BsdfIn &p) {
-    frame = gram_shmidt3(p.ns, p.dpdu, p.dpdv);
     eta = p.eta;
     albedo = p.albedo;
     roughness = p.roughness;
     metal = p.metal;
     anisotropy = p.anisotropy;
-    if (p.wo_dot_ng < 0) {
-      frame.c0 = -frame.c0;
-      frame.c1 = -frame.c1;
-      frame.c2 = -frame.c2;
-      if (eta.x != 0.f && eta.y != 0.f && eta.z != 0.f) eta = mk3(1.f / eta.x, 1.f / eta.y, 1.f / eta.z);
-    }
+    if (p.wo_dot_ng < 0 && eta.x != 0.f && eta.y != 0.f && eta.z != 0.f) eta = mk3(1.f / eta.x, 1.f / eta.y, 1.f / eta.z);
     const float ac = fabsf(p.wo_dot_ng);
     w_diffuse = (1 - p.transmission) * (1 - p.metal);
     const float w_sheen = (1 - p.metal) * 0.f * (1.f - p.transmission);
@@ -395,6 +390,14 @@ struct Principled {
     p_diffuse = pd / W;
     p_specular = ps / W;
     p_transmission = w_transmission / W;
+  }
+  NOVA_HD void orient(const BsdfIn &p) {
+    frame = gram_shmidt3(p.ns, p.dpdu, p.dpdv);
+    if (p.wo_dot_ng < 0) {
+      frame.c0 = -frame.c0;
+      frame.c1 = -frame.c1;
+      frame.c2 = -frame.c2;
+    }
   }
   // constructBXDF (BSDF.h:68-79)
   NOVA_HD void construct(float uc) {
@@ -413,15 +416,6 @@ struct Principled {
       lobe_weight = w_transmission;
       lobe_prob = p_transmission;
     }
-  }
-  NOVA_HD unsigned flags(const VNDF &g) const {
-    if (lobe == LOBE_DIFFUSE) return BX_DIFFUSE | BX_REFLECTION;
-    if (lobe == LOBE_SPECULAR) return g.full_specular() ? (BX_SPECULAR | BX_REFLECTION) : (BX_GLOSSY | BX_REFLECTION);
-    if (lobe == LOBE_DIELECTRIC) {
-      unsigned f = eta.x == 1.f ? BX_TRANSMISSION : (BX_REFLECTION | BX_TRANSMISSION);
-      return f | (g.full_specular() ? BX_SPECULAR : BX_GLOSSY);
-    }
-    return 0;
   }
 };
 
@@ -463,10 +457,11 @@ NOVA_HD bool sample_disney(const Principled &b, f3 wo, float x, float y, BsdfSam
 // ran them twice (with the one sincos for both lobes in sample_surface, shading of the 1080p job of 64
 // frames 14.2 -> 13.1 ms, a 256x256 frame of 36 triangles 294 -> 260 us).
 // g samples and weights by its pdf; ge gives the BSDF value. They are the same distribution
-// (`same`) except in the detached-sampling gradient checks. (px, py): the disk point of the
-// normal's sample. The record is written once: per-branch field stores made the compiler keep it
+// (`same`) except in the detached-sampling gradient checks. uc() is the sample that chooses
+// between a dielectric's reflection and transmission; (px, py) the disk point of the normal's. The record is written once: per-branch field stores made the compiler keep it
 // in scratch memory.
-NOVA_HD bool sample_microfacet(const Principled &b, const VNDF &g, const VNDF &ge, bool same, f3 wo, float uc, float px, float py, BsdfSample &s) {
+template <class Uc>
+NOVA_HD bool sample_microfacet(const Principled &b, const VNDF &g, const VNDF &ge, bool same, f3 wo, Uc uc, float px, float py, BsdfSample &s) {
   const bool specular = b.lobe == LOBE_SPECULAR;
   const float ior = b.eta.x;
   f3 f, wi, wm = mk3(0.f, 0.f, 0.f);
@@ -476,7 +471,7 @@ NOVA_HD bool sample_microfacet(const Principled &b, const VNDF &g, const VNDF &g
     const float R = fresnel_real(ior, wo.z), T = 1 - R;
     const float pr = R, pt = T;
     if (pr == 0.f && pt == 0.f) return false;
-    if (uc < (pr / (pr + pt))) {
+    if (uc() < (pr / (pr + pt))) {
       wi = reflect(-wo, mk3(0, 0, 1.f));
       ct = abscos(wi);
       f = b.lobe_weight * b.albedo * R / ct;
@@ -504,7 +499,7 @@ NOVA_HD bool sample_microfacet(const Principled &b, const VNDF &g, const VNDF &g
       pr = R;
       pt = T;
       if (pr == 0.f && pt == 0.f) return false;
-      reflects = uc < (pr / (pr + pt));
+      reflects = uc() < (pr / (pr + pt));
     }
     if (reflects) {
       wi = reflect(-wo, wm);

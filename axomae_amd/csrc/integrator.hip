@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void generate_kernel(FrameParams fp, const uin
   const SobolNibbles sobn{sob_tab, 0};
   const uint32_t n = q.cap;  // plane stride
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < active; i += gridDim.x * blockDim.x) {
-    const uint32_t slot = path_slot(fp, i);
+    const PathPixel slot = path_pixel(fp, i);
     f3 o, d;
     camera_ray(fp, sobn, slot, o, d);
     float *r = q.ray[0];
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
         if (adj.hit_cache && (uint32_t)sp.bounce < adj.cache_bounces)
           adj.hit_cache[(size_t)sp.bounce * adj.cache_paths + pid] = make_float4(__builtin_bit_cast(float, prim), ht, hu, hv);
       }
-      cont = shade_path<kAdj>(sp, sc, sobn, path_slot(sp.fp, (uint32_t)pid), o, d, prim, ht, hu, hv, T, L, A, no, nd, escaped, &padj, &splat);
+      cont = shade_path<kAdj>(sp, sc, sobn, path_pixel(sp.fp, (uint32_t)pid), o, d, prim, ht, hu, hv, T, L, A, no, nd, escaped, &padj, &splat);
       const bool done = !cont;
       q.T[pid] = T.x;
       q.T[paths + pid] = T.y;
@@ -488,7 +488,7 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TAIL_OCCUPANCY void tail_kernel(T
     f3 T = mk3(q.T[pid], q.T[paths + pid], q.T[2 * paths + pid]);
     f3 L = mk3(q.L[pid], q.L[paths + pid], q.L[2 * paths + pid]);
     float A = q.A[pid];
-    const uint32_t slot = path_slot(sp.fp, (uint32_t)pid);
+    const PathPixel slot = path_pixel(sp.fp, (uint32_t)pid);
     ShadeParams s = sp;
     for (int k = sp.bounce; k <= max_depth; k++) {
       s.bounce = k;
