@@ -68,9 +68,9 @@ struct BatchQueues {
   int32_t *slot[2];  // wave-relative slot
   int32_t *sid[2];   // scene index
   float4 *hit;        // closest hit per queue entry: (prim id bits, t, u, v), one 16-byte record
-  float *T, *L, *A;
+  PathState *state;   // by wave-relative slot
   float *partial;  // wave-relative slot x 4
-  uint32_t cap;    // paths of a wave (plane stride of the path state)
+  uint32_t cap;    // paths of a wave
   uint32_t entries, shard_bits, seg;  // of a queue: plane stride; its shards
 };
 
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void batch_generate(const BatchScene *__restri
   __syncthreads();
   const SobolNibbles sobn{sob_tab, 0};
   const WaveDesc w = waves[st->wave];
-  const size_t n = q.cap, qn = q.entries;
+  const size_t qn = q.entries;
   for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < w.count; r += gridDim.x * blockDim.x) {
     const uint64_t g = w.start + r;
     const int s = find_scene(scenes, nscenes, g);
@@ -109,9 +109,6 @@ __global__ __launch_bounds__(256) void batch_generate(const BatchScene *__restri
     ray[5 * qn + r] = d.z;
     q.slot[0][r] = (int32_t)r;
     q.sid[0][r] = s;
-    q.T[r] = q.T[n + r] = q.T[2 * n + r] = 1.f;
-    q.L[r] = q.L[n + r] = q.L[2 * n + r] = 0.f;
-    q.A[r] = 0.f;
   }
   if (blockIdx.x == 0 && threadIdx.x < (1u << q.shard_bits)) {
     const uint32_t k = threadIdx.x;
@@ -200,7 +197,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   __syncthreads();
   const SobolNibbles sobn{sob_tab, dim0};
   const uint64_t wstart = waves[st->wave].start;
-  const size_t cap = q.cap, qn = q.entries;
+  const size_t qn = q.entries;
   const float *rin = q.ray[which];
   float *rout = q.ray[which ^ 1];
   // the workgroup's shard of the queue; its survivors go to the same shard of the next one
@@ -219,9 +216,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       sid = q.sid[which][i];
       const f3 o = mk3(rin[i], rin[qn + i], rin[2 * qn + i]);
       const f3 d = mk3(rin[3 * qn + i], rin[4 * qn + i], rin[5 * qn + i]);
-      f3 T = mk3(q.T[slot], q.T[cap + slot], q.T[2 * cap + slot]);
-      f3 L = mk3(q.L[slot], q.L[cap + slot], q.L[2 * cap + slot]);
-      float A = q.A[slot];
+      f3 T = mk3(1.f, 1.f, 1.f), L = mk3(0.f, 0.f, 0.f);  // camera rays start fresh
+      float A = 0.f;
+      if (bounce != 0) load_state(q.state + slot, T, L, A);
       const float4 h = q.hit[i];
       const BatchScene &S = scenes[sid];
       ShadeParams sp;
@@ -232,17 +229,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       sp.dim0 = dim0;
       const uint32_t l = (uint32_t)(wstart + (uint64_t)slot - S.first);
       cont = shade_path(sp, S.sc, sobn, path_pixel(S.fp, l), o, d, __builtin_bit_cast(int32_t, h.x), h.y, h.z, h.w, T, L, A, no, nd, escaped);
-      q.T[slot] = T.x;
-      q.T[cap + slot] = T.y;
-      q.T[2 * cap + slot] = T.z;
-      if (!cont) {
+      if (cont)
+        store_state(q.state + slot, T, L, A);
+      else
         reinterpret_cast<float4 *>(q.partial)[slot] = make_float4(L.x, L.y, L.z, A);
-      } else {
-        q.L[slot] = L.x;
-        q.L[cap + slot] = L.y;
-        q.L[2 * cap + slot] = L.z;
-        q.A[slot] = A;
-      }
     }
     const uint64_t m = __ballot(cont);
     const uint32_t lane_rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
@@ -386,9 +376,7 @@ static int alloc_buffers(nova_hip_ctx *ex, const BatchPlan &bp, const WavePlan &
   B.q.sid[1] = ip + 3 * qn;
   B.q.hit = reinterpret_cast<float4 *>(ip + 4 * qn);
   float *hf = (float *)(ip + 8 * qn);
-  B.q.T = hf;
-  B.q.L = hf + 3 * (size_t)cap;
-  B.q.A = hf + 6 * (size_t)cap;
+  B.q.state = reinterpret_cast<PathState *>(hf);
   B.q.partial = hf + 7 * (size_t)cap;  // 4 floats per slot
   B.scenes = (BatchScene *)ensure_scratch(ex, 7, bp.scenes.size() * sizeof(BatchScene), &e);
   if (!B.scenes) return check_hip(ex, e, "batch scene table alloc");

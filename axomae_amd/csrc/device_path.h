@@ -209,6 +209,20 @@ NOVA_HD bool tri_hit(const TriMT &tr, TieGet tie, f3 o, f3 d, float tnear, float
   return mt_test(tr, o, d, tnear, tbest, t, u, v);
 }
 
+// A path's throughput, radiance and alpha between two bounces: one record of 28 bytes by path id.
+// Seven planes of floats took seven loads and stores, and once few paths are left each of them
+// moved a line for one float.
+struct PathState {
+  float T[3], L[3], A;
+};
+NOVA_HD void load_state(const PathState *p, f3 &T, f3 &L, float &A) {
+  const PathState s = *p;
+  T = mk3(s.T[0], s.T[1], s.T[2]);
+  L = mk3(s.L[0], s.L[1], s.L[2]);
+  A = s.A;
+}
+NOVA_HD void store_state(PathState *p, f3 T, f3 L, float A) { *p = PathState{{T.x, T.y, T.z}, {L.x, L.y, L.z}, A}; }
+
 // Path-replay adjoint inputs: the primal radiance of every path slot (the batch's partial
 // buffers), the loss gradient per pixel (scaled) and the gradient pool (FP32 texel layout).
 struct AdjointCtx {
@@ -331,9 +345,12 @@ NOVA_HD void sample_surface(const ShadeParams &sp, const ShadeCtx &sc, Sobol sob
   const float r_sampling = detached ? sample_f32_bilinear(sc, sc.sampling_roughness, h.u, h.v).x : b.roughness;
   // a glossy or reflecting lobe (every lobe but a delta transmission and none)
   const bool no_reflection = b.lobe == LOBE_NONE || (b.lobe == LOBE_DIELECTRIC && b.eta.x == 1.f && VNDF(b.anisotropy, r_sampling).full_specular());
-  // the corrected shading normal moves the frame; the chosen lobe and its weights do not depend on it
-  if (!no_reflection && bi.wo_dot_ng >= 0) bi.ns = normalize(correct_specular_shading_normal(bi.ng, wo, bi.ns));
-  if (!no_reflection && bi.wo_dot_ng >= 0) b.orient(bi);
+  // The corrected shading normal moves the frame; the chosen lobe and its weights do not depend on
+  // it. (One orient() after this test would do, and made the shade kernel spill 59 registers for 11.)
+  if (!no_reflection && bi.wo_dot_ng >= 0) {
+    bi.ns = normalize(correct_specular_shading_normal(bi.ng, wo, bi.ns));
+    b.orient(bi);
+  }
   // PrincipledBSDF::sample_f (BSDF.h:107-130)
   const float u0 = sobol_dim(sobol, sp.dim0 + 1, g);
   const float u1 = sobol_dim(sobol, sp.dim0 + 2, g);

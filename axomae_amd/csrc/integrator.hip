@@ -46,10 +46,9 @@ struct Queues {
                                 // per-ray walk: [8] wave loop turns, [9] active lanes summed over turns, [10] wave rounds of the triangle loop;
                                 // tail_kernel: [16] segments, [17] node visits, [18] triangle tests
   float4 *hit;        // closest hit per queue entry: (prim id bits, t, u, v), one 16-byte record
-  float *T, *L, *A;   // path state by path id: T,L 3 planes of `paths` each; A alpha
+  PathState *state;   // by path id
   float *partial;     // frames x W x H x 4
   uint32_t cap;       // entries of a queue (plane stride)
-  uint32_t paths;     // paths of a batch (plane stride of the path state)
   uint32_t shard_bits, seg;
 };
 
@@ -356,7 +355,7 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
   }
   __syncthreads();
   const SobolNibbles sobn{sob_tab, sp.dim0};
-  const size_t cap = q.cap, paths = q.paths;
+  const size_t cap = q.cap;
   const float *rin = q.ray[which];
   float *rout = q.ray[which ^ 1];
   int32_t *sout = q.slot[which ^ 1];
@@ -381,9 +380,9 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
       pid = first ? (int32_t)i : q.slot[which][i];
       const f3 o = mk3(rin[i], rin[cap + i], rin[2 * cap + i]);
       const f3 d = mk3(rin[3 * cap + i], rin[4 * cap + i], rin[5 * cap + i]);
-      f3 T = first ? mk3(1.f, 1.f, 1.f) : mk3(q.T[pid], q.T[paths + pid], q.T[2 * paths + pid]);
-      f3 L = first ? mk3(0.f, 0.f, 0.f) : mk3(q.L[pid], q.L[paths + pid], q.L[2 * paths + pid]);
-      float A = first ? 0.f : q.A[pid];
+      f3 T = mk3(1.f, 1.f, 1.f), L = mk3(0.f, 0.f, 0.f);
+      float A = 0.f;
+      if (!first) load_state(q.state + pid, T, L, A);
       int prim;
       float ht, hu, hv;
       AdjointCtx padj = adj;
@@ -414,18 +413,10 @@ __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel
           adj.hit_cache[(size_t)sp.bounce * adj.cache_paths + pid] = make_float4(__builtin_bit_cast(float, prim), ht, hu, hv);
       }
       cont = shade_path<kAdj>(sp, sc, sobn, path_pixel(sp.fp, (uint32_t)pid), o, d, prim, ht, hu, hv, T, L, A, no, nd, escaped, &padj, &splat);
-      const bool done = !cont;
-      q.T[pid] = T.x;
-      q.T[paths + pid] = T.y;
-      q.T[2 * paths + pid] = T.z;
-      if (done) {
-        if (!kAdj) write_partial(q, (uint32_t)pid, L.x, L.y, L.z, A);  // a replay reads the primal's
-      } else {
-        q.L[pid] = L.x;
-        q.L[paths + pid] = L.y;
-        q.L[2 * paths + pid] = L.z;
-        q.A[pid] = A;
-      }
+      if (cont)
+        store_state(q.state + pid, T, L, A);
+      else if (!kAdj)
+        write_partial(q, (uint32_t)pid, L.x, L.y, L.z, A);  // a replay reads the primal's
     }
     if constexpr (kAdj) splat_to_table(sc, adj, table, splat);
     escapes += (uint32_t)__popcll(__ballot(escaped));
@@ -475,7 +466,7 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TAIL_OCCUPANCY void tail_kernel(T
   const SobolNibbles sobn{sob_tab, sp.dim0};
   const uint32_t shard = block_shard(q.shard_bits), n = q.shard_n[which][shard * kCounterStride];
   const float *rin = q.ray[which];
-  const size_t cap = q.cap, paths = q.paths;
+  const size_t cap = q.cap;
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   LdsStack stk{tail_lds, tc.gstack, tc.gstride, gtid, threadIdx.x};
   uint32_t nv = 0, nt = 0, segs = 0, escapes = 0;
@@ -485,9 +476,9 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TAIL_OCCUPANCY void tail_kernel(T
     const int32_t pid = q.slot[which][i];
     f3 o = mk3(rin[i], rin[cap + i], rin[2 * cap + i]);
     f3 d = mk3(rin[3 * cap + i], rin[4 * cap + i], rin[5 * cap + i]);
-    f3 T = mk3(q.T[pid], q.T[paths + pid], q.T[2 * paths + pid]);
-    f3 L = mk3(q.L[pid], q.L[paths + pid], q.L[2 * paths + pid]);
-    float A = q.A[pid];
+    f3 T, L;
+    float A;
+    load_state(q.state + pid, T, L, A);
     const PathPixel slot = path_pixel(sp.fp, (uint32_t)pid);
     ShadeParams s = sp;
     for (int k = sp.bounce; k <= max_depth; k++) {
@@ -828,7 +819,7 @@ static size_t counter_bytes(uint32_t bits) { return bits == 0 ? kControlBytes : 
 // per path), the counters and the traversal overflow stacks of `threads` lanes.
 static size_t noalloc_bytes(size_t cap, uint32_t max_bits, uint32_t threads, uint32_t stack_bound) {
   const QueueShape qs = queue_shape(cap, max_bits);
-  const size_t pieces[] = {qs.entries * 12 * sizeof(float), qs.entries * 2 * sizeof(int32_t), qs.entries * 4 * sizeof(float), cap * 7 * sizeof(float),
+  const size_t pieces[] = {qs.entries * 12 * sizeof(float), qs.entries * 2 * sizeof(int32_t), qs.entries * 4 * sizeof(float), cap * sizeof(PathState),
                            cap * 4 * sizeof(float)};
   size_t total = 256 + counter_bytes(qs.bits);
   for (size_t b : pieces) total += (b + 255) / 256 * 256;
@@ -1035,7 +1026,6 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
   const size_t qn = qs.entries;
   Queues q;
   q.cap = (uint32_t)qn;
-  q.paths = (uint32_t)cap;
   q.shard_bits = qs.bits;
   q.seg = qs.seg;
   float *rays = (float *)piece(0, qn * 12 * sizeof(float));
@@ -1047,7 +1037,7 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
   unsigned long long *stats64 = (unsigned long long *)(counts + 8);
   float *hits = (float *)piece(3, qn * 4 * sizeof(float));
   if (!hits) return check_hip(ctx, e, "hit alloc");
-  float *state = (float *)piece(4, cap * 7 * sizeof(float));
+  PathState *state = (PathState *)piece(4, cap * sizeof(PathState));
   if (!state) return check_hip(ctx, e, "state alloc");
   float *partial = (float *)piece(5, cap * 4 * sizeof(float));
   if (!partial) return check_hip(ctx, e, "partial alloc");
@@ -1067,9 +1057,7 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
   }
   q.stats64 = stats64;
   q.hit = reinterpret_cast<float4 *>(hits);
-  q.T = state;
-  q.L = state + 3 * cap;
-  q.A = state + 6 * cap;
+  q.state = state;
   q.partial = partial;
   Queues q0 = q;  // camera-ray launches count their node visits and triangle tests apart
   q0.stats64 = stats64 + 4;
