@@ -295,22 +295,42 @@ __device__ __forceinline__ int32_t push_inner(LdsStack &stack, int &sp, const in
 }
 #endif
 
+// A node's four 16-byte words.
+struct NodeWords {
+  float4 g0, g1;
+  uint4 g2;
+  int4 ch;
+};
+NOVA_HD void load_node(const TraceCtx &tc, int32_t node, NodeWords &w) {
+  const NOVA_GLOBAL float4 *np = (const NOVA_GLOBAL float4 *)(tc.nodes + node);
+  w.g0 = np[0];
+  w.g1 = np[1];
+  w.g2 = *(const NOVA_GLOBAL uint4 *)(np + 2);
+  w.ch = *(const NOVA_GLOBAL int4 *)(np + 3);
+}
+
 // One node of the walk: test the node's four children with a slightly widened slab (no box
 // holding a hit the reference's division-form test accepts is culled), order them near to
 // far, push the inner ones, intersect the leaves (exact Moller-Trumbore; exact equal-t ties
 // settled in the reference's visiting order). Returns true when the walk is over; the hit is
 // then st.best / st.tbest / st.bu / st.bv. Stack provides push(level, node) and at(level);
-// tie_of(tc) gives the tie tables.
+// tie_of(tc) gives the tie tables. With `ahead`, which holds st.node's words, the next node's are
+// on their way while the leaves are tested: 14 registers for the latency of a node, which pays
+// where few waves are in flight.
 template <bool kCount, class Stack, class TieOf = TieFromCtx>
 NOVA_HD bool trace_step(const TraceCtx &tc, Stack &stack, TraceState &st, float tnear, uint32_t &nodes_visited, uint32_t &tri_tests,
-                        TieOf tie_of = TieOf()) {
+                        TieOf tie_of = TieOf(), NodeWords *ahead = nullptr) {
   const float kUp = 1.000001f;
   const float kInf = __builtin_inff();
     if (kCount) nodes_visited++;
-    const NOVA_GLOBAL float4 *np = (const NOVA_GLOBAL float4 *)(tc.nodes + st.node);
-    const float4 g0 = np[0], g1 = np[1];
-    const uint4 g2 = *(const NOVA_GLOBAL uint4 *)(np + 2);
-    const int4 ch = *(const NOVA_GLOBAL int4 *)(np + 3);
+    NodeWords nw;
+    if (ahead)
+      nw = *ahead;
+    else
+      load_node(tc, st.node, nw);
+    const float4 g0 = nw.g0, g1 = nw.g1;
+    const uint4 g2 = nw.g2;
+    const int4 ch = nw.ch;
     const float orgx = g0.x, orgy = g0.y, orgz = g0.z, sx = g0.w, sy = g1.x, sz = g1.y;
     const uint32_t qmnx = __builtin_bit_cast(uint32_t, g1.z), qmxx = __builtin_bit_cast(uint32_t, g1.w);
     const uint32_t qmny = g2.x, qmxy = g2.y, qmnz = g2.z, qmxz = g2.w;
@@ -393,6 +413,14 @@ NOVA_HD bool trace_step(const TraceCtx &tc, Stack &stack, TraceState &st, float 
     exch(1, 3);
     exch(1, 2);
     const int32_t next = push_inner(stack, st.sp, cref);  // far to near; the nearest is visited next
+    bool done = false;
+    if (next >= 0)
+      st.node = next;
+    else if (st.sp == 0)
+      done = true;
+    else
+      st.node = (int32_t)stack.at(--st.sp);
+    if (ahead && !done) load_node(tc, st.node, *ahead);
     // Leaves now, near to far, one triangle of a lane's own list each round: lanes whose leaves
     // lie at different places among the children are tested in the same round (and one copy of the
     // test serves all four: the walk shrinks from 3,395 to 1,311 instructions; a 256x256 frame
@@ -436,24 +464,20 @@ NOVA_HD bool trace_step(const TraceCtx &tc, Stack &stack, TraceState &st, float 
       }
       i++;
     }
-    if (next >= 0) {
-      st.node = next;
-      return false;
-    }
-    if (st.sp == 0) return true;
-    st.node = (int32_t)stack.at(--st.sp);
-    return false;
+    return done;
 }
 
 // Closest hit of one ray: the steps until the walk ends (each node is visited once; the cap
 // only guards against a malformed tree).
-template <bool kCount, class Stack>
+template <bool kCount, bool kAhead = false, class Stack>
 NOVA_HD int trace_closest(const TraceCtx &tc, Stack &stack, f3 o, f3 d, float tnear, float &t_out, float &u_out, float &v_out,
                           uint32_t &nodes_visited, uint32_t &tri_tests) {
   TraceState st;
   trace_init(st, o, d);
+  NodeWords words;
+  if (kAhead) load_node(tc, st.node, words);
   for (uint32_t visits = 0; visits < (1u << 24); visits++)
-    if (trace_step<kCount>(tc, stack, st, tnear, nodes_visited, tri_tests)) break;
+    if (trace_step<kCount>(tc, stack, st, tnear, nodes_visited, tri_tests, TieFromCtx(), kAhead ? &words : nullptr)) break;
   t_out = st.tbest;
   u_out = st.bu;
   v_out = st.bv;

@@ -82,11 +82,12 @@ struct WalkCounts {
   uint32_t nodes = 0, tests = 0, wave_turns = 0, lane_turns = 0, tri_rounds = 0;  // instrumented launches only
 };
 
-template <bool kCount, class Share, class Fetch, class Store, class TieOf = TieFromCtx>
+template <bool kCount, bool kAhead = false, class Share, class Fetch, class Store, class TieOf = TieFromCtx>
 __device__ __forceinline__ void refill_walk(const TraceCtx &tc, LdsStack &stk, const Share &share, uint32_t *claims, Fetch fetch, Store store,
                                             WalkCounts &c, TieOf tie_of = TieOf()) {
   const uint32_t lane = threadIdx.x & 63, n = share.n, handed = share.handed;
   TraceState ts;
+  NodeWords words;
   bool have = false, exhausted = handed >= n;
   uint32_t ray = 0;
   for (uint32_t turns = 0; turns < (1u << 30); turns++) {
@@ -107,6 +108,7 @@ __device__ __forceinline__ void refill_walk(const TraceCtx &tc, LdsStack &stk, c
         f3 o, d;
         fetch(p, o, d);
         trace_init(ts, o, d);
+        if (kAhead) load_node(tc, ts.node, words);
         ray = p;
         have = true;
       }
@@ -117,7 +119,7 @@ __device__ __forceinline__ void refill_walk(const TraceCtx &tc, LdsStack &stk, c
       c.wave_turns++;
       c.lane_turns += (uint32_t)__popcll(busy);
     }
-    if (have && trace_step<kCount>(tc, stk, ts, 0.000001f, c.nodes, c.tests, tie_of)) {
+    if (have && trace_step<kCount>(tc, stk, ts, 0.000001f, c.nodes, c.tests, tie_of, kAhead ? &words : nullptr)) {
       store(ray, ts);
       have = false;
       if (kCount) c.tri_rounds += ts.tri_rounds;

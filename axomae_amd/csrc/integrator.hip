@@ -87,25 +87,31 @@ __global__ __launch_bounds__(256) void generate_kernel(FrameParams fp, const uin
   }
 }
 
+// Waves per SIMD of the refilled walks, and with that their workgroups per CU: as many as are
+// resident at once (a 256-thread workgroup is one wave on each of the CU's 4 SIMDs). A lane's first
+// ray is fixed by its thread index, so a workgroup that waits for a free slot would start its rays
+// only after the queue has drained and add a whole walk's latency at the end of the launch.
+// A walk that has the next node's words on their way (trace_step's `ahead`) takes 14 registers
+// more: 5 waves instead of 6. It is the faster one where a launch has few rays per lane and ends
+// with the latency of the last (1 frame of 1080p against 1,048,576 triangles 1.77 -> 1.68 ms, its
+// normals 468 -> 425 us, 1,000,000 rays 290 -> 282 us); with 64 frames, whose walks keep every lane
+// busy, 6 waves are (41.9 against 42.7 ms).
 #ifndef NOVA_TRACE_WAVES
-#define NOVA_TRACE_WAVES 6  // waves per SIMD the extend kernel is compiled for (0: compiler's choice)
+#define NOVA_TRACE_WAVES 6
 #endif
-// Extend workgroups per CU: as many as are resident at once (a 256-thread workgroup is one
-// wave on each of the CU's 4 SIMDs). A lane's first ray is fixed by its thread index, so a
-// workgroup that waits for a free slot would start its rays only after the queue has drained
-// and add a whole walk's latency at the end of the launch.
-#ifndef NOVA_TRACE_BLOCKS_PER_CU
-#define NOVA_TRACE_BLOCKS_PER_CU (NOVA_TRACE_WAVES > 0 ? NOVA_TRACE_WAVES : 6)
+#ifndef NOVA_AHEAD_WAVES
+#define NOVA_AHEAD_WAVES 5
+#endif
+#ifndef NOVA_AHEAD_PATHS
+#define NOVA_AHEAD_PATHS (6u << 20)  // batches of at most this many paths walk with the next node ahead (2 frames of 1080p: 2.506 against
+                                     // 2.527 ms, 4 frames 3.995 against 3.970)
 #endif
 static_assert(kTraceBlock == 256, "the workgroups-per-CU count assumes one wave per SIMD per workgroup");
-#if NOVA_TRACE_WAVES > 0
-#define NOVA_TRACE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(NOVA_TRACE_WAVES, NOVA_TRACE_WAVES)))
-#else
-#define NOVA_TRACE_OCCUPANCY
-#endif
+#define NOVA_AHEAD_OCCUPANCY __attribute__((amdgpu_waves_per_eu(NOVA_AHEAD_WAVES, NOVA_AHEAD_WAVES)))
 
-template <bool kCount>
-__global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void extend_kernel(TraceCtx tc, Queues q, int which, int bounce, uint32_t tail_rays,
+template <bool kCount, bool kAhead>
+__global__ __launch_bounds__(kTraceBlock)
+    __attribute__((amdgpu_waves_per_eu(kAhead ? NOVA_AHEAD_WAVES : NOVA_TRACE_WAVES, kAhead ? NOVA_AHEAD_WAVES : NOVA_TRACE_WAVES))) void extend_kernel(TraceCtx tc, Queues q, int which, int bounce, uint32_t tail_rays,
                                                                                   int tail_force) {
   __shared__ uint32_t lds[kLdsStack * kTraceBlock];
   const uint32_t n = queue_total(q.shard_n[which], q.shard_bits);
@@ -127,7 +133,7 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void extend_kerne
     d = mk3(r[3 * cap + p], r[4 * cap + p], r[5 * cap + p]);
   };
   auto store = [&](uint32_t p, const TraceState &st) { q.hit[p] = hit_record(st); };
-  refill_walk<kCount>(tc, stk, shard_share(q.shard_n[which], q.shard_bits, q.seg, bounce == 0), q.work + block_shard(q.shard_bits) * kCounterStride, fetch, store, c);
+  refill_walk<kCount, kAhead>(tc, stk, shard_share(q.shard_n[which], q.shard_bits, q.seg, bounce == 0), q.work + block_shard(q.shard_bits) * kCounterStride, fetch, store, c);
   if (kCount) {
     atomicAdd(&q.stats64[8], (unsigned long long)c.wave_turns);
     atomicAdd(&q.stats64[9], (unsigned long long)c.lane_turns);
@@ -486,7 +492,7 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TAIL_OCCUPANCY void tail_kernel(T
       s.last = k == max_depth ? 1 : 0;
       s.rr = (rr_start >= 0 && k >= rr_start) ? 1 : 0;
       float t, u, v;
-      const int prim = trace_closest<kCount>(tc, stk, o, d, 0.000001f, t, u, v, nv, nt);
+      const int prim = trace_closest<kCount, true>(tc, stk, o, d, 0.000001f, t, u, v, nv, nt);
       segs++;
       f3 no = mk3(0, 0, 0), nd = mk3(0, 0, 0);
       bool escaped = false;
@@ -637,7 +643,7 @@ __global__ __launch_bounds__(kTraceBlock) void closest_hit_kernel(TraceCtx tc, c
 // its claim counter in LDS (nothing for a caller to clear, no rate of a shared counter, and calls
 // on several streams share no claims). 3,000,000 rays into 100,480 triangles: 670 -> 515 us, into
 // 1,048,576: 888 -> 690 us.
-__global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void closest_hit_refill_kernel(TraceCtx tc, const float *__restrict__ rays, uint32_t n,
+__global__ __launch_bounds__(kTraceBlock) NOVA_AHEAD_OCCUPANCY void closest_hit_refill_kernel(TraceCtx tc, const float *__restrict__ rays, uint32_t n,
                                                                                               int32_t *__restrict__ prim, float *__restrict__ tuv) {
   __shared__ uint32_t lds[kLdsStack * kTraceBlock], claims;
   if (threadIdx.x == 0) claims = 0;
@@ -645,7 +651,7 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void closest_hit_
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   LdsStack stk{lds, tc.gstack, tc.gstride, gtid, threadIdx.x};
   WalkCounts c;
-  refill_walk<false>(
+  refill_walk<false, true>(
       tc, stk, workgroup_share(n), &claims,
       [&](uint32_t i, f3 &o, f3 &d) {
         const float *r = rays + (size_t)i * 6;
@@ -667,14 +673,14 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void closest_hit_
 // and with lane refill, at its own register budget. One kernel that walked row by row and shaded
 // in place ran at 205 registers, two waves per SIMD, and computed a whole BSDF sample whatever
 // the pass: 1.08 ms for the normals of the 1,048,576-triangle scene at 1080p, these two 0.47.
-__global__ __launch_bounds__(kTraceBlock) NOVA_TRACE_OCCUPANCY void pass_trace_kernel(TraceCtx tc, FrameParams fp, float *__restrict__ hits) {
+__global__ __launch_bounds__(kTraceBlock) NOVA_AHEAD_OCCUPANCY void pass_trace_kernel(TraceCtx tc, FrameParams fp, float *__restrict__ hits) {
   __shared__ uint32_t lds[kLdsStack * kTraceBlock], claims;
   if (threadIdx.x == 0) claims = 0;
   __syncthreads();
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   LdsStack stk{lds, tc.gstack, tc.gstride, gtid, threadIdx.x};
   WalkCounts c;
-  refill_walk<false>(
+  refill_walk<false, true>(
       tc, stk, workgroup_share((uint32_t)fp.width * (uint32_t)fp.height), &claims,
       [&](uint32_t i, f3 &o, f3 &d) { camera_ray_pass(fp, pixel_of_rank(fp, i), o, d); },
       [&](uint32_t i, const TraceState &st) {
@@ -840,8 +846,8 @@ extern "C" int nova_hip_closest_hit(nova_hip_ctx *ctx, const float *rays_dev, ui
   const uint64_t cus = (uint64_t)device_cus(ctx);
   // From two rays per lane on, lanes refill (1,000,000 rays into 1,048,576 triangles: 396 -> 340 us);
   // below that a refilled walk has nothing to win and its lanes take longer (262,147 rays: 127 against 135 us).
-  const bool refill = n >= 2 * cus * NOVA_TRACE_BLOCKS_PER_CU * kTraceBlock;
-  const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + kTraceBlock - 1) / kTraceBlock, cus * (refill ? NOVA_TRACE_BLOCKS_PER_CU : 8));
+  const bool refill = n >= 2 * cus * 6 * kTraceBlock;
+  const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + kTraceBlock - 1) / kTraceBlock, cus * (refill ? NOVA_AHEAD_WAVES : 8));
   const uint32_t threads = blocks * kTraceBlock;
   int st = ensure_gstack(ctx, threads);
   if (st) return st;
@@ -888,7 +894,7 @@ static int render_pass(nova_hip_ctx *ctx, const nova_hip_render_params *p, int p
                        hipStream_t s, bool async) {
   const uint32_t npix = (uint32_t)p->width * (uint32_t)p->height;
   const uint32_t cus = (uint32_t)device_cus(ctx);
-  const uint32_t blocks = std::min<uint32_t>((npix + kTraceBlock - 1) / kTraceBlock, cus * NOVA_TRACE_BLOCKS_PER_CU);
+  const uint32_t blocks = std::min<uint32_t>((npix + kTraceBlock - 1) / kTraceBlock, cus * NOVA_AHEAD_WAVES);
   const uint32_t threads = blocks * kTraceBlock;
   int st = ensure_gstack(ctx, threads);
   if (st) return st;
@@ -997,7 +1003,7 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
   int fb = (int)std::max<size_t>(1, std::min<size_t>((size_t)p->frame_count, kPathsPerBatch / npix));
   const int cus = device_cus(ctx);
   auto trace_threads_of = [&](size_t c) {
-    return (uint32_t)std::min<size_t>((c + kTraceBlock - 1) / kTraceBlock, (size_t)cus * NOVA_TRACE_BLOCKS_PER_CU) * kTraceBlock;
+    return (uint32_t)std::min<size_t>((c + kTraceBlock - 1) / kTraceBlock, (size_t)cus * NOVA_TRACE_WAVES) * kTraceBlock;
   };
   uint32_t max_bits = kMaxShardBits;
   if (noalloc) {
@@ -1063,7 +1069,8 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
   q0.stats64 = stats64 + 4;
 
   const uint32_t trace_threads = trace_threads_of(cap);
-  const uint32_t trace_blocks = trace_threads / kTraceBlock;
+  const bool ahead = cap <= NOVA_AHEAD_PATHS;
+  const uint32_t trace_blocks = std::min<uint32_t>(trace_threads / kTraceBlock, (uint32_t)cus * (ahead ? NOVA_AHEAD_WAVES : NOVA_TRACE_WAVES));
   uint32_t *gstack = nullptr;
   if (noalloc) {
     const uint32_t bound = traversal_stack_bound(ctx);
@@ -1189,12 +1196,14 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
           hipLaunchKernelGGL(extend_coherent_kernel<true>, dim3(cblocks), dim3(kCoherentBlock), 0, s, tc, q0, which);
         else
           hipLaunchKernelGGL(extend_coherent_kernel<false>, dim3(cblocks), dim3(kCoherentBlock), 0, s, tc, q, which);
-      } else if (counting) {
-        hipLaunchKernelGGL(extend_kernel<true>, dim3(trace_blocks), dim3(kTraceBlock), 0, s, tc, k == 0 ? q0 : q, which, k, tail_here ? tail_rays : 0u,
-                           tail_last ? 1 : 0);
       } else {
-        hipLaunchKernelGGL(extend_kernel<false>, dim3(trace_blocks), dim3(kTraceBlock), 0, s, tc, q, which, k, tail_here ? tail_rays : 0u,
-                           tail_last ? 1 : 0);
+        auto extend = [&](auto kernel, const Queues &queues) {
+          hipLaunchKernelGGL(kernel, dim3(trace_blocks), dim3(kTraceBlock), 0, s, tc, queues, which, k, tail_here ? tail_rays : 0u, tail_last ? 1 : 0);
+        };
+        if (counting)
+          extend(ahead ? extend_kernel<true, true> : extend_kernel<true, false>, k == 0 ? q0 : q);
+        else
+          extend(ahead ? extend_kernel<false, true> : extend_kernel<false, false>, q);
       }
       if (timing && (st = stamp())) return st;
       hipLaunchKernelGGL(reset_count_kernel, dim3(1), dim3(64), 0, s, q, which ^ 1);
