@@ -3,7 +3,7 @@
 // Every path of every scene gets a global slot: scenes back to back (in the order given),
 // each scene pixel-major as nova_hip_render_frames numbers its paths (path = pixel * frames +
 // frame; the sampler slot of a path is its frame-major slot, path_slot). The slots are cut into
-// waves of `queue_capacity` paths; a wave runs generate -> (extend, reset, shade) per depth
+// waves of `queue_capacity` paths; a wave runs generate -> (extend, shade) per depth
 // level -> accumulate -> advance, and each of those is one grid-stride launch over the
 // wave's combined queue, whatever scenes the paths belong to (a path carries its scene id
 // through the compaction). Wave parameters live in device memory, so the sequence of one
@@ -125,6 +125,11 @@ struct SceneTie {
   const int32_t *sid;
   __device__ const TieTables *operator()(const TraceCtx &) const { return &scenes[*sid].tie; }
 };
+// The shade's output queue is cleared by the walk before it, the next walk's claims by the shade.
+__device__ __forceinline__ void clear_counters(uint32_t *words, uint32_t bits) {
+  if (blockIdx.x == 0 && threadIdx.x < (1u << bits)) words[threadIdx.x * kCounterStride] = 0;
+}
+
 // Closest hits of the queue: the single-scene renderer's walk, each lane's scene loaded when it
 // takes a ray (not at every step). The scene pointers take its registers past the budget of 6
 // waves per SIMD; at 5 nothing spills. 16 scenes, 55 M paths: 10.5 ms with one claim counter for
@@ -137,6 +142,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5, 
   const size_t qn = q.entries;
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   if (gtid == 0) st->segments += n;
+  clear_counters(st->shard_n[which ^ 1], q.shard_bits);
   LdsStack stk{lds, gstack, gstride, gtid, threadIdx.x};
   TraceCtx tc{nullptr, nullptr, nullptr, 0, nullptr};
   int32_t sid = 0;
@@ -165,6 +171,7 @@ __global__ __launch_bounds__(kBatchCoherentBlock) void batch_extend_coherent(con
   const size_t cap = q.entries;
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if (blockIdx.x == 0 && threadIdx.x == 0) st->segments += n;
+  clear_counters(st->shard_n[1], q.shard_bits);
   uint32_t nv = 0, nt = 0;
   for (uint32_t base = (blockIdx.x * (kBatchCoherentBlock / 64) + wv) * 64u; base < n; base += gridDim.x * kBatchCoherentBlock) {
     const uint32_t i = base + lane;
@@ -182,19 +189,13 @@ __global__ __launch_bounds__(kBatchCoherentBlock) void batch_extend_coherent(con
   }
 }
 
-// Between an extend and a shade launch: the shade's output queue and the next extend's work
-// counter start at zero.
-__global__ void batch_reset(BatchState *st, int which) {
-  st->shard_n[which][threadIdx.x * kCounterStride] = 0;
-  st->work[threadIdx.x * kCounterStride] = 0;
-}
-
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void batch_shade(const BatchScene *__restrict__ scenes, const WaveDesc *__restrict__ waves, BatchState *st,
                                                    const uint32_t *__restrict__ sobol, BatchQueues q, int which, int bounce, int last, int rr,
                                                    uint32_t dim0) {
   __shared__ uint32_t sob_tab[5 * 128];  // nibble tables of dims dim0 .. dim0+4
   sobol_nibble_fill(sobol, dim0, 5, sob_tab, threadIdx.x, blockDim.x);
   __syncthreads();
+  clear_counters(st->work, q.shard_bits);
   const SobolNibbles sobn{sob_tab, dim0};
   const uint64_t wstart = waves[st->wave].start;
   const size_t qn = q.entries;
@@ -414,7 +415,6 @@ static void launch_wave(const BatchPlan &bp, const BatchBuffers &B, const nova_h
     else
       hipLaunchKernelGGL(batch_extend, dim3(trace_blocks), dim3(kTraceBlock), 0, s, B.scenes, B.state, B.q, which, k, B.gstack,
                          trace_blocks * (uint32_t)kTraceBlock);
-    hipLaunchKernelGGL(batch_reset, dim3(1), dim3(1u << kMaxShardBits), 0, s, B.state, which ^ 1);
     const int rr = (bp.rr_start >= 0 && k >= bp.rr_start) ? 1 : 0;
     hipLaunchKernelGGL(batch_shade, dim3(shade_blocks), dim3(256), 0, s, B.scenes, B.waves, B.state, sobol, B.q, which, k,
                        k == bp.max_depth ? 1 : 0, rr, dim);

@@ -52,6 +52,15 @@ struct Queues {
   uint32_t shard_bits, seg;
 };
 
+// Counters that start at zero for a later launch are cleared by one that does not use them: the
+// shade's output queue by the walk before it, the next walk's claims by the shade.
+__device__ __forceinline__ void clear_queue(const Queues &q, int which) {
+  if (blockIdx.x == 0 && threadIdx.x < (1u << q.shard_bits)) q.shard_n[which][threadIdx.x * kCounterStride] = 0;
+}
+__device__ __forceinline__ void clear_claims(const Queues &q) {
+  if (blockIdx.x == 0 && threadIdx.x < (1u << q.shard_bits)) q.work[threadIdx.x * kCounterStride] = 0;
+}
+
 // AbstractIntegrator::render per pixel (Integrator.h:53-95): one camera ray per path slot.
 // The first shade takes the path id from the queue position and starts every path at T = 1,
 // L = 0, A = 0, so neither path ids nor path state are written here.
@@ -118,6 +127,7 @@ __global__ __launch_bounds__(kTraceBlock)
   const float *r = q.ray[which];
   const size_t cap = q.cap;
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
+  clear_queue(q, which ^ 1);
   if (tail_rays) {  // this bounce may hand the batch's remaining paths to tail_kernel
     if (q.count[kTailSlot] != 0) return;  // an earlier bounce did
     if (n <= tail_rays || tail_force) {   // forced: the host launches no later bounce (bit 31: more than tail_rays rays)
@@ -161,6 +171,7 @@ template <bool kCount>
 __global__ __launch_bounds__(kCoherentBlock) NOVA_COHERENT_OCCUPANCY void extend_coherent_kernel(TraceCtx tc, Queues q, int which) {
   uint32_t nv = 0, nt = 0;
   const uint32_t n = q.count[0];  // the first queue: linear
+  clear_queue(q, which ^ 1);
   const float *r = q.ray[which];
   const size_t cap = q.cap;
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -351,6 +362,7 @@ template <bool kAdj>
 __global__ __launch_bounds__(kShadeBlock) NOVA_SHADE_OCCUPANCY void shade_kernel(ShadeParams sp, ShadeCtx sc, const uint32_t *__restrict__ sobol, Queues q, int which,
                                                     AdjointCtx adj) {
   if (q.count[kTailSlot] != 0) return;  // tail_kernel finishes this batch's paths
+  clear_claims(q);
   // nibble tables of this scatter's sampler dimensions (dim0 .. dim0+4)
   __shared__ uint32_t sob_tab[5 * 128];
   sobol_nibble_fill(sobol, sp.dim0, 5, sob_tab, threadIdx.x, blockDim.x);
@@ -518,14 +530,9 @@ __global__ __launch_bounds__(kTraceBlock) NOVA_TAIL_OCCUPANCY void tail_kernel(T
   }
 }
 
-// Between an extend and a shade launch: the shade's output queue and the next extend's claims
-// start at zero.
-__global__ void reset_count_kernel(Queues q, int which) {
-  if (threadIdx.x < (1u << q.shard_bits)) {
-    q.shard_n[which][threadIdx.x * kCounterStride] = 0;
-    q.work[threadIdx.x * kCounterStride] = 0;
-  }
-}
+// A replay that reads its hits from the cache launches no walk, which clears the next queue's
+// counters otherwise.
+__global__ void clear_queue_kernel(Queues q, int which) { clear_queue(q, which); }
 
 // Engine::writeFramebuffer per frame, in frame order (engine.cpp:351-363); one thread per
 // pixel channel, the pixel's frames contiguous in the path-id-ordered partial buffer.
@@ -1190,6 +1197,7 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
       if (timing) kkind.push_back(k == 0 ? 0 : 1);
       if (pass == 1 && replay.hit_cache && (uint32_t)k < replay.cache_bounces) {
         // the replay's rays are pass 0's: their hits are in the cache
+        hipLaunchKernelGGL(clear_queue_kernel, dim3(1), dim3(64), 0, s, q, which ^ 1);
       } else if (k == 0 && coherent0) {
         const uint32_t cblocks = std::min<uint32_t>((active + kCoherentBlock - 1) / kCoherentBlock, (uint32_t)cus * NOVA_COHERENT_BLOCKS_PER_CU);
         if (counting)
@@ -1206,7 +1214,6 @@ static int render_impl(nova_hip_ctx *ctx, const nova_hip_render_params *p, float
           extend(ahead ? extend_kernel<false, true> : extend_kernel<false, false>, q);
       }
       if (timing && (st = stamp())) return st;
-      hipLaunchKernelGGL(reset_count_kernel, dim3(1), dim3(64), 0, s, q, which ^ 1);
       ShadeParams spp;
       spp.fp = fp;
       spp.bounce = k;
