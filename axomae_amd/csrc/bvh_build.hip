@@ -1542,14 +1542,16 @@ extern "C" int nova_hip_bvh_build(nova_hip_ctx *ctx, int build_candidates, nova_
   BuildPlan P{};
   char *temps = nullptr;
   const size_t temp_bytes = carve_build(P, nullptr, n);
-  const bool keep_temps = temp_bytes <= kKeptTemps;
+  bool keep_temps = temp_bytes <= kKeptTemps;
   if (keep_temps) {
     hipError_t e = hipSuccess;
     temps = (char *)ensure_scratch(ctx, kTempSlot, temp_bytes, &e);
-    if (!temps) return check_hip(ctx, e, "build temporaries alloc");
-  } else {
-    NOVA_HIP_CHECK(ctx, hipMalloc(&temps, temp_bytes));
+    if (!temps) {  // no room for a slot with its reserve: just the bytes, for this build
+      (void)hipGetLastError();
+      keep_temps = false;
+    }
   }
+  if (!keep_temps) NOVA_HIP_CHECK(ctx, hipMalloc(&temps, temp_bytes));
   carve_build(P, temps, n);
   P.b.prim_idx = ctx->prim_idx;
 
