@@ -9,7 +9,6 @@
 #include "../../axomae_amd/csrc/device_path.h"
 #include "../../axomae_amd/csrc/device_scene.h"
 #include "../../axomae_amd/csrc/device_trace.h"
-#include "../../axomae_amd/csrc/device_trig.h"
 
 using namespace nova_hip;
 
@@ -354,14 +353,4 @@ extern "C" int emu_sobol_nibble(uint32_t dim0, const uint32_t *idx, int n, float
     }
   }
   return 0;
-}
-
-// The float results of device_trig.h: for n arguments, sin and cos of x, acos of y and
-// atan2(y, x), four floats each.
-extern "C" void emu_trig(const float *x, const float *y, int64_t n, float *out) {
-  for (int64_t i = 0; i < n; i++) {
-    sincos_turns(x[i], out[4 * i], out[4 * i + 1]);
-    out[4 * i + 2] = (float)acos_moderate(y[i]);
-    out[4 * i + 3] = (float)atan2_moderate(y[i], x[i]);
-  }
 }

@@ -2,13 +2,24 @@
 double functions rounded to float: equal wherever the double result is not within its own error
 of the middle between two floats (at most one argument in 10^6), and then one unit apart."""
 import ctypes as C
+import os
+import subprocess
 
 import numpy as np
+import pytest
 
-from test_device_code_on_cpu import emu  # noqa: F401
+HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-def test_trig_rounds_like_the_double_functions(emu):  # noqa: F811
+@pytest.fixture(scope="module")
+def emu(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("trig") / "libtrig_emu.so")
+    subprocess.check_call(["/opt/rocm/bin/hipcc", "-O2", "-std=c++17", "-fPIC", "-shared", "--offload-arch=gfx950", "-ffp-contract=off",
+                           "-fno-fast-math", os.path.join(HERE, "emu", "trig_emu.hip"), "-o", lib])
+    return C.CDLL(lib)
+
+
+def test_trig_rounds_like_the_double_functions(emu):
     rs = np.random.RandomState(3)
     n = 1 << 20
     x = np.concatenate([rs.uniform(-7, 7, n), rs.uniform(-1e-3, 1e-3, n)]).astype(np.float32)
@@ -27,7 +38,7 @@ def test_trig_rounds_like_the_double_functions(emu):  # noqa: F811
         assert np.all(np.abs(out[:, k] - want) <= np.spacing(np.abs(want))), k
 
 
-def test_trig_passes_nan_on(emu):  # noqa: F811
+def test_trig_passes_nan_on(emu):
     x, y = np.array([np.nan, 0.5], np.float32), np.array([0.5, 1.0000001], np.float32)
     out = np.zeros((2, 4), np.float32)
     emu.emu_trig(x.ctypes.data_as(C.c_void_p), y.ctypes.data_as(C.c_void_p), C.c_int64(2), out.ctypes.data_as(C.c_void_p))
