@@ -363,18 +363,19 @@ __global__ __launch_bounds__(kBakeThreads) __attribute__((amdgpu_waves_per_eu(4,
 
 // BRDF tables: computeLut (brdf_lookup_table_baker.frag:74-113) at texel (i, j): NdotV =
 // (i + 0.5) / ow, roughness = (j + 0.5) / oh; the split-sum scale A and bias B over `samples`
-// Hammersley GGX half vectors. A wave takes 64 columns of one row, so its roughness and with it
-// every half vector are the same in all lanes: lane l computes the half vector of each 64
-// samples' l-th once and the wave reads it into scalar registers. The sums stay one by one in
-// sample order (a tree moves them by 1.5e-5 from the shader's). What bounds it is the one wave per
-// SIMD that 256x256 texels give; four samples' arithmetic is interleaved (256x256, 1,024 samples:
-// 565 -> 261 us).
+// Hammersley GGX half vectors. A wave takes kLutColumns columns of one row, so every half vector is
+// the same for all of them: lane l computes the l-th of each 64 once. The lower lanes evaluate the
+// even samples, the upper ones the odd, and the lower add both one by one in sample order (a tree
+// moves the sums by 1.5e-5 from the shader's). What bounds it is arithmetic of too few waves:
+// 256x256, 1,024 samples: 565 us with a texel and all its arithmetic per lane, 256 with shared half
+// vectors and 64 columns a wave (one wave per SIMD), 195 with 32 columns.
+constexpr unsigned kLutColumns = 32;
 __global__ __launch_bounds__(64) void lut_kernel(const BakeMap *__restrict__ maps, int count, uint64_t total, int samples) {
-  const unsigned lane = threadIdx.x;
+  const unsigned lane = threadIdx.x, odd = lane / kLutColumns, column = lane % kLutColumns;
   for (uint64_t g = blockIdx.x; g < total; g += gridDim.x) {
     const BakeMap m = maps[find_map(maps, count, g)];
     const uint64_t local = g - m.first;
-    const unsigned i = (unsigned)(local % m.block_row) * 64u + lane, j = (unsigned)(local / m.block_row);
+    const unsigned i = (unsigned)(local % m.block_row) * kLutColumns + column, j = (unsigned)(local / m.block_row);
     const float ndotv = ((float)i + 0.5f) / (float)m.ow, roughness = ((float)j + 0.5f) / (float)m.oh;
     // with N = +z and up = +x the tangent is -y and the bitangent +x
     const f3 V = mk3(sqrtf(1.0f - ndotv * ndotv), 0.0f, ndotv);
@@ -389,21 +390,24 @@ __global__ __launch_bounds__(64) void lut_kernel(const BakeMap *__restrict__ map
       float sp, cp;
       sincos_2pi(xi0, sp, cp);
       const f3 half = normalize(mk3(sp * st, -(cp * st), ct));
-      for (int k0 = 0; k0 < n; k0 += 4)  // four samples' arithmetic side by side
+      for (int k0 = 0; k0 < n; k0 += 8) {
 #pragma unroll
-      for (int k = k0; k < k0 + 4; k++) {
-        const f3 H = mk3(from_lane(half.x, k), from_lane(half.y, k), from_lane(half.z, k));
-        const f3 L = normalize_mid(H * (2.0f * dot(V, H)) - V);
-        const float ndl = fmaxf(L.z, 0.0f), ndh = fmaxf(H.z, 0.0f), vdh = fmaxf(dot(V, H), 0.0f);
-        const float G = schlick_ggx_ibl(ndl, roughness) * gv;
-        const float g_vis = div_mid(G * vdh, ndh * ndotv);
-        const float fc = pow5(1.0f - vdh);
-        const bool counts = (ndl > 0.0f) & (k < n);
-        A = counts ? A + (1.0f - fc) * g_vis : A;
-        B = counts ? B + fc * g_vis : B;
+        for (int p = 0; p < 8; p += 2) {  // four pairs of samples side by side
+          const int k = k0 + p + (int)odd;
+          const f3 H = mk3(__shfl(half.x, k, 64), __shfl(half.y, k, 64), __shfl(half.z, k, 64));
+          const f3 L = normalize_mid(H * (2.0f * dot(V, H)) - V);
+          const float ndl = fmaxf(L.z, 0.0f), ndh = fmaxf(H.z, 0.0f), vdh = fmaxf(dot(V, H), 0.0f);
+          const float G = schlick_ggx_ibl(ndl, roughness) * gv;
+          const float g_vis = div_mid(G * vdh, ndh * ndotv);
+          const float fc = pow5(1.0f - vdh);
+          const bool counts = (ndl > 0.0f) & (k < n);
+          const float dA = counts ? (1.0f - fc) * g_vis : 0.f, dB = counts ? fc * g_vis : 0.f;
+          A = (A + dA) + __shfl_xor(dA, kLutColumns, 64);
+          B = (B + dB) + __shfl_xor(dB, kLutColumns, 64);
+        }
       }
     }
-    if (i < (unsigned)m.ow) {
+    if (odd == 0 && i < (unsigned)m.ow) {
       float *o = m.out + ((size_t)j * (unsigned)m.ow + i) * 2;
       o[0] = A / (float)samples;
       o[1] = B / (float)samples;
@@ -536,7 +540,7 @@ static int launch_batch(const nova_hip_bake_job *jobs, uint32_t count, int32_t s
     const bool is_riemann = jb.kind == NOVA_HIP_BAKE_IRRADIANCE_RIEMANN;
     const bool is_direct = jb.kind == NOVA_HIP_BAKE_CUBEMAP || (jb.kind == NOVA_HIP_BAKE_PREFILTER && jb.roughness == 0.f);
     const bool is_lut = jb.kind == NOVA_HIP_BAKE_BRDF_LUT;
-    const uint32_t block_row = is_lut ? ((uint32_t)jb.out_width + 63) / 64 : ((uint32_t)jb.out_width + 15) / 16;
+    const uint32_t block_row = is_lut ? ((uint32_t)jb.out_width + kLutColumns - 1) / kLutColumns : ((uint32_t)jb.out_width + 15) / 16;
     uint64_t &first = is_riemann ? riemann_total : is_direct ? direct_total : is_lut ? lut_total : total;
     (is_riemann ? riemann : is_direct ? direct : is_lut ? luts : maps)
         .push_back(BakeMap{jb.env, jb.out, jb.width, jb.height, jb.channels, jb.out_width, jb.out_height, jb.kind, jb.roughness, first, block_row});
